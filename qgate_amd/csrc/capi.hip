@@ -26,6 +26,8 @@ struct qghip_qubit_states {
     // the pending gates; a calc_probability that comes next runs it in the same pass.
     int dec_lane = -1, dec_value = 0;
     double dec_norm = 0.;
+    // lanes that launched collapses fixed and that nothing has written since
+    KnownLanes known;
     // bounded sampling pools that read this state vector when they draw
     std::vector<qghip_sampling_pool *> readers;
 
@@ -125,13 +127,34 @@ void unlist(qghip_qubit_states *qs) {
     v.erase(std::remove(v.begin(), v.end(), qs), v.end());
 }
 
+template <class R>
+Cx<R> *amps(qghip_qubit_states *qs) {
+    return static_cast<Cx<R> *>(qs->d_ptr);
+}
+
+template <class R>
+const Cx<R> *camps(const qghip_qubit_states *qs) {
+    return static_cast<const Cx<R> *>(qs->d_ptr);
+}
+
+// Dispatch on precision: f(float()) or f(double()).
+template <class F>
+void by_prec(Prec p, F &&f) {
+    if (p == precFP32)
+        f(float());
+    else
+        f(double());
+}
+
 constexpr int kDenseWidth = 6;   // default block width of QGHIP_FUSION_DENSE
 
 bool queued(const qghip_qubit_states *qs) { return !qs->pending.empty() || qs->dec_lane >= 0; }
 
-// qs is about to be written or freed: bounded pools drawing from it can no longer draw.
+// qs is about to be written or freed: bounded pools drawing from it can no longer draw, and
+// nothing is known of its lanes.
 void touch(qghip_qubit_states *qs) {
     if (qs == nullptr) return;
+    qs->known = KnownLanes();
     for (qghip_sampling_pool *pl : qs->readers) {
         pl->stale = true;
         pl->src = nullptr;
@@ -139,24 +162,43 @@ void touch(qghip_qubit_states *qs) {
     qs->readers.clear();
 }
 
+// The collapse recorded on qs: run(known, norm) launches it with the norm in the state
+// precision R. A norm that is not finite (a collapse onto probability 0) makes every amplitude
+// of the kept half NaN, zeros included, so nothing is known before or after it.
+template <class R, class F>
+void collapse(qghip_qubit_states *qs, F &&run) {
+    const R norm = (R)qs->dec_norm;
+    const bool finite = std::isfinite(norm);
+    const int lane = qs->dec_lane;
+    qs->dec_lane = -1;
+    KnownLanes known = finite ? qs->known : KnownLanes();
+    qs->known = KnownLanes();
+    run(known, lane, norm);
+    if (!finite) return;
+    known.mask |= u64(1) << lane;
+    known.ones = (known.ones & ~(u64(1) << lane)) | ((u64)qs->dec_value << lane);
+    qs->known = known;
+}
+
 // Apply the queued work of qs: the recorded collapse, then the queued gates.
 void flush(qghip_qubit_states *qs) {
     if (qs == nullptr || !queued(qs)) return;
     std::vector<QueuedGate> gates;
     gates.swap(qs->pending);
-    const int dec_lane = qs->dec_lane;
-    qs->dec_lane = -1;
     unlist(qs);
-    if (qs->d_ptr == nullptr) return;
-    if (dec_lane >= 0) {
-        if (qs->prec == precFP32)
-            launch_decohere<float>(static_cast<Cx<float> *>(qs->d_ptr), qs->n_lanes, dec_lane, qs->dec_value,
-                                   (float)qs->dec_norm);
-        else
-            launch_decohere<double>(static_cast<Cx<double> *>(qs->d_ptr), qs->n_lanes, dec_lane, qs->dec_value,
-                                    qs->dec_norm);
+    if (qs->d_ptr == nullptr) {
+        qs->dec_lane = -1;
+        return;
     }
+    if (qs->dec_lane >= 0)
+        by_prec(qs->prec, [&](auto r) {
+            typedef decltype(r) R;
+            collapse<R>(qs, [&](const KnownLanes &known, int lane, R norm) {
+                launch_decohere<R>(amps<R>(qs), qs->n_lanes, lane, qs->dec_value, norm, known);
+            });
+        });
     if (gates.empty()) return;
+    qs->known = KnownLanes();
     try {
         if (qs->fuse_mode == QGHIP_FUSION_DENSE) {
             const int width = qs->tile_bits > 0 ? qs->tile_bits : kDenseWidth;
@@ -204,25 +246,6 @@ void release(qghip_qubit_states *qs) {
     if (qs->d_ptr) dev_free(qs->d_ptr, qs->bytes);
     qs->d_ptr = nullptr;
     qs->bytes = 0;
-}
-
-template <class R>
-Cx<R> *amps(qghip_qubit_states *qs) {
-    return static_cast<Cx<R> *>(qs->d_ptr);
-}
-
-template <class R>
-const Cx<R> *camps(const qghip_qubit_states *qs) {
-    return static_cast<const Cx<R> *>(qs->d_ptr);
-}
-
-// Dispatch on precision: f(float()) or f(double()).
-template <class F>
-void by_prec(Prec p, F &&f) {
-    if (p == precFP32)
-        f(float());
-    else
-        f(double());
 }
 
 void apply_matrix(const qghip_qubit_processor *p, Prec prec, qghip_qubit_states *qs,
@@ -481,20 +504,19 @@ int qghip_qubit_processor_calc_probability(qghip_qubit_processor *p, qghip_qubit
         check_lane(qs, local_lane);
         if (qs->dec_lane >= 0 && qs->pending.empty()) {
             // the recorded collapse and this probability in one pass over the state
-            const int dec_lane = qs->dec_lane;
-            qs->dec_lane = -1;
             unlist(qs);
             by_prec(p->prec, [&](auto r) {
                 typedef decltype(r) R;
-                *prob = decohere_prob<R>(amps<R>(qs), qs->n_lanes, dec_lane, qs->dec_value, (R)qs->dec_norm,
-                                         local_lane);
+                collapse<R>(qs, [&](const KnownLanes &known, int lane, R norm) {
+                    *prob = decohere_prob<R>(amps<R>(qs), qs->n_lanes, lane, qs->dec_value, norm, local_lane, known);
+                });
             });
             return;
         }
         flush(qs);
         by_prec(p->prec, [&](auto r) {
             typedef decltype(r) R;
-            *prob = calc_prob<R>(camps<R>(qs), qs->n_lanes, local_lane);
+            *prob = calc_prob<R>(camps<R>(qs), qs->n_lanes, local_lane, qs->known);
         });
     });
 }
@@ -556,7 +578,9 @@ int qghip_qubit_processor_decohere(qghip_qubit_processor *p, int value, double p
         check_lane(qs, local_lane);
         if (value != 0 && value != 1) value_error("value must be 0 or 1");
         flush(qs);
+        const KnownLanes known = qs->known;   // a collapse keeps the zeros of the earlier ones
         touch(qs);
+        qs->known = known;
         // norm in FP64, rounded to the state precision (CPUQubitProcessor.cpp:227, :235). The
         // collapse is recorded and launched by the next call that touches qs (flush), or
         // together with the probability when that call is calc_probability.

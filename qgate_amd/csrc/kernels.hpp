@@ -81,15 +81,21 @@ template <class R> void launch_set_zero_state(Cx<R> *a, int n_lanes);
 // dst = src (bytes a multiple of 16): the non-temporal streaming copy used as the HBM ceiling.
 void launch_stream_copy(void *dst, const void *src, u64 bytes);
 // P(bit `lane` == 0), FP64 accumulation; synchronises.
-template <class R> double calc_prob(const Cx<R> *a, int n_lanes, int lane);
+// Lanes on which earlier collapses left nothing but one value (mask), and the ones among those
+// values (ones): every amplitude whose index differs there is zero.
+struct KnownLanes {
+    u64 mask = 0, ones = 0;
+};
+template <class R> double calc_prob(const Cx<R> *a, int n_lanes, int lane, const KnownLanes &known);
 // Doubles of partial-sum buffer calc_prob_in needs for this lane (the partials, run sums and
 // total), and calc_prob with that buffer given instead of taken from the allocator (no
 // allocation; the buffer must hold at least that many doubles).
 template <class R> u64 calc_prob_buffer_len(int n_lanes, int lane);
 template <class R> double calc_prob_in(const Cx<R> *a, int n_lanes, int lane, double *buf, u64 buf_len);
-template <class R> void launch_decohere(Cx<R> *a, int n_lanes, int lane, int value, R norm);
+template <class R> void launch_decohere(Cx<R> *a, int n_lanes, int lane, int value, R norm, const KnownLanes &known);
 // launch_decohere, then calc_prob(prob_lane) of the collapsed state, in one pass; synchronises.
-template <class R> double decohere_prob(Cx<R> *a, int n_lanes, int lane, int value, R norm, int prob_lane);
+template <class R> double decohere_prob(Cx<R> *a, int n_lanes, int lane, int value, R norm, int prob_lane,
+                                         const KnownLanes &known);
 // Pauli string P over lanes x | z (X: x, Z: z, Y: both): P(measuring P gives +1) in FP64,
 // i.e. sum over pairs of |((1 + P) psi)_y|^2 / 2; synchronises.
 template <class R> double calc_pauli_prob(const Cx<R> *a, int n_lanes, u64 x, u64 z);
