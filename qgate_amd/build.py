@@ -20,6 +20,9 @@ ARCH = os.environ.get('QGATE_HIP_ARCH', 'gfx950')
 HIPFLAGS = ['-std=c++17', '-O3', '-fPIC', '--offload-arch=' + ARCH, '-munsafe-fp-atomics',
             '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
             '-Wall', '-Wno-unused-function', '-Wno-unused-command-line-argument']
+# Register tile passes (csrc/tile_reg.hpp) dispatch their ops by uniform branches. Structurized
+# like divergent ones, every arm of the dispatch copied the whole register array.
+EXTRA_FLAGS = {src: ['-mllvm', '-structurizecfg-skip-uniform-regions=true'] for src in ('k_tile.hip', 'k_batch.hip')}
 
 
 def lib_path():
@@ -34,7 +37,7 @@ def _hipcc():
 
 
 def _compile(src, obj, verbose):
-    cmd = [_hipcc()] + HIPFLAGS + ['-c', os.path.join(CSRC, src), '-o', obj]
+    cmd = [_hipcc()] + HIPFLAGS + EXTRA_FLAGS.get(src, []) + ['-c', os.path.join(CSRC, src), '-o', obj]
     if verbose:
         print(' '.join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -32,6 +32,7 @@
 #include "kernels.hpp"
 #include "qg_runtime.hpp"
 #include "tile_common.hpp"
+#include "tile_pauli.hpp"
 #include "tile_reg.hpp"
 
 using namespace qg;
@@ -47,6 +48,15 @@ struct BGate {          // one gate of a group's structure
 template <class R>
 struct BMats {
     Mat2<R> fwd, bwd;
+};
+
+template <class R>
+struct BRow {           // one row of a register-pass coefficient table (kCoefs numbers per item)
+    R c[8];             // fixed gates: the coefficients
+    int kind;           // RegGate kind
+    int pauli;          // rotations: 1 X, 2 Y, 3 Z; 0: fixed
+    int param;
+    int back;           // the inverse (sweep)
 };
 
 struct BOp {            // a gate inside a pass
@@ -104,6 +114,39 @@ __global__ __launch_bounds__(256) void k_batch_mats(const BGate *__restrict__ ga
     out.bwd.m10 = cx<R>((R)m[2], (R)-m[3]);
     out.bwd.m11 = cx<R>((R)m[6], (R)-m[7]);
     mats[i] = out;
+}
+
+// Coefficients of the register passes' rows for every item, in FP64 and rounded once.
+template <class R>
+__global__ __launch_bounds__(256) void k_batch_coefs(const BRow<R> *__restrict__ rows, int n_rows,
+                                                     const double *__restrict__ params, int n_params, u64 n_items,
+                                                     R *__restrict__ coefs) {
+    const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_items * (u64)n_rows) return;
+    const u64 item = i / (u64)n_rows;
+    const BRow<R> row = rows[i % (u64)n_rows];
+    R c[kCoefs];
+    for (int k = 0; k < kCoefs; ++k) c[k] = row.c[k];
+    if (row.pauli != 0) {
+        const double th = params[item * (u64)n_params + (u64)row.param];
+        const double co = cos(0.5 * th), si = row.back ? -sin(0.5 * th) : sin(0.5 * th);
+        if (row.kind == kGateY) {          // m00 = co, m01 = -si
+            rotation_coefs(c, co, -si);
+        } else if (row.kind == kGateX) {   // m00 = co, m01 = -i si
+            rotation_coefs(c, co, si);
+        } else if (row.kind == kGateDiag) {   // co - i si, co + i si and their ratio
+            c[0] = (R)co;  c[1] = (R)-si;
+            c[2] = (R)co;  c[3] = (R)si;
+            c[4] = (R)(co * co - si * si);  c[5] = (R)(2. * co * si);
+        } else {                           // controlled RX, RY: the whole matrix
+            const double isx = row.pauli == 1 ? 1. : 0., isy = row.pauli == 2 ? 1. : 0.;
+            c[0] = (R)co;  c[1] = R(0);
+            c[2] = (R)(-si * isy);  c[3] = (R)(-si * isx);
+            c[4] = (R)(si * isy);   c[5] = (R)(-si * isx);
+            c[6] = (R)co;  c[7] = R(0);
+        }
+    }
+    for (int k = 0; k < kCoefs; ++k) coefs[i * kCoefs + k] = c[k];
 }
 
 // every item to |0...0>
@@ -229,6 +272,29 @@ __global__ __launch_bounds__(T) void k_batch_pauli(const Cx<R> *__restrict__ psi
     }
 }
 
+// The same for full-size tiles (tile_pauli.hpp), one tile a workgroup.
+template <class R, int MB>
+__global__ __launch_bounds__((kPauliThreads<R>)) void k_batch_pauli_full(const Cx<R> *__restrict__ psi,
+                                                                    Cx<R> *__restrict__ lam, const BPass ps,
+                                                                    const PauliWork *__restrict__ works,
+                                                                    const PauliZ *__restrict__ zs,
+                                                                    const double *__restrict__ coefs, int n_terms,
+                                                                    int n, double *__restrict__ partial, u64 first) {
+    __shared__ Cx<R> tp[1 << MB];
+    __shared__ double scratch[kPauliThreads<R> / 64];
+    constexpr int lw = Unit<R>::W == 2 ? 1 : 0;
+    const u64 w = first + blockIdx.x;
+    const u64 base = tile_base(w, ps.pos, MB);
+    tile_to_lds<R, kPauliThreads<R>, (1 << (MB - lw)) / kPauliThreads<R>>(tp, psi, base, ps.pos, MB, ps.low);
+    __syncthreads();
+    double dot = pauli_full_tile<R, MB>(tp, lam, base, ps.pos, ps.low, ps.accumulate != 0, ps.n_slots != 0,
+                                        works + ps.op_begin, ps.n_ops, zs, coefs + (base >> n) * (u64)n_terms * 2);
+    if (ps.n_slots) {
+        dot = block_sum_tile<kPauliThreads<R>>(dot, scratch);
+        if (threadIdx.x == 0) partial[w] = dot;
+    }
+}
+
 // Backward sweep pass over psi and lambda tiles: per gate, the gradient term of a rotation
 // (partial[slot * n_tiles + w] for tile w = item * tiles_per_item + tile index in the item)
 // and U^dagger on both.
@@ -351,8 +417,8 @@ struct BCfg<double> {
     static constexpr int SweepBits = 10;
     static constexpr int Low = 4;
 };
-// Register-resident passes: 256 threads, 2^12 / 2^11 amplitudes per forward tile (16 / 8 per
-// thread) and 2^11 / 2^10 per sweep tile (8 / 4 per thread and state), as in the
+// Register-resident passes (tile_reg.hpp): 256 threads, 2^12 / 2^11 amplitudes per forward tile
+// (16 / 8 per thread) and 2^11 / 2^10 per sweep tile (8 / 4 per thread and state), as in the
 // single-circuit passes.
 constexpr int kBatchRegThreads = 256;
 static_assert(BCfg<float>::MaxBits == TileCfg<float>::MaxBits && BCfg<double>::MaxBits == TileCfg<double>::MaxBits,
@@ -532,6 +598,9 @@ struct Group {
     void *d_mats = nullptr;
     BGate *d_gates = nullptr;
     BOp *d_fops = nullptr, *d_sops = nullptr;
+    bool pauli_full = false;
+    PauliWork *d_pworks = nullptr;
+    PauliZ *d_pzs = nullptr;
     PauliGroup *d_pgroups = nullptr;
     BTermMask *d_tmask = nullptr;
     int *d_slot_out = nullptr, *d_pptr = nullptr, *d_pgate = nullptr, *d_zero = nullptr;
@@ -543,8 +612,11 @@ struct Group {
     std::vector<RegProgram<float>> rprog32;
     std::vector<RegProgram<double>> rprog64;
     std::vector<SweepPass> rspasses;
-    void *d_rsops = nullptr;                // SweepOp<R>[]
-    SweepPhase *d_rphases = nullptr;
+    void *d_rsops = nullptr;                // RegOp<R>[]
+    PhaseBits *d_rphases = nullptr;
+    int n_frows = 0, n_srows = 0;           // rows of the coefficient tables
+    void *d_frows = nullptr, *d_srows = nullptr;   // BRow<R>[]
+    void *d_fcoefs = nullptr, *d_scoefs = nullptr;
     size_t n_items() const { return items.size(); }
 };
 
@@ -609,35 +681,43 @@ std::vector<RegProgram<double>> &reg_programs<double>(Group &g) {
     return g.rprog64;
 }
 
-// A gate's matrix as far as its form goes: fixed gates as they are, rotations at a generic
-// angle (every angle gives the same form: RX general / imaginary off-diagonal, RY real, RZ
-// diagonal with m00 != 1), so one classification holds for every item.
-GateMatrix form_matrix(const CircuitOp &op) { return op.kind == 1 ? rotation(op.pauli, 1.) : op.mat; }
-
-// Register-pass input of one forward gate (the fields plan_phases reads).
+// The register gates of a group's structure, forward or (back) inverted in sweep order, and the
+// row of each in the coefficient table. Rotations keep their form at every angle; fixed gates
+// are split as in the single-circuit passes. RegGate::source is the gate of the structure.
 template <class R>
-struct BRegInput {
-    Mat2<R> m;
-    u64 gctrl;
-    unsigned lctrl;
-    int target, kind;
-};
-
-// Tile-pass kind of a forward gate in a register pass: pair kinds split into swap / real /
-// general, local diagonals with m00 == 1 into kOpDiagPhase (from the matrix rounded to R).
-template <class R>
-int reg_forward_kind(const CircuitOp &op, int kind) {
-    const Mat2<R> mm = round_matrix<R>(form_matrix(op));
-    const R zero = R(0), one = R(1);
-    if (kind == kOpPair) {
-        const bool swap = op.kind == 0 && mm.m00.re == zero && mm.m00.im == zero && mm.m11.re == zero &&
-                          mm.m11.im == zero && mm.m01.re == one && mm.m01.im == zero && mm.m10.re == one &&
-                          mm.m10.im == zero;
-        const bool real = mm.m00.im == zero && mm.m01.im == zero && mm.m10.im == zero && mm.m11.im == zero;
-        return swap ? kOpPairSwap : real ? kOpPairReal : kOpPair;
+std::vector<RegGate> group_gates(const std::vector<CircuitOp> &ops, bool back, std::vector<BRow<R>> &rows) {
+    std::vector<RegGate> out;
+    const int n = (int)ops.size();
+    for (int k = 0; k < n; ++k) {
+        const int i = back ? n - 1 - k : k;
+        const CircuitOp &op = ops[i];
+        if (op.kind == 0) {
+            append_fixed(out, back ? dagger(op.mat) : op.mat, op.ctrl, op.target, i);
+            continue;
+        }
+        RegGate g;
+        g.kind = op.pauli == 3 ? kGateDiag : !op.ctrl.empty() ? kGateAny : op.pauli == 1 ? kGateX : kGateY;
+        g.target = op.target;
+        g.pauli = back ? op.pauli : 0;
+        g.source = i;
+        g.ctrl = op.ctrl;
+        g.m = rotation(op.pauli, back ? -1. : 1.);   // its form; the angle is each item's own
+        out.push_back(g);
     }
-    if (kind == kOpDiagLocal && op.kind == 0 && mm.m00.re == one && mm.m00.im == zero) return kOpDiagPhase;
-    return kind;
+    rows.clear();
+    for (const RegGate &g : out) {
+        BRow<R> r;
+        std::memset(&r, 0, sizeof(r));
+        gate_coefs<R>(g, r.c);
+        r.kind = g.kind;
+        if (ops[g.source].kind == 1) {
+            r.pauli = ops[g.source].pauli;
+            r.param = ops[g.source].param;
+        }
+        r.back = back ? 1 : 0;
+        rows.push_back(r);
+    }
+    return out;
 }
 
 // Plans and device tables of a group for a tuning (allocates; not during capture).
@@ -658,6 +738,8 @@ void build_group(Group &g, const Tuning &t) {
     typedef TileCfg<R> TC;
     const bool fregs = t.registers != 0 && mf == TC::MaxBits && use_register_tiles();
     const bool sregs = t.registers != 0 && ms == C::SweepBits && use_register_tiles();
+    constexpr int kFA = (1 << TC::MaxBits) / kBatchRegThreads, kSA = (1 << C::SweepBits) / kBatchRegThreads;
+    constexpr int kWB = Log2<kBatchRegThreads / 64>::v;
 
     // forward passes
     // (a rotation counts as diagonal only with generator Z: diagonal for every item's angle)
@@ -669,14 +751,9 @@ void build_group(Group &g, const Tuning &t) {
         dlanes[i] = diag ? (u64(1) << op.target) : 0;
         for (int c : op.ctrl) dlanes[i] |= u64(1) << c;
     }
-    auto lanes_of = [&](int gi) {
-        std::vector<int> l(g.ops[gi].ctrl);
-        l.push_back(g.ops[gi].target);
-        return l;
-    };
     std::vector<int> ford;   // forward gates pass by pass
     std::vector<Layout> fl =
-        plan_layouts_ahead(need, dlanes, n, mf, lowf, c64, fregs ? TC::MaxOps : 1 << 30, nullptr, 1 << 30, ford);
+        plan_layouts_ahead(need, dlanes, n, mf, lowf, c64, 1 << 30, nullptr, 1 << 30, ford);
     std::vector<BOp> fops(std::max(1, n_gates));
     g.fpasses.clear();
     std::vector<RegProgram<R>> &progs = reg_programs<R>(g);
@@ -684,12 +761,6 @@ void build_group(Group &g, const Tuning &t) {
     for (const Layout &l : fl) {
         int local[64];
         BPass p = make_pass(l, local);
-        if (fregs) {   // diagonal gates where none of their lanes is a register bit
-            constexpr int A = (1 << TC::MaxBits) / kBatchRegThreads;
-            place_diagonals(
-                ford, l.begin, l.end, local, p.m, Log2<A>::v, Log2<kBatchRegThreads / 64>::v,
-                [&](int gi) { return need[gi] == 0; }, [&](int gi) { return g.ops[gi].target; }, lanes_of);
-        }
         for (int i = l.begin; i < l.end; ++i) {
             const CircuitOp &op = g.ops[ford[i]];
             BOp &o = fops[i];
@@ -709,28 +780,12 @@ void build_group(Group &g, const Tuning &t) {
             o.slot = -1;
         }
         g.fpasses.push_back(p);
-        if (fregs) {
-            RegProgram<R> rp;
-            std::memset(&rp, 0, sizeof(rp));
-            rp.n_ops = p.n_ops;
-            rp.low = p.low;
-            std::memcpy(rp.pos, p.pos, sizeof(rp.pos));
-            std::vector<BRegInput<R>> in(std::max(1, p.n_ops));
-            for (int k = 0; k < p.n_ops; ++k) {
-                const BOp &o = fops[l.begin + k];
-                std::memset(&in[k], 0, sizeof(in[k]));
-                in[k].gctrl = o.gctrl;
-                in[k].lctrl = o.lctrl;
-                in[k].target = o.target;
-                in[k].kind = reg_forward_kind<R>(g.ops[ford[l.begin + k]], o.kind);
-            }
-            constexpr int A = (1 << TC::MaxBits) / kBatchRegThreads;
-            QG_REQUIRE(plan_phases<R>(rp, in.data(), p.m, Log2<A>::v, Log2<kBatchRegThreads / 64>::v),
-                       "batch: register pass with too many phases");
-            for (int k = 0; k < p.n_ops; ++k) rp.ops[k].gate = ford[l.begin + k];
-            progs.push_back(rp);
-        }
     }
+    std::vector<BRow<R>> frows, srows;
+    if (fregs)
+        for (const BuiltPass<R> &bp : build_passes<R>(group_gates<R>(g.ops, false, frows), n, TC::MaxBits, lowf,
+                                                      Log2<kFA>::v, kWB, TC::MaxOps, TC::MaxRegOps, kMaxPhases))
+            progs.push_back(reg_program(bp));
     // sweep passes: the gates in reverse order
     std::vector<u64> sneed(n_gates), sdl(n_gates);
     for (int i = 0; i < n_gates; ++i) sneed[i] = need[n_gates - 1 - i];
@@ -740,9 +795,8 @@ void build_group(Group &g, const Tuning &t) {
     std::vector<int> sord;   // sweep entries (entry e is gate n_gates - 1 - e) pass by pass
     std::vector<Layout> sl = plan_layouts_ahead(sneed, sdl, n, ms, lows, c64, 1 << 30, &srot, kMaxSweepSlots, sord);
     std::vector<BOp> sops(std::max(1, n_gates));
-    std::vector<SweepOp<R>> rsops(std::max(1, n_gates));
-    std::memset(rsops.data(), 0, sizeof(SweepOp<R>) * rsops.size());
-    std::vector<SweepPhase> rphases;
+    std::vector<RegOp<R>> rsops;
+    std::vector<PhaseBits> rphases;
     std::vector<int> slot_out;
     g.spasses.clear();
     g.rspasses.clear();
@@ -751,13 +805,6 @@ void build_group(Group &g, const Tuning &t) {
     for (const Layout &l : sl) {
         int local[64];
         BPass p = make_pass(l, local);
-        if (sregs) {   // diagonal gates where none of their lanes is a register bit
-            constexpr int A = (1 << C::SweepBits) / kBatchRegThreads;
-            place_diagonals(
-                sord, l.begin, l.end, local, p.m, Log2<A>::v, Log2<kBatchRegThreads / 64>::v,
-                [&](int e) { return sneed[e] == 0; }, [&](int e) { return g.ops[n_gates - 1 - e].target; },
-                [&](int e) { return lanes_of(n_gates - 1 - e); });
-        }
         g.spass_slot_begin.push_back((int)slot_out.size());
         int slots = 0;
         for (int i = l.begin; i < l.end; ++i) {
@@ -779,51 +826,35 @@ void build_group(Group &g, const Tuning &t) {
             o.pauli = op.kind == 1 ? op.pauli : 0;
             o.slot = op.kind == 1 ? slots++ : -1;
             if (op.kind == 1) slot_out.push_back(gi);
-            SweepOp<R> &r = rsops[i];
-            r.gctrl = o.gctrl;
-            r.lctrl = o.lctrl;
-            r.target = o.target;
-            r.kind = o.kind;
-            r.slot = o.slot;
-            r.form = sweep_form(dagger(form_matrix(op)), o.pauli, o.kind != kOpPair);
-            r.gate = gi;
         }
         p.n_slots = slots;
         max_slots = std::max(max_slots, slots);
         g.spasses.push_back(p);
-        if (sregs) {
+    }
+    if (sregs) {
+        const std::vector<RegGate> gates = group_gates<R>(g.ops, true, srows);
+        slot_out.clear();
+        g.spass_slot_begin.clear();
+        max_slots = 1;
+        for (const BuiltPass<R> &bp :
+             build_passes<R>(gates, n, C::SweepBits, lows, Log2<kSA>::v, kWB, 1 << 30, 1 << 30, 1 << 30)) {
             SweepPass rp;
-            std::memset(&rp, 0, sizeof(rp));
-            rp.m = p.m;
-            rp.low = p.low;
-            rp.op_begin = l.begin;
-            rp.n_ops = p.n_ops;
-            rp.n_slots = slots;
+            rp.low = bp.low;
+            rp.op_begin = (int)rsops.size();
             rp.phase_begin = (int)rphases.size();
-            std::memcpy(rp.pos, p.pos, sizeof(rp.pos));
-            std::vector<int> pair(p.n_ops);
-            for (int k = 0; k < p.n_ops; ++k)
-                pair[k] = rsops[l.begin + k].kind == kOpPair ? rsops[l.begin + k].target : -1;
-            constexpr int A = (1 << C::SweepBits) / kBatchRegThreads;
-            const std::vector<PhaseLayout> L =
-                plan_phase_layouts(pair, p.m, Log2<A>::v, Log2<kBatchRegThreads / 64>::v);
-            for (const PhaseLayout &P : L) {
-                for (int k = P.begin; k < P.end; ++k) {
-                    SweepOp<R> &r = rsops[l.begin + k];
-                    const RegSplit sp = split_for_phase(P, r.kind, r.target, r.lctrl);
-                    r.rkind = sp.kind;
-                    r.rtarget = sp.target;
-                    r.creg = sp.creg;
-                    r.cthr = sp.cthr;
-                }
-                rphases.push_back(phase_bits(P));
-            }
-            rp.n_phases = (int)L.size();
-            QG_REQUIRE(rp.n_ops == 0 || rp.n_phases > 0, "batch: register sweep pass without phases");
+            rp.n_phases = (int)bp.phases.size();
+            rp.n_slots = (int)bp.slot_gate.size();
+            set_positions(rp.pos, bp.bits);
+            g.spass_slot_begin.push_back((int)slot_out.size());
+            for (int gi : bp.slot_gate) slot_out.push_back(gates[gi].source);
+            max_slots = std::max(max_slots, rp.n_slots);
+            rsops.insert(rsops.end(), bp.ops.begin(), bp.ops.end());
+            rphases.insert(rphases.end(), bp.phases.begin(), bp.phases.end());
             g.rspasses.push_back(rp);
         }
     }
-    if (rphases.empty()) rphases.push_back(SweepPhase());
+    rsops.push_back(RegOp<R>());   // one more is read than there are
+    if (rphases.empty()) rphases.push_back(PhaseBits());
     if (slot_out.empty()) slot_out.push_back(0);
     // Pauli passes
     std::vector<u64> pneed;
@@ -843,6 +874,20 @@ void build_group(Group &g, const Tuning &t) {
         p.accumulate = k > 0 ? 1 : 0;
         p.n_slots = k + 1 == pl.size() ? 1 : 0;
         g.ppasses.push_back(p);
+    }
+    // full-size tiles: works and terms sorted by pattern
+    g.pauli_full = mf == C::MaxBits;
+    std::vector<PauliWork> pworks;
+    std::vector<PauliZ> pzs;
+    if (g.pauli_full) {
+        std::vector<int> ny(g.zmask.size());
+        for (size_t k = 0; k < ny.size(); ++k) ny[k] = __builtin_popcountll(g.xmask[k] & g.zmask[k]);
+        for (size_t k = 0; k < pl.size(); ++k) {
+            const int begin = (int)pworks.size();
+            plan_pauli_pass<R>(pgroups, pl[k].begin, pl[k].end - pl[k].begin, g.zmask, [&](int t) { return ny[t]; },
+                               pl[k].bits, pworks, pzs);
+            g.ppasses[k].op_begin = begin;
+        }
     }
     std::vector<BTermMask> tmask;
     for (u64 z : g.zmask) tmask.push_back(BTermMask{z});
@@ -875,8 +920,10 @@ void build_group(Group &g, const Tuning &t) {
         g.block = nullptr;
     }
     u64 max_part = 0;
-    for (const BPass &p : g.spasses)
-        max_part = std::max<u64>(max_part, (u64)ni * (u64)max_slots * (u64(1) << (n - p.m)));
+    max_part = (u64)ni * (u64)max_slots * (u64(1) << (n - (sregs ? (int)C::SweepBits : g.spasses[0].m)));
+    if (!sregs)
+        for (const BPass &p : g.spasses)
+            max_part = std::max<u64>(max_part, (u64)ni * (u64)max_slots * (u64(1) << (n - p.m)));
     max_part = std::max<u64>(max_part, (u64)ni << (n - g.ppasses.back().m));
     const size_t n_terms = g.zmask.size();
     std::vector<std::pair<size_t, size_t>> parts;   // (offset, bytes)
@@ -897,9 +944,15 @@ void build_group(Group &g, const Tuning &t) {
     const size_t o_gates = carve(sizeof(BGate) * gates.size());
     const size_t o_fops = carve(sizeof(BOp) * fops.size());
     const size_t o_sops = carve(sizeof(BOp) * sops.size());
-    const size_t o_rsops = carve(sizeof(SweepOp<R>) * rsops.size());
-    const size_t o_rph = carve(sizeof(SweepPhase) * rphases.size());
+    const size_t o_rsops = carve(sizeof(RegOp<R>) * rsops.size());
+    const size_t o_rph = carve(sizeof(PhaseBits) * rphases.size());
+    const size_t o_frows = carve(sizeof(BRow<R>) * frows.size());
+    const size_t o_srows = carve(sizeof(BRow<R>) * srows.size());
+    const size_t o_fcoefs = carve(sizeof(R) * kCoefs * ni * frows.size());
+    const size_t o_scoefs = carve(sizeof(R) * kCoefs * ni * srows.size());
     const size_t o_pg = carve(sizeof(PauliGroup) * std::max<size_t>(1, pgroups.size()));
+    const size_t o_pw = carve(sizeof(PauliWork) * pworks.size());
+    const size_t o_pz = carve(sizeof(PauliZ) * pzs.size());
     const size_t o_tm = carve(sizeof(BTermMask) * tmask.size());
     const size_t o_slot = carve(sizeof(int) * slot_out.size());
     const size_t o_pptr = carve(sizeof(int) * pptr.size());
@@ -918,8 +971,16 @@ void build_group(Group &g, const Tuning &t) {
     g.d_fops = reinterpret_cast<BOp *>(g.block + o_fops);
     g.d_sops = reinterpret_cast<BOp *>(g.block + o_sops);
     g.d_rsops = g.block + o_rsops;
-    g.d_rphases = reinterpret_cast<SweepPhase *>(g.block + o_rph);
+    g.d_rphases = reinterpret_cast<PhaseBits *>(g.block + o_rph);
+    g.n_frows = (int)frows.size();
+    g.n_srows = (int)srows.size();
+    g.d_frows = g.block + o_frows;
+    g.d_srows = g.block + o_srows;
+    g.d_fcoefs = g.block + o_fcoefs;
+    g.d_scoefs = g.block + o_scoefs;
     g.d_pgroups = reinterpret_cast<PauliGroup *>(g.block + o_pg);
+    g.d_pworks = reinterpret_cast<PauliWork *>(g.block + o_pw);
+    g.d_pzs = reinterpret_cast<PauliZ *>(g.block + o_pz);
     g.d_tmask = reinterpret_cast<BTermMask *>(g.block + o_tm);
     g.d_slot_out = reinterpret_cast<int *>(g.block + o_slot);
     g.d_pptr = reinterpret_cast<int *>(g.block + o_pptr);
@@ -930,11 +991,18 @@ void build_group(Group &g, const Tuning &t) {
     QG_HIP(hipMemcpyAsync(g.d_gates, gates.data(), sizeof(BGate) * gates.size(), hipMemcpyHostToDevice, s));
     QG_HIP(hipMemcpyAsync(g.d_fops, fops.data(), sizeof(BOp) * fops.size(), hipMemcpyHostToDevice, s));
     QG_HIP(hipMemcpyAsync(g.d_sops, sops.data(), sizeof(BOp) * sops.size(), hipMemcpyHostToDevice, s));
-    QG_HIP(hipMemcpyAsync(g.d_rsops, rsops.data(), sizeof(SweepOp<R>) * rsops.size(), hipMemcpyHostToDevice, s));
-    QG_HIP(hipMemcpyAsync(g.d_rphases, rphases.data(), sizeof(SweepPhase) * rphases.size(), hipMemcpyHostToDevice,
-                          s));
+    QG_HIP(hipMemcpyAsync(g.d_rsops, rsops.data(), sizeof(RegOp<R>) * rsops.size(), hipMemcpyHostToDevice, s));
+    QG_HIP(hipMemcpyAsync(g.d_rphases, rphases.data(), sizeof(PhaseBits) * rphases.size(), hipMemcpyHostToDevice, s));
+    if (!frows.empty())
+        QG_HIP(hipMemcpyAsync(g.d_frows, frows.data(), sizeof(BRow<R>) * frows.size(), hipMemcpyHostToDevice, s));
+    if (!srows.empty())
+        QG_HIP(hipMemcpyAsync(g.d_srows, srows.data(), sizeof(BRow<R>) * srows.size(), hipMemcpyHostToDevice, s));
     if (!pgroups.empty())
         QG_HIP(hipMemcpyAsync(g.d_pgroups, pgroups.data(), sizeof(PauliGroup) * pgroups.size(), hipMemcpyHostToDevice, s));
+    if (!pworks.empty()) {
+        QG_HIP(hipMemcpyAsync(g.d_pworks, pworks.data(), sizeof(PauliWork) * pworks.size(), hipMemcpyHostToDevice, s));
+        QG_HIP(hipMemcpyAsync(g.d_pzs, pzs.data(), sizeof(PauliZ) * pzs.size(), hipMemcpyHostToDevice, s));
+    }
     QG_HIP(hipMemcpyAsync(g.d_tmask, tmask.data(), sizeof(BTermMask) * tmask.size(), hipMemcpyHostToDevice, s));
     QG_HIP(hipMemcpyAsync(g.d_slot_out, slot_out.data(), sizeof(int) * slot_out.size(), hipMemcpyHostToDevice, s));
     QG_HIP(hipMemcpyAsync(g.d_pptr, pptr.data(), sizeof(int) * pptr.size(), hipMemcpyHostToDevice, s));
@@ -959,31 +1027,48 @@ void launch_group_t(Group &g) {
     BMats<R> *mats = static_cast<BMats<R> *>(g.d_mats);
     Cx<R> *psi = static_cast<Cx<R> *>(g.psi), *lam = static_cast<Cx<R> *>(g.lam);
     const u64 nm = ni * (u64)std::max(1, n_gates);
-    if (n_gates > 0)
+    if (n_gates > 0 && !(g.fregs && g.sregs))
         hipLaunchKernelGGL((k_batch_mats<R>), (unsigned)((nm + 255) / 256), 256, 0, s, g.d_gates, n_gates, g.d_params,
                            g.n_params, ni, mats);
+    R *fcoefs = static_cast<R *>(g.d_fcoefs), *scoefs = static_cast<R *>(g.d_scoefs);
+    if (g.n_frows > 0)
+        hipLaunchKernelGGL((k_batch_coefs<R>), (unsigned)((ni * (u64)g.n_frows + 255) / 256), 256, 0, s,
+                           static_cast<const BRow<R> *>(g.d_frows),
+                           g.n_frows, g.d_params, g.n_params, ni, fcoefs);
+    if (g.n_srows > 0)
+        hipLaunchKernelGGL((k_batch_coefs<R>), (unsigned)((ni * (u64)g.n_srows + 255) / 256), 256, 0, s,
+                           static_cast<const BRow<R> *>(g.d_srows),
+                           g.n_srows, g.d_params, g.n_params, ni, scoefs);
     const u64 n_units = (ni << n) / W;
     const int unit_bits = n - (W == 2 ? 1 : 0);
     hipLaunchKernelGGL((k_batch_zero<R>), (unsigned)((n_units + 255) / 256), 256, 0, s, psi, n_units, unit_bits);
-    const Mat2<R> *umats = reinterpret_cast<const Mat2<R> *>(mats);   // U of (item, gate): umats[2 (item n_gates + gate)]
     const u64 piece = launch_piece_items() / kBatchRegThreads;         // register passes: one tile per workgroup
-    for (size_t k = 0; k < g.fpasses.size(); ++k) {
-        const BPass &p = g.fpasses[k];
-        if (p.n_ops == 0) continue;
-        const u64 n_tiles = ni << (n - p.m);
-        if (g.fregs) {
-            const RegProgram<R> &rp = reg_programs<R>(g)[k];
+    if (g.fregs) {
+        const u64 n_tiles = ni << (n - TileCfg<R>::MaxBits);
+        for (const RegProgram<R> &rp : reg_programs<R>(g))
             for (u64 first = 0; first < n_tiles; first += piece)
                 hipLaunchKernelGGL((k_tile_reg<R, TileCfg<R>::MaxBits, kBatchRegThreads, true>),
                                    (unsigned)std::min(piece, n_tiles - first), kBatchRegThreads, 0, s, psi, rp, first,
-                                   umats, n_gates, n);
-            continue;
+                                   (const R *)fcoefs, g.n_frows, n);
+    } else {
+        for (const BPass &p : g.fpasses) {
+            if (p.n_ops == 0) continue;
+            const u64 n_tiles = ni << (n - p.m);
+            const unsigned grid = (unsigned)std::min<u64>(n_tiles, grid_cap);
+            hipLaunchKernelGGL((k_batch_pass<R, C::MaxBits, T>), grid, T, 0, s, psi, p, g.d_fops, mats, n_gates, n,
+                               n_tiles);
         }
-        const unsigned grid = (unsigned)std::min<u64>(n_tiles, grid_cap);
-        hipLaunchKernelGGL((k_batch_pass<R, C::MaxBits, T>), grid, T, 0, s, psi, p, g.d_fops, mats, n_gates, n, n_tiles);
     }
     for (const BPass &p : g.ppasses) {
         const u64 n_tiles = ni << (n - p.m);
+        if (g.pauli_full) {
+            const u64 ppiece = launch_piece_items() / kPauliThreads<R>;
+            for (u64 first = 0; first < n_tiles; first += ppiece)
+                hipLaunchKernelGGL((k_batch_pauli_full<R, C::MaxBits>), (unsigned)std::min(ppiece, n_tiles - first),
+                                   kPauliThreads<R>, 0, s, psi, lam, p, g.d_pworks, g.d_pzs, g.d_coefs,
+                                   (int)g.zmask.size(), n, g.d_partial, first);
+            continue;
+        }
         const unsigned grid = (unsigned)std::min<u64>(n_tiles, grid_cap);
         hipLaunchKernelGGL((k_batch_pauli<R, C::MaxBits, T>), grid, T, 0, s, psi, lam, p, g.d_pgroups, g.d_tmask,
                            g.d_coefs, (int)g.zmask.size(), n, g.d_partial, n_tiles);
@@ -993,27 +1078,26 @@ void launch_group_t(Group &g) {
         const u64 len = u64(1) << (n - p.m);
         hipLaunchKernelGGL(k_rows_sum, (unsigned)ni, 64, 0, s, g.d_partial, len, ni, ni, g.d_zero, 1, g.d_values);
     }
-    for (size_t k = 0; k < g.spasses.size(); ++k) {
-        const BPass &p = g.spasses[k];
-        if (p.n_ops == 0) continue;
-        const u64 tpi = u64(1) << (n - p.m);
+    const size_t n_spasses = g.sregs ? g.rspasses.size() : g.spasses.size();
+    for (size_t k = 0; k < n_spasses; ++k) {
+        if (!g.sregs && g.spasses[k].n_ops == 0) continue;
+        const u64 tpi = u64(1) << (n - (g.sregs ? (int)C::SweepBits : g.spasses[k].m));
         const u64 n_tiles = ni * tpi;
+        const int n_slots = g.sregs ? g.rspasses[k].n_slots : g.spasses[k].n_slots;
         if (g.sregs) {
-            const SweepPass &rp = g.rspasses[k];
-            const Mat2<R> *udmats = umats + 1;   // U^dagger entries
             for (u64 first = 0; first < n_tiles; first += piece)
                 hipLaunchKernelGGL((k_tile_sweep_reg<R, C::SweepBits, kBatchRegThreads, true>),
-                                   (unsigned)std::min(piece, n_tiles - first), kBatchRegThreads, 0, s, psi, lam, rp,
-                                   static_cast<const SweepOp<R> *>(g.d_rsops), g.d_rphases, g.d_partial, n_tiles,
-                                   first, udmats, n_gates, n);
+                                   (unsigned)std::min(piece, n_tiles - first), kBatchRegThreads, 0, s, psi, lam,
+                                   g.rspasses[k], static_cast<const RegOp<R> *>(g.d_rsops), g.d_rphases, g.d_partial,
+                                   n_tiles, first, (const R *)scoefs, g.n_srows, n);
         } else {
             const unsigned grid = (unsigned)std::min<u64>(n_tiles, grid_cap);
-            hipLaunchKernelGGL((k_batch_sweep<R, C::SweepBits, T>), grid, T, 0, s, psi, lam, p, g.d_sops, mats,
-                               n_gates, n, g.d_partial, n_tiles);
+            hipLaunchKernelGGL((k_batch_sweep<R, C::SweepBits, T>), grid, T, 0, s, psi, lam, g.spasses[k], g.d_sops,
+                               mats, n_gates, n, g.d_partial, n_tiles);
         }
-        if (p.n_slots > 0)
-            hipLaunchKernelGGL(k_rows_sum, (unsigned)(ni * (u64)p.n_slots), 64, 0, s, g.d_partial, tpi,
-                               ni * (u64)p.n_slots, ni, g.d_slot_out + g.spass_slot_begin[k], n_gates, g.d_terms);
+        if (n_slots > 0)
+            hipLaunchKernelGGL(k_rows_sum, (unsigned)(ni * (u64)n_slots), 64, 0, s, g.d_partial, tpi,
+                               ni * (u64)n_slots, ni, g.d_slot_out + g.spass_slot_begin[k], n_gates, g.d_terms);
     }
     if (g.n_params > 0) {
         const u64 nq = ni * (u64)g.n_params;
@@ -1347,7 +1431,8 @@ int qghip_batch_describe(const qghip_batch *b, char *buf, int size) {
                      "\"sweep_passes\": %zu}",
                      k ? ", " : "", g.n, g.n_items(), g.ops.size(), g.tune.tile_bits, g.tune.threads,
                      g.tune.grid_per_cu, g.tune.registers, g.fregs ? 1 : 0, g.sregs ? 1 : 0, g.tune.ms,
-                     g.fpasses.size(), g.spasses.size());
+                     !g.fregs ? g.fpasses.size() : b->prec == precFP32 ? g.rprog32.size() : g.rprog64.size(),
+                     g.sregs ? g.rspasses.size() : g.spasses.size());
             out += line;
         }
         out += "]";

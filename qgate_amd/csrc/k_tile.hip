@@ -21,6 +21,7 @@
 #include "kernels.hpp"
 #include "qg_runtime.hpp"
 #include "tile_common.hpp"
+#include "tile_pauli.hpp"
 #include "tile_reg.hpp"
 
 namespace qg {
@@ -183,60 +184,6 @@ void launch_pass(Cx<R> *a, int n_lanes, const PassPlan &plan, int low, int max_b
     hipStream_t s = stream();
     // one workgroup per tile; pieces keep every grid within launch_piece_items() threads
     const u64 piece = launch_piece_items() / kTileThreads;
-    if ((prog.m == C::MaxBits || prog.m == WideCfg<R>::Bits) && use_register_tiles()) {
-        RegProgram<R> rp;
-        rp.n_ops = prog.n_ops;
-        rp.low = prog.low;
-        std::memcpy(rp.pos, prog.pos, sizeof(rp.pos));
-        TileOp<R> tops[C::MaxOps];
-        for (int k = 0; k < prog.n_ops; ++k) {
-            tops[k] = prog.ops[k];
-            TileOp<R> &op = tops[k];
-            const Mat2<R> &mm = op.m;
-            const R zero = R(0), one = R(1);
-            if (op.kind == kOpPair) {
-                const bool swap = mm.m00.re == zero && mm.m00.im == zero && mm.m11.re == zero && mm.m11.im == zero &&
-                                  mm.m01.re == one && mm.m01.im == zero && mm.m10.re == one && mm.m10.im == zero;
-                const bool real = mm.m00.im == zero && mm.m01.im == zero && mm.m10.im == zero && mm.m11.im == zero;
-                op.kind = (short)(swap ? kOpPairSwap : real ? kOpPairReal : kOpPair);
-            } else if (op.kind == kOpDiagLocal && mm.m00.re == one && mm.m00.im == zero) {
-                op.kind = (short)kOpDiagPhase;
-            }
-        }
-        if (prog.m == WideCfg<R>::Bits) {
-            constexpr int WB = WideCfg<R>::Bits, WT = WideCfg<R>::Threads, A = (1 << WB) / WT;
-            if (plan_phases<R>(rp, tops, prog.m, Log2<A>::v, Log2<WT / 64>::v)) {
-                const u64 wpiece = launch_piece_items() / WT;
-                for (u64 first = 0; first < n_tiles; first += wpiece) {
-                    const u64 count = std::min(wpiece, n_tiles - first);
-                    hipLaunchKernelGGL((k_tile_reg<R, WB, WT, false>), (unsigned)count, WT, 0, s, a, rp, first,
-                                       (const Mat2<R> *)nullptr, 0, 0);
-                }
-                QG_HIP(hipGetLastError());
-                return;
-            }
-        } else {
-            constexpr int A = (1 << C::MaxBits) / kTileThreads;
-            if (plan_phases<R>(rp, tops, prog.m, Log2<A>::v, Log2<kTileThreads / 64>::v)) {
-                for (u64 first = 0; first < n_tiles; first += piece) {
-                    const u64 count = std::min(piece, n_tiles - first);
-                    hipLaunchKernelGGL((k_tile_reg<R, C::MaxBits, kTileThreads, false>), (unsigned)count, kTileThreads,
-                                       0, s, a, rp, first, (const Mat2<R> *)nullptr, 0, 0);
-                }
-                QG_HIP(hipGetLastError());
-                return;
-            }
-        }
-    }
-    if (prog.m > C::MaxBits) {
-        // a wide tile whose gates need more register phases than a program holds
-        for (u64 first = 0; first < n_tiles; first += piece) {
-            const u64 count = std::min(piece, n_tiles - first);
-            hipLaunchKernelGGL((k_tile_pass<R, WideCfg<R>::Bits>), (unsigned)count, kTileThreads, 0, s, a, prog, first);
-        }
-        QG_HIP(hipGetLastError());
-        return;
-    }
     for (u64 first = 0; first < n_tiles; first += piece) {
         const u64 count = std::min(piece, n_tiles - first);
         hipLaunchKernelGGL((k_tile_pass<R, C::MaxBits>), (unsigned)count, kTileThreads, 0, s, a, prog, first);
@@ -246,12 +193,29 @@ void launch_pass(Cx<R> *a, int n_lanes, const PassPlan &plan, int low, int max_b
 
 // ---- adjoint sweep ----------------------------------------------------------------------
 
+template <class R>
+struct SweepOp {
+    Mat2<R> udag;       // applied to phi and lambda
+    Mat2<R> gen;        // generator of a rotation (entries 0, +-1, +-i)
+    u64 gctrl;
+    unsigned lctrl;
+    int target;         // local bit (pair, diag-local) or state bit (diag-outer)
+    int kind;           // (dwords: a uniform dword field is one scalar load)
+    int slot;           // gradient slot within the pass, -1 for fixed gates
+};
+
+struct LdsSweepPass {
+    int m, low;
+    int op_begin, n_ops, n_slots;
+    alignas(4) signed char pos[kTilePosMax];
+};
+
 // One pass of the adjoint backward sweep over a phi tile and a lambda tile: for each op in
 // order, the gradient term Im<lambda| C G |phi> of the tile (FP64, written to
 // partial[slot * n_tiles + tile]) and then phi, lambda <- U^dagger.
 template <class R, int MB>
 __global__ __launch_bounds__(kTileThreads) void k_tile_sweep(Cx<R> *__restrict__ phi, Cx<R> *__restrict__ lam,
-                                                             const SweepPass pass,
+                                                             const LdsSweepPass pass,
                                                              const SweepOp<R> *__restrict__ ops,
                                                              double *__restrict__ partial, u64 n_tiles,
                                                              u64 first) {
@@ -378,7 +342,7 @@ struct PauliCfg<double> {
 
 struct PauliPass {
     int m, low;
-    int g_begin, n_groups;
+    int g_begin, n_groups;   // groups, or works of a pass on full-size tiles
     int accumulate;     // add to lambda (later passes) instead of writing it
     int dot;            // last pass: partial[tile] = Re<psi|lambda> over the tile
     alignas(4) signed char pos[kTilePosMax];
@@ -435,6 +399,29 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_pauli(const Cx<R> *__rest
     }
     if (pass.dot) {
         dot = block_sum_tile<kTileThreads>(dot, scratch);
+        if (threadIdx.x == 0) partial[tile] = dot;
+    }
+}
+
+// The same for full-size tiles (tile_pauli.hpp).
+template <class R, int MB>
+__global__ __launch_bounds__((kPauliThreads<R>)) void k_tile_pauli_full(const Cx<R> *__restrict__ psi,
+                                                                   Cx<R> *__restrict__ lam, const PauliPass pass,
+                                                                   const PauliWork *__restrict__ works,
+                                                                   const PauliZ *__restrict__ zs,
+                                                                   const double *__restrict__ coefs,
+                                                                   double *__restrict__ partial, u64 first) {
+    __shared__ Cx<R> tp[1 << MB];
+    __shared__ double scratch[kPauliThreads<R> / 64];
+    constexpr int lw = Unit<R>::W == 2 ? 1 : 0;
+    const u64 tile = first + blockIdx.x;
+    const u64 base = tile_base(tile, pass.pos, MB);
+    tile_to_lds<R, kPauliThreads<R>, (1 << (MB - lw)) / kPauliThreads<R>>(tp, psi, base, pass.pos, MB, pass.low);
+    __syncthreads();
+    double dot = pauli_full_tile<R, MB>(tp, lam, base, pass.pos, pass.low, pass.accumulate != 0, pass.dot != 0,
+                                        works + pass.g_begin, pass.n_groups, zs, coefs);
+    if (pass.dot) {
+        dot = block_sum_tile<kPauliThreads<R>>(dot, scratch);
         if (threadIdx.x == 0) partial[tile] = dot;
     }
 }
@@ -507,6 +494,47 @@ static std::vector<QueuedGate> merge_lane_runs(const std::vector<QueuedGate> &ga
     return out;
 }
 
+// Register passes over a whole gate sequence, in tiles of M bits and T threads.
+template <class R, int M, int T>
+static void run_register_passes(Cx<R> *a, int n_lanes, const std::vector<QueuedGate> &gates_in, int low) {
+    constexpr int A = (1 << M) / T;
+    const std::vector<RegGate> gates =
+        merged_gates((int)gates_in.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates_in[i]; });
+    const std::vector<BuiltPass<R>> passes = build_passes<R>(gates, n_lanes, M, low, Log2<A>::v, Log2<T / 64>::v,
+                                                             TileCfg<R>::MaxRegOps, TileCfg<R>::MaxRegOps, kMaxPhases);
+    hipStream_t s = stream();
+    const u64 n_tiles = u64(1) << (n_lanes - M);
+    const u64 piece = launch_piece_items() / T;   // keeps every grid within launch_piece_items() threads
+    for (const BuiltPass<R> &bp : passes) {
+        // a pass that comes to one gate streams faster than through a tile
+        const RegGate &g0 = gates[bp.gates[0]];
+        bool lone = bp.gates.size() == 1;
+        GateMatrix m = g0.m;
+        if (g0.ctrl.empty() && !lone) {
+            lone = true;
+            for (size_t k = 1; k < bp.gates.size() && lone; ++k) {
+                const RegGate &g = gates[bp.gates[k]];
+                lone = g.ctrl.empty() && g.target == g0.target;
+                GateMatrix p;
+                for (int r = 0; r < 2; ++r)
+                    for (int c = 0; c < 2; ++c) p.m[r][c] = g.m.m[r][0] * m.m[0][c] + g.m.m[r][1] * m.m[1][c];
+                m = p;
+            }
+        }
+        if (lone) {
+            launch_gate<R>(a, n_lanes, m, g0.ctrl, g0.target);
+            continue;
+        }
+        const RegProgram<R> rp = reg_program(bp);
+        for (u64 first = 0; first < n_tiles; first += piece) {
+            const u64 count = std::min(piece, n_tiles - first);
+            hipLaunchKernelGGL((k_tile_reg<R, M, T, false>), (unsigned)count, T, 0, s, a, rp, first,
+                               (const R *)nullptr, 0, 0);
+        }
+    }
+    QG_HIP(hipGetLastError());
+}
+
 template <class R>
 void apply_gate_sequence(Cx<R> *a, int n_lanes, const std::vector<QueuedGate> &gates_in, int max_bits,
                          int low_bits) {
@@ -517,6 +545,10 @@ void apply_gate_sequence(Cx<R> *a, int n_lanes, const std::vector<QueuedGate> &g
     const int mb = std::min(max_bits > 0 ? std::min(max_bits, cap) : cap, n_lanes);
     const int low = std::min(low_bits >= 0 ? low_bits : C::Low, mb);
     QG_REQUIRE(Unit<R>::W == 1 || low >= 1, "complex64 tiles need bit 0");
+    if (use_register_tiles() && low < mb) {
+        if (mb == WideCfg<R>::Bits) return run_register_passes<R, WideCfg<R>::Bits, WideCfg<R>::Threads>(a, n_lanes, gates_in, low);
+        if (mb == C::MaxBits) return run_register_passes<R, C::MaxBits, kTileThreads>(a, n_lanes, gates_in, low);
+    }
     const std::vector<QueuedGate> gates = merge_lane_runs(gates_in, n_lanes);
     // Each pass scans the gates not yet applied in program order and takes every gate that
     // commutes with all the gates it left out before it and whose target is a tile bit (or
@@ -577,110 +609,190 @@ void apply_gate_sequence(Cx<R> *a, int n_lanes, const std::vector<QueuedGate> &g
 template void apply_gate_sequence<float>(Cx<float> *, int, const std::vector<QueuedGate> &, int, int);
 template void apply_gate_sequence<double>(Cx<double> *, int, const std::vector<QueuedGate> &, int, int);
 
-template <class R>
-void adjoint_sweep(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<SweepGate> &gates, double *d_terms,
-                   int max_bits, int low_bits) {
-    typedef SweepCfg<R> C;
-    const bool regs = use_register_tiles();
-    const int cap = regs ? C::RegBits : C::LdsBits;
-    const int mb = std::min(max_bits > 0 ? std::min(max_bits, cap) : cap, n_lanes);
-    const int low = std::min(low_bits >= 0 ? low_bits : C::Low, mb);
-    // plan the passes as apply_gate_sequence does (each pass takes every gate not yet swept
-    // that commutes with the gates it left out before it and fits the tile), with at most
-    // kMaxSweepSlots rotations a pass. A gate counts as diagonal only if it is for every
-    // parameter value (a fixed gate, or generator Z), so a reordered rotation has the same
-    // derivative. `order` lists the gates pass by pass; a pass is a range [begin, end) of it.
-    struct Plan {
-        std::vector<int> bits;
-        int begin, end, slots;
-    };
-    constexpr int kLookahead = 256;
-    const int n_gates = (int)gates.size();
-    std::vector<int> order;
-    order.reserve(n_gates);
-    std::vector<char> done(n_gates, 0);
-    std::vector<unsigned char> held(n_lanes);   // 0 free, 1 used diagonally, 2 otherwise
-    std::vector<Plan> plans;
-    for (int first = 0; first < n_gates;) {
-        Plan cur;
-        for (int b = 0; b < low; ++b) cur.bits.push_back(b);
-        cur.begin = (int)order.size();
-        cur.slots = 0;
-        auto has = [&](int b) { return std::find(cur.bits.begin(), cur.bits.end(), b) != cur.bits.end(); };
-        std::fill(held.begin(), held.end(), (unsigned char)0);
-        int left = 0, held_all = 0;
-        for (int i = first; i < n_gates; ++i) {
-            if (done[i]) continue;
-            const SweepGate &g = gates[i];
-            const bool diag = is_diagonal(g.udag) && (g.pauli == 0 || g.pauli == 3);
-            bool conflict = diag ? held[g.target] == 2 : held[g.target] != 0;
-            for (int c : g.ctrl) conflict = conflict || held[c] == 2;
-            const bool slot_ok = g.pauli == 0 || cur.slots < kMaxSweepSlots;
-            if (!conflict && slot_ok && (diag || has(g.target) || (int)cur.bits.size() < mb)) {
-                if (!(diag || has(g.target))) cur.bits.push_back(g.target);
-                if (g.pauli != 0) ++cur.slots;
-                order.push_back(i);
-                done[i] = 1;
-                continue;
-            }
-            auto hold = [&](int lane, unsigned char v) {
-                if (held[lane] < 2 && v == 2) ++held_all;
-                held[lane] = std::max(held[lane], v);
-            };
-            hold(g.target, diag ? 1 : 2);
-            for (int c : g.ctrl) hold(c, 1);
-            if (++left >= kLookahead || held_all == n_lanes) break;
+// The register gates of the gate list of a sweep: rotations whole (their gradient terms are
+// taken right before them), fixed gates split as in the forward pass.
+static std::vector<RegGate> sweep_gates(const std::vector<SweepGate> &gates) {
+    std::vector<RegGate> out;
+    out.reserve(gates.size() + gates.size() / 4);
+    for (int i = 0; i < (int)gates.size(); ++i) {
+        const SweepGate &g = gates[i];
+        if (g.pauli == 0) {
+            append_fixed(out, g.udag, g.ctrl, g.target, i);
+            continue;
         }
-        if ((int)order.size() == cur.begin) {   // no tile bit left (tile bits == low bits): as before,
-            const SweepGate &g = gates[first];     // the first gate widens the tile by its target
-            cur.bits.push_back(g.target);
-            if (g.pauli != 0) ++cur.slots;
-            order.push_back(first);
-            done[first] = 1;
+        RegGate r;
+        r.kind = g.pauli == 3 ? kGateDiag : !g.ctrl.empty() ? kGateAny : g.pauli == 1 ? kGateX : kGateY;
+        r.target = g.target;
+        r.pauli = g.pauli;
+        r.source = i;
+        r.ctrl = g.ctrl;
+        r.m = g.udag;
+        out.push_back(r);
+    }
+    return out;
+}
+
+// Gradient terms of consecutive passes: their partial rows (one per slot, one entry per tile)
+// accumulate in one device buffer, up to kSweepPartialBytes, and are summed by one launch when
+// it is full or the sweep ends, not by a small launch after each pass.
+class SweepRows {
+  public:
+    // slots[p]: gradient slots of pass p. Device tables of `table_bytes` are allocated with the rows.
+    SweepRows(const std::vector<int> &slots, u64 n_tiles, size_t table_bytes) : n_tiles_(n_tiles) {
+        int most = 0, total = 0;
+        for (int n : slots) {
+            most = std::max(most, n);
+            total += n;
         }
-        cur.end = (int)order.size();
-        plans.push_back(cur);
-        while (first < n_gates && done[first]) ++first;
+        const size_t row_bytes = sizeof(double) * (size_t)n_tiles;
+        cap_ = (int)std::max<size_t>((size_t)most, std::min<size_t>((size_t)total, kSweepPartialBytes / row_bytes));
+        o_part_ = (table_bytes + 255) & ~size_t(255);
+        bytes_ = o_part_ + std::max<size_t>(8, row_bytes * (size_t)cap_);
+        buf_ = static_cast<char *>(dev_alloc(bytes_));
+    }
+    ~SweepRows() { dev_free(buf_, bytes_); }
+    char *tables() const { return buf_; }
+    // rows of the next pass; sums the pending ones first if it would not fit
+    double *rows(int n_slots, const int *d_slot_gate, double *d_terms) {
+        if (pending_ + n_slots > cap_) sum(d_slot_gate, d_terms);
+        double *at = part() + (u64)pending_ * n_tiles_;
+        pending_ += n_slots;
+        return at;
+    }
+    // terms of the pending rows land at d_terms[gate index]
+    void sum(const int *d_slot_gate, double *d_terms) {
+        if (pending_ > 0)
+            hipLaunchKernelGGL(k_slot_rows, (unsigned)pending_, kRowThreads, 0, stream(), part(), n_tiles_,
+                               d_slot_gate + begin_, d_terms);
+        begin_ += pending_;
+        pending_ = 0;
     }
 
+  private:
+    double *part() const { return reinterpret_cast<double *>(buf_ + o_part_); }
+    u64 n_tiles_;
+    int cap_ = 0, pending_ = 0, begin_ = 0;
+    size_t o_part_ = 0, bytes_ = 0;
+    char *buf_ = nullptr;
+};
+
+// Copies host tables one after another (each 256-byte aligned) to device memory.
+class TableLayout {
+  public:
+    template <class T>
+    size_t add(const std::vector<T> &v) {
+        const size_t at = (bytes_ + 255) & ~size_t(255);
+        bytes_ = at + sizeof(T) * v.size();
+        parts_.push_back(Part{at, sizeof(T) * v.size(), v.data()});
+        return at;
+    }
+    size_t bytes() const { return bytes_; }
+    void upload(char *dst) const {
+        for (const Part &p : parts_)
+            if (p.bytes > 0) QG_HIP(hipMemcpyAsync(dst + p.at, p.src, p.bytes, hipMemcpyHostToDevice, stream()));
+    }
+
+  private:
+    struct Part {
+        size_t at, bytes;
+        const void *src;
+    };
+    std::vector<Part> parts_;
+    size_t bytes_ = 0;
+};
+
+template <class R>
+static void sweep_in_registers(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<SweepGate> &gates,
+                               double *d_terms, int low) {
+    typedef SweepCfg<R> C;
     constexpr int A = (1 << C::RegBits) / C::RegThreads;
-    // device tables: ops (pass by pass), phases of register passes, slot -> gate index
-    std::vector<SweepOp<R>> hops(std::max<size_t>(1, gates.size()));
-    std::vector<SweepPhase> hphases;
-    std::vector<int> slot_gate;
-    std::vector<SweepPass> passes;
-    std::vector<bool> pass_regs;
-    int max_slots = 0;
-    for (const Plan &pl : plans) {
-        std::vector<int> bits(pl.bits);
-        for (int b = 0; (int)bits.size() < mb && b < n_lanes; ++b)
-            if (std::find(bits.begin(), bits.end(), b) == bits.end()) bits.push_back(b);
-        std::sort(bits.begin(), bits.end());
+    const std::vector<RegGate> rg = sweep_gates(gates);
+    const std::vector<BuiltPass<R>> passes = build_passes<R>(
+        rg, n_lanes, C::RegBits, low, Log2<A>::v, Log2<C::RegThreads / 64>::v, 1 << 30, 1 << 30,
+        1 << 30);
+    if (passes.empty()) return;
+    std::vector<RegOp<R>> ops;
+    std::vector<PhaseBits> phases;
+    std::vector<int> slot_gate, slots;
+    std::vector<SweepPass> sp;
+    for (const BuiltPass<R> &bp : passes) {
         SweepPass ps;
-        ps.m = (int)bits.size();
-        ps.low = low;
-        ps.op_begin = pl.begin;
-        ps.n_ops = pl.end - pl.begin;
-        ps.phase_begin = (int)hphases.size();
-        ps.n_phases = 0;
-        for (int j = 0; j < 16; ++j) ps.pos[j] = j < ps.m ? (signed char)bits[j] : (signed char)0;
+        ps.low = bp.low;
+        ps.op_begin = (int)ops.size();
+        ps.phase_begin = (int)phases.size();
+        ps.n_phases = (int)bp.phases.size();
+        ps.n_slots = (int)bp.slot_gate.size();
+        set_positions(ps.pos, bp.bits);
+        ops.insert(ops.end(), bp.ops.begin(), bp.ops.end());
+        phases.insert(phases.end(), bp.phases.begin(), bp.phases.end());
+        for (int gi : bp.slot_gate) slot_gate.push_back(rg[gi].source);
+        slots.push_back(ps.n_slots);
+        sp.push_back(ps);
+    }
+    ops.push_back(RegOp<R>());   // one more is read than there are
+    hipStream_t s = stream();
+    const u64 n_tiles = u64(1) << (n_lanes - C::RegBits);
+    TableLayout tab;
+    const size_t o_ops = tab.add(ops), o_ph = tab.add(phases), o_sg = tab.add(slot_gate);
+    SweepRows rows(slots, n_tiles, tab.bytes());
+    tab.upload(rows.tables());
+    const RegOp<R> *d_ops = reinterpret_cast<const RegOp<R> *>(rows.tables() + o_ops);
+    const PhaseBits *d_ph = reinterpret_cast<const PhaseBits *>(rows.tables() + o_ph);
+    const int *d_sg = reinterpret_cast<const int *>(rows.tables() + o_sg);
+    const u64 piece = launch_piece_items() / (u64)C::RegThreads;
+    for (const SweepPass &ps : sp) {
+        double *part = rows.rows(ps.n_slots, d_sg, d_terms);
+        for (u64 first = 0; first < n_tiles; first += piece) {
+            const u64 count = std::min(piece, n_tiles - first);
+            hipLaunchKernelGGL((k_tile_sweep_reg<R, C::RegBits, C::RegThreads, false>), (unsigned)count, C::RegThreads,
+                               0, s, phi, lam, ps, d_ops, d_ph, part, n_tiles, first, (const R *)nullptr, 0, 0);
+        }
+        QG_HIP(hipGetLastError());
+    }
+    rows.sum(d_sg, d_terms);
+    QG_HIP(hipGetLastError());
+    QG_HIP(hipStreamSynchronize(s));   // the tables are host temporaries
+}
+
+template <class R>
+static void sweep_in_lds(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<SweepGate> &gates, double *d_terms,
+                         int mb, int low) {
+    typedef SweepCfg<R> C;
+    const int n_gates = (int)gates.size();
+    // a gate counts as diagonal only if it is for every parameter value (a fixed gate, or
+    // generator Z), so a reordered rotation has the same derivative
+    std::vector<PlanGate> pg(n_gates);
+    for (int i = 0; i < n_gates; ++i) {
+        const SweepGate &g = gates[i];
+        pg[i] = PlanGate{g.target, &g.ctrl, is_diagonal(g.udag) && (g.pauli == 0 || g.pauli == 3), 1,
+                         g.pauli != 0 ? 1 : 0};
+    }
+    std::vector<char> done(n_gates, 0);
+    std::vector<SweepOp<R>> ops;
+    std::vector<int> slot_gate, slots;
+    std::vector<LdsSweepPass> passes;
+    for (int first = 0; first < n_gates;) {
+        PassBits pb = next_pass(pg, done, first, n_lanes, mb, low, 1 << 30, kMaxSweepSlots);
+        if (pb.gates.empty()) {   // no tile bit left (tile bits == low bits): the first gate widens the tile
+            const int t = gates[first].target;
+            pb.gates.push_back(first);
+            done[first] = 1;
+            pb.bits.insert(std::upper_bound(pb.bits.begin(), pb.bits.end(), t), t);
+        }
+        LdsSweepPass ps;
+        ps.m = (int)pb.bits.size();
+        QG_REQUIRE(ps.m <= C::LdsBits, "adjoint sweep: tile of %d bits", ps.m);
+        ps.low = pb.low;
+        ps.op_begin = (int)ops.size();
+        ps.n_ops = (int)pb.gates.size();
+        set_positions(ps.pos, pb.bits);
         int local[64];
         for (int b = 0; b < 64; ++b) local[b] = -1;
-        for (int j = 0; j < ps.m; ++j) local[bits[j]] = j;
-        if (regs && ps.m == C::RegBits)   // diagonal gates where none of their lanes is a register bit
-            place_diagonals(
-                order, pl.begin, pl.end, local, ps.m, Log2<A>::v, Log2<C::RegThreads / 64>::v,
-                [&](int gi) { return is_diagonal(gates[gi].udag) && (gates[gi].pauli == 0 || gates[gi].pauli == 3); },
-                [&](int gi) { return gates[gi].target; },
-                [&](int gi) {
-                    std::vector<int> l(gates[gi].ctrl);
-                    l.push_back(gates[gi].target);
-                    return l;
-                });
-        int slots = 0;
-        for (int i = pl.begin; i < pl.end; ++i) {
-            const SweepGate &g = gates[order[i]];
-            SweepOp<R> &op = hops[i];
+        for (int j = 0; j < ps.m; ++j) local[pb.bits[j]] = j;
+        int n_slots = 0;
+        for (int gi : pb.gates) {
+            const SweepGate &g = gates[gi];
+            SweepOp<R> op;
             op.udag = round_matrix<R>(g.udag);
             GateMatrix gen;
             set_pauli(gen, g.pauli);
@@ -693,109 +805,53 @@ void adjoint_sweep(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<SweepG
                 else
                     op.gctrl |= u64(1) << c;
             }
-            const bool diag = is_diagonal(g.udag) && (g.pauli == 0 || g.pauli == 3);
-            if (local[g.target] >= 0) {
-                op.target = (short)local[g.target];
-                op.kind = (short)(diag ? kOpDiagLocal : kOpPair);
-            } else {
-                QG_REQUIRE(diag, "adjoint sweep: non-diagonal gate outside the tile");
-                op.target = (short)g.target;
-                op.kind = (short)kOpDiagOuter;
-            }
-            op.form = sweep_form(g.udag, g.pauli, op.kind != kOpPair);
-            op.slot = g.pauli != 0 ? slots++ : -1;
-            if (g.pauli != 0) slot_gate.push_back(order[i]);
+            op.target = local[g.target] >= 0 ? local[g.target] : g.target;
+            op.kind = local[g.target] < 0 ? kOpDiagOuter : pg[gi].diag ? kOpDiagLocal : kOpPair;
+            QG_REQUIRE(op.kind != kOpDiagOuter || pg[gi].diag, "adjoint sweep: non-diagonal gate outside the tile");
+            op.slot = g.pauli != 0 ? n_slots++ : -1;
+            if (g.pauli != 0) slot_gate.push_back(gi);
+            ops.push_back(op);
         }
-        ps.n_slots = slots;
-        const bool use_regs = regs && ps.m == C::RegBits;
-        QG_REQUIRE(use_regs || ps.m <= C::LdsBits, "adjoint sweep: tile of %d bits", ps.m);
-        if (use_regs) {
-            std::vector<int> pair(ps.n_ops);
-            for (int k = 0; k < ps.n_ops; ++k)
-                pair[k] = hops[pl.begin + k].kind == kOpPair ? hops[pl.begin + k].target : -1;
-            const std::vector<PhaseLayout> L = plan_phase_layouts(pair, ps.m, Log2<A>::v, Log2<C::RegThreads / 64>::v);
-            for (const PhaseLayout &P : L) {
-                for (int k = P.begin; k < P.end; ++k) {
-                    SweepOp<R> &op = hops[pl.begin + k];
-                    const RegSplit r = split_for_phase(P, op.kind, op.target, op.lctrl);
-                    op.rkind = r.kind;
-                    op.rtarget = r.target;
-                    op.creg = r.creg;
-                    op.cthr = r.cthr;
-                }
-                hphases.push_back(phase_bits(P));
-            }
-            ps.n_phases = (int)L.size();
-            QG_REQUIRE(ps.n_phases > 0, "adjoint sweep: register pass without phases");
-        }
-        pass_regs.push_back(use_regs);
-        max_slots = std::max(max_slots, slots);
+        ps.n_slots = n_slots;
+        slots.push_back(n_slots);
         passes.push_back(ps);
+        while (first < n_gates && done[first]) ++first;
     }
     if (passes.empty()) return;
-    if (hphases.empty()) hphases.push_back(SweepPhase());
-    if (slot_gate.empty()) slot_gate.push_back(0);
-
     hipStream_t s = stream();
-    // Every pass has the same tile count (tiles are filled up to mb bits). The partial rows of
-    // consecutive passes accumulate in one buffer (up to kSweepPartialBytes) and are summed
-    // by one launch when it is full or the sweep ends, not by a small launch after each pass.
     const u64 n_tiles = u64(1) << (n_lanes - passes[0].m);
-    for (const SweepPass &ps : passes) QG_REQUIRE(ps.m == passes[0].m, "adjoint sweep: passes of unequal tiles");
-    int total_slots = 0;
-    for (const SweepPass &ps : passes) total_slots += ps.n_slots;
-    const size_t row_bytes = sizeof(double) * (size_t)n_tiles;
-    const int cap_slots = (int)std::max<size_t>(
-        (size_t)max_slots, std::min<size_t>((size_t)total_slots, kSweepPartialBytes / row_bytes));
-    const size_t part_bytes = std::max<size_t>(8, row_bytes * (size_t)cap_slots);
-    const size_t ops_bytes = sizeof(SweepOp<R>) * hops.size();
-    const size_t ph_bytes = sizeof(SweepPhase) * hphases.size();
-    const size_t sg_bytes = sizeof(int) * slot_gate.size();
-    const size_t o_ph = (ops_bytes + 255) & ~size_t(255), o_sg = (o_ph + ph_bytes + 255) & ~size_t(255);
-    const size_t o_part = (o_sg + sg_bytes + 255) & ~size_t(255);
-    const size_t total = o_part + part_bytes;
-    char *buf = static_cast<char *>(dev_alloc(total));
-    SweepOp<R> *d_ops = reinterpret_cast<SweepOp<R> *>(buf);
-    SweepPhase *d_ph = reinterpret_cast<SweepPhase *>(buf + o_ph);
-    int *d_sg = reinterpret_cast<int *>(buf + o_sg);
-    double *d_part = reinterpret_cast<double *>(buf + o_part);
-    hipError_t e = hipMemcpyAsync(d_ops, hops.data(), ops_bytes, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_ph, hphases.data(), ph_bytes, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_sg, slot_gate.data(), sg_bytes, hipMemcpyHostToDevice, s);
-    int pending = 0, pending_begin = 0;   // rows in the buffer, and the slot_gate index of the first
-    auto sum_rows = [&]() {                // terms of the pending rows land at d_terms[gate index]
-        if (pending > 0)
-            hipLaunchKernelGGL(k_slot_rows, (unsigned)pending, kRowThreads, 0, s, d_part, n_tiles,
-                               d_sg + pending_begin, d_terms);
-        pending_begin += pending;
-        pending = 0;
-    };
-    for (size_t pi = 0; pi < passes.size() && e == hipSuccess; ++pi) {
-        const SweepPass &ps = passes[pi];
-        if (pending + ps.n_slots > cap_slots) sum_rows();
-        double *part = d_part + (u64)pending * n_tiles;
-        const int threads = pass_regs[pi] ? C::RegThreads : kTileThreads;
-        const u64 piece = launch_piece_items() / (u64)threads;
-        for (u64 first = 0; first < n_tiles; first += piece) {
-            const u64 count = std::min(piece, n_tiles - first);
-            if (pass_regs[pi])
-                hipLaunchKernelGGL((k_tile_sweep_reg<R, C::RegBits, C::RegThreads, false>), (unsigned)count,
-                                   C::RegThreads, 0, s, phi, lam, ps, d_ops, d_ph, part, n_tiles, first,
-                                   (const Mat2<R> *)nullptr, 0, 0);
-            else
-                hipLaunchKernelGGL((k_tile_sweep<R, C::LdsBits>), (unsigned)count, kTileThreads, 0, s, phi, lam, ps,
-                                   d_ops, part, n_tiles, first);
-        }
-        pending += ps.n_slots;
-        e = hipGetLastError();
+    for (const LdsSweepPass &ps : passes) QG_REQUIRE(ps.m == passes[0].m, "adjoint sweep: passes of unequal tiles");
+    TableLayout tab;
+    const size_t o_ops = tab.add(ops), o_sg = tab.add(slot_gate);
+    SweepRows rows(slots, n_tiles, tab.bytes());
+    tab.upload(rows.tables());
+    const SweepOp<R> *d_ops = reinterpret_cast<const SweepOp<R> *>(rows.tables() + o_ops);
+    const int *d_sg = reinterpret_cast<const int *>(rows.tables() + o_sg);
+    const u64 piece = launch_piece_items() / kTileThreads;
+    for (const LdsSweepPass &ps : passes) {
+        double *part = rows.rows(ps.n_slots, d_sg, d_terms);
+        for (u64 first = 0; first < n_tiles; first += piece)
+            hipLaunchKernelGGL((k_tile_sweep<R, C::LdsBits>), (unsigned)std::min(piece, n_tiles - first), kTileThreads,
+                               0, s, phi, lam, ps, d_ops, part, n_tiles, first);
+        QG_HIP(hipGetLastError());
     }
-    if (e == hipSuccess) {
-        sum_rows();
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(s);   // the tables are host temporaries
-    dev_free(buf, total);
-    QG_HIP(e);
+    rows.sum(d_sg, d_terms);
+    QG_HIP(hipGetLastError());
+    QG_HIP(hipStreamSynchronize(s));   // the tables are host temporaries
+}
+
+template <class R>
+void adjoint_sweep(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<SweepGate> &gates, double *d_terms,
+                   int max_bits, int low_bits) {
+    typedef SweepCfg<R> C;
+    const bool regs = use_register_tiles();
+    const int cap = regs ? C::RegBits : C::LdsBits;
+    const int mb = std::min(max_bits > 0 ? std::min(max_bits, cap) : cap, n_lanes);
+    const int low = std::min(low_bits >= 0 ? low_bits : C::Low, mb);
+    if (regs && mb == C::RegBits && low < mb)
+        sweep_in_registers<R>(phi, lam, n_lanes, gates, d_terms, low);
+    else
+        sweep_in_lds<R>(phi, lam, n_lanes, gates, d_terms, mb, low);
 }
 
 template void adjoint_sweep<float>(Cx<float> *, Cx<float> *, int, const std::vector<SweepGate> &, double *, int,
@@ -885,37 +941,66 @@ double pauli_expectation(const Cx<R> *psi, Cx<R> *lam, int n_lanes, const std::v
     passes.back().dot = 1;
 
     hipStream_t s = stream();
-    const size_t gbytes = sizeof(PauliGroup) * std::max<size_t>(1, groups.size());
-    const size_t tbytes = sizeof(PauliTerm) * std::max<size_t>(1, terms.size());
-    const u64 n_tiles_last = u64(1) << (n_lanes - passes.back().m);
-    const size_t pbytes = sizeof(double) * (size_t)(n_tiles_last + 1);
-    char *buf = static_cast<char *>(dev_alloc(gbytes + tbytes + pbytes));
-    PauliGroup *d_groups = reinterpret_cast<PauliGroup *>(buf);
-    PauliTerm *d_terms = reinterpret_cast<PauliTerm *>(buf + gbytes);
-    double *d_part = reinterpret_cast<double *>(buf + gbytes + tbytes);
-    Runtime &rt = runtime();
-    hipError_t e = hipMemcpyAsync(d_groups, groups.data(), sizeof(PauliGroup) * groups.size(), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(d_terms, terms.data(), sizeof(PauliTerm) * terms.size(), hipMemcpyHostToDevice, s);
-    for (size_t pi = 0; pi < passes.size() && e == hipSuccess; ++pi) {
-        const PauliPass &ps = passes[pi];
-        const u64 n_tiles = u64(1) << (n_lanes - ps.m);
-        const u64 piece = launch_piece_items() / kTileThreads;
-        for (u64 first = 0; first < n_tiles; first += piece) {
-            const u64 count = std::min(piece, n_tiles - first);
-            hipLaunchKernelGGL((k_tile_pauli<R, C::MaxBits>), (unsigned)count, kTileThreads, 0, s, psi, lam, ps,
-                               d_groups, d_terms, d_part, first);
+    const bool full = mb == C::MaxBits;
+    std::vector<PauliWork> works;
+    std::vector<PauliZ> zs;
+    std::vector<double> coefs;
+    if (full) {
+        std::vector<u64> zmask;
+        std::vector<int> ny;
+        for (const PauliGroup &g : groups)
+            for (int k = g.first; k < g.first + g.count; ++k) {
+                QG_REQUIRE(k == (int)zmask.size(), "Pauli groups out of order");
+                zmask.push_back(terms[k].zmask);
+                ny.push_back(__builtin_popcountll(g.xmask & terms[k].zmask));
+                coefs.push_back(terms[k].cre);
+                coefs.push_back(terms[k].cim);
+            }
+        for (PauliPass &ps : passes) {
+            const std::vector<int> bits(ps.pos, ps.pos + ps.m);
+            const int begin = (int)works.size();
+            plan_pauli_pass<R>(groups, ps.g_begin, ps.n_groups, zmask, [&](int k) { return ny[k]; }, bits, works, zs);
+            ps.g_begin = begin;
         }
-        e = hipGetLastError();
     }
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_sum_slots, 1, kRowThreads, 0, s, d_part, n_tiles_last, d_part + n_tiles_last);
-        e = hipGetLastError();
+    TableLayout tab;
+    const size_t o_a = full ? tab.add(works) : tab.add(groups), o_b = full ? tab.add(zs) : tab.add(terms);
+    const size_t o_c = tab.add(coefs);
+    const u64 n_tiles_last = u64(1) << (n_lanes - passes.back().m);
+    const size_t o_part = (tab.bytes() + 255) & ~size_t(255);
+    const size_t bytes = o_part + sizeof(double) * (size_t)n_tiles_last;
+    char *buf = static_cast<char *>(dev_alloc(bytes));
+    double *d_part = reinterpret_cast<double *>(buf + o_part);
+    Runtime &rt = runtime();
+    hipError_t e = hipSuccess;
+    try {
+        tab.upload(buf);
+        for (const PauliPass &ps : passes) {
+            const u64 n_tiles = u64(1) << (n_lanes - ps.m);
+            const u64 piece = launch_piece_items() / (full ? kPauliThreads<R> : kTileThreads);
+            for (u64 first = 0; first < n_tiles; first += piece) {
+                const unsigned count = (unsigned)std::min(piece, n_tiles - first);
+                if (full)
+                    hipLaunchKernelGGL((k_tile_pauli_full<R, C::MaxBits>), count, kPauliThreads<R>, 0, s, psi, lam, ps,
+                                       reinterpret_cast<const PauliWork *>(buf + o_a),
+                                       reinterpret_cast<const PauliZ *>(buf + o_b),
+                                       reinterpret_cast<const double *>(buf + o_c), d_part, first);
+                else
+                    hipLaunchKernelGGL((k_tile_pauli<R, C::MaxBits>), count, kTileThreads, 0, s, psi, lam, ps,
+                                       reinterpret_cast<const PauliGroup *>(buf + o_a),
+                                       reinterpret_cast<const PauliTerm *>(buf + o_b), d_part, first);
+            }
+            QG_HIP(hipGetLastError());
+        }
+        // the total goes straight to pinned host memory
+        hipLaunchKernelGGL(k_sum_slots, 1, kRowThreads, 0, s, d_part, n_tiles_last, rt.h_pinned);
+        QG_HIP(hipGetLastError());
+        e = hipStreamSynchronize(s);   // the tables are host temporaries
+    } catch (...) {
+        dev_free(buf, bytes);
+        throw;
     }
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(rt.h_pinned, d_part + n_tiles_last, sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);   // group and term tables are host temporaries
-    dev_free(buf, gbytes + tbytes + pbytes);
+    dev_free(buf, bytes);
     QG_HIP(e);
     return rt.h_pinned[0];
 }

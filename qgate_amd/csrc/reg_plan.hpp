@@ -1,0 +1,391 @@
+// Planning of register-resident tile passes (reg_engine.hpp), on the host: how a gate list
+// becomes the ops, phases and passes that the kernels run. Shared by the single-circuit passes
+// (k_tile.hip) and the batched ones (k_batch.hip).
+#pragma once
+
+#include <algorithm>
+#include <cmath>
+#include <complex>
+#include <cstring>
+#include <vector>
+
+#include "gate_matrix.hpp"
+#include "qg_common.hpp"
+
+namespace qg {
+
+// ---- gates as the register passes apply them ----------------------------------------------
+//
+// Any 2x2 unitary is diag . RY . diag, and a diagonal factor is nearly free in a register pass
+// wherever its lane is no register bit (one factor per thread), so an uncontrolled general gate
+// becomes one real rotation, which takes a quarter of its multiplications.
+enum : int {
+    kGateDiag = 0,   // diag(m00, m11), controls allowed
+    kGateY = 1,      // [[c, -s], [s, c]], no controls
+    kGateX = 2,      // [[c, -i s], [-i s, c]], no controls
+    kGateSwap = 3,   // X, with or without controls
+    kGateAny = 4     // any other 2x2, controls allowed
+};
+
+struct RegGate {
+    int kind = kGateAny;
+    int target = 0;
+    int pauli = 0;      // gradient generator (1 X, 2 Y, 3 Z) of a sweep's rotation, 0: none
+    int source = 0;     // the gate of the caller's list that it came from
+    std::vector<int> ctrl;
+    GateMatrix m;
+};
+
+inline bool is_x(const GateMatrix &g) {
+    return g.m[0][0] == 0. && g.m[1][1] == 0. && g.m[0][1] == 1. && g.m[1][0] == 1.;
+}
+
+inline bool diag2(const GateMatrix &g) { return g.m[0][1] == 0. && g.m[1][0] == 0.; }
+
+// [[c, -s], [s, c]] with real entries, exactly
+inline bool is_y_rotation(const GateMatrix &g) {
+    for (int r = 0; r < 2; ++r)
+        for (int c = 0; c < 2; ++c)
+            if (g.m[r][c].imag() != 0.) return false;
+    return g.m[0][0] == g.m[1][1] && g.m[0][1] == -g.m[1][0] && (g.m[0][0] != 0. || g.m[0][1] != 0.);
+}
+
+// [[c, -i s], [-i s, c]], exactly
+inline bool is_x_rotation(const GateMatrix &g) {
+    return g.m[0][0].imag() == 0. && g.m[1][1].imag() == 0. && g.m[0][1].real() == 0. && g.m[1][0].real() == 0. &&
+           g.m[0][0] == g.m[1][1] && g.m[0][1] == g.m[1][0] && (g.m[0][0] != 0. || g.m[0][1] != 0.);
+}
+
+// U = diag(a0, a1) RY diag(1, b) for a unitary U (to FP64 rounding); false for any other. In
+// extended precision and rounded once, so that the factors' moduli are as close to 1 as those of
+// rounded sines and cosines.
+inline bool split_unitary(const GateMatrix &u, std::complex<double> &a0, std::complex<double> &a1,
+                          std::complex<double> &b, GateMatrix &ry) {
+    typedef std::complex<long double> cl;
+    const cl m00 = cl(u.m[0][0]), m01 = cl(u.m[0][1]), m10 = cl(u.m[1][0]), m11 = cl(u.m[1][1]);
+    const long double tol = 4e-15L;
+    if (!(std::abs(std::norm(m00) + std::norm(m01) - 1.L) < tol &&
+          std::abs(std::norm(m10) + std::norm(m11) - 1.L) < tol &&
+          std::abs(m00 * std::conj(m10) + m01 * std::conj(m11)) < tol))
+        return false;
+    const long double r0 = std::abs(m00), r1 = std::abs(m10), r = std::sqrt(r0 * r0 + r1 * r1);
+    auto phase = [](const cl &v) {
+        const long double n = std::abs(v);
+        return n > 0.L ? v / n : cl(1.L);
+    };
+    const cl p0 = phase(m00), p1 = phase(m10);
+    const cl pb = r0 >= r1 ? phase(m11) * std::conj(p1) : -phase(m01) * std::conj(p0);
+    auto rounded = [](const cl &v) { return std::complex<double>((double)v.real(), (double)v.imag()); };
+    a0 = rounded(p0);
+    a1 = rounded(p1);
+    b = rounded(pb);
+    const double c = (double)(r0 / r), s = (double)(r1 / r);
+    ry.m[0][0] = c;
+    ry.m[0][1] = -s;
+    ry.m[1][0] = s;
+    ry.m[1][1] = c;
+    return true;
+}
+
+inline RegGate diag_gate(std::complex<double> d0, std::complex<double> d1, int target, int source) {
+    RegGate g;
+    g.kind = kGateDiag;
+    g.target = target;
+    g.source = source;
+    g.m.m[0][0] = d0;
+    g.m.m[0][1] = g.m.m[1][0] = 0.;
+    g.m.m[1][1] = d1;
+    return g;
+}
+
+// A diagonal gate with m00 == 0 (or nearly) has no ratio m11 / m00 for the register passes.
+inline bool has_ratio(const GateMatrix &g) {
+    const double a = std::abs(g.m[0][0]);
+    return a > 1e-30 && a < 1e30;
+}
+
+inline bool trivial_diag(std::complex<double> d0, std::complex<double> d1) { return d0 == 1. && d1 == 1.; }
+
+// Appends the register gates of one fixed gate (no parameter), in the order they apply.
+inline void append_fixed(std::vector<RegGate> &out, const GateMatrix &m, const std::vector<int> &ctrl, int target,
+                         int source) {
+    RegGate g;
+    g.target = target;
+    g.source = source;
+    g.ctrl = ctrl;
+    g.m = m;
+    if (diag2(m) && has_ratio(m)) {
+        g.kind = kGateDiag;
+        if (!trivial_diag(m.m[0][0], m.m[1][1])) out.push_back(g);
+        return;
+    }
+    if (is_x(m)) {
+        g.kind = kGateSwap;
+        out.push_back(g);
+        return;
+    }
+    if (ctrl.empty()) {
+        if (is_y_rotation(m) || is_x_rotation(m)) {
+            g.kind = is_y_rotation(m) ? kGateY : kGateX;
+            out.push_back(g);
+            return;
+        }
+        std::complex<double> a0, a1, b;
+        GateMatrix ry;
+        if (split_unitary(m, a0, a1, b, ry)) {
+            if (!trivial_diag(1., b)) out.push_back(diag_gate(1., b, target, source));
+            g.kind = kGateY;
+            g.m = ry;
+            out.push_back(g);
+            if (!trivial_diag(a0, a1)) out.push_back(diag_gate(a0, a1, target, source));
+            return;
+        }
+    }
+    g.kind = kGateAny;
+    out.push_back(g);
+}
+
+// The register gates of a gate list whose matrices are all known. The uncontrolled gates of a lane
+// between controlled ones multiply into one (in FP64); of its split diag . RY . diag the last
+// diagonal waits for the lane's next gate where what comes between acts diagonally on the lane.
+// gate(i) has m, ctrl and target.
+template <class GateAt>
+std::vector<RegGate> merged_gates(int n_gates, int n_lanes, GateAt gate) {
+    std::vector<RegGate> out;
+    out.reserve((size_t)n_gates * 2);
+    std::vector<GateMatrix> run(n_lanes);
+    std::vector<int> last(n_lanes, -1);   // source of the lane's run, -1: none
+    auto emit = [&](int lane, bool keep_diagonal) {
+        if (last[lane] < 0) return;
+        GateMatrix &m = run[lane];
+        if (keep_diagonal && diag2(m)) return;
+        std::complex<double> a0, a1, b;
+        GateMatrix ry;
+        if (keep_diagonal && !is_x(m) && !is_y_rotation(m) && !is_x_rotation(m) && split_unitary(m, a0, a1, b, ry)) {
+            append_fixed(out, diag_gate(1., b, lane, last[lane]).m, {}, lane, last[lane]);
+            append_fixed(out, ry, {}, lane, last[lane]);
+            m = diag_gate(a0, a1, lane, last[lane]).m;
+            return;
+        }
+        append_fixed(out, m, {}, lane, last[lane]);
+        last[lane] = -1;
+    };
+    for (int i = 0; i < n_gates; ++i) {
+        const auto &g = gate(i);
+        if (g.ctrl.empty()) {
+            GateMatrix &m = run[g.target];
+            if (last[g.target] < 0) {
+                m = g.m;
+            } else {
+                GateMatrix p;
+                for (int r = 0; r < 2; ++r)
+                    for (int c = 0; c < 2; ++c) p.m[r][c] = g.m.m[r][0] * m.m[0][c] + g.m.m[r][1] * m.m[1][c];
+                m = p;
+            }
+            last[g.target] = i;
+            continue;
+        }
+        for (int c : g.ctrl) emit(c, true);
+        emit(g.target, diag2(g.m));
+        append_fixed(out, g.m, g.ctrl, g.target, i);
+    }
+    for (int l = 0; l < n_lanes; ++l) emit(l, false);
+    return out;
+}
+
+// ---- passes and phases ----------------------------------------------------------------------
+
+// Bit layout of one phase: local tile bits that are register, lane and wave bits.
+struct PhasePlan {
+    std::vector<int> regs, lanes, waves;
+    std::vector<int> order;    // gates, in the order they apply
+};
+
+struct PassBits {
+    std::vector<int> bits;     // state bits of the tile, ascending
+    int low = 0;               // bits[j] == j for j < low
+    std::vector<int> gates;    // gates, in an order they may apply in
+};
+
+// What the planner needs of a gate: its lanes, whether it acts diagonally on the target.
+struct PlanGate {
+    int target;
+    const std::vector<int> *ctrl;
+    bool diag;
+    int weight;    // ops it may take
+    int slots;     // gradient slots
+};
+
+// Lanes held by the gates left out of a scan: two gates commute when on every lane they share
+// both act diagonally there (a control, or the target of a diagonal gate).
+class HeldLanes {
+  public:
+    explicit HeldLanes(int n) : held_(n, 0) {}
+    bool conflicts(const PlanGate &g) const {
+        if (g.diag ? held_[g.target] == 2 : held_[g.target] != 0) return true;
+        for (int c : *g.ctrl)
+            if (held_[c] == 2) return true;
+        return false;
+    }
+    void hold(const PlanGate &g) {
+        put(g.target, g.diag ? 1 : 2);
+        for (int c : *g.ctrl) put(c, 1);
+    }
+    bool all() const { return full_ == (int)held_.size(); }
+
+  private:
+    void put(int lane, char v) {
+        if (held_[lane] < 2 && v == 2) ++full_;
+        held_[lane] = std::max(held_[lane], v);
+    }
+    std::vector<char> held_;
+    int full_ = 0;
+};
+
+constexpr int kLookahead = 256;   // gates a scan may leave out
+
+// The next pass over the gates not yet done: every gate that commutes with the ones left out
+// before it and whose target is a tile bit, can become one, or needs none (diagonal), up to
+// max_weight and max_slots. Marks them done. (A pass of consecutive gates only: a 2000-gate
+// random circuit on 30 qubits took 120 passes instead of 75.)
+inline PassBits next_pass(const std::vector<PlanGate> &g, std::vector<char> &done, int first, int n, int m, int low,
+                          int max_weight, int max_slots) {
+    PassBits p;
+    std::vector<char> in(n, 0);
+    int n_bits = 0, weight = 0, slots = 0, left = 0;
+    for (int b = 0; b < low; ++b) in[b] = 1, ++n_bits;
+    HeldLanes held(n);
+    for (int i = first; i < (int)g.size(); ++i) {
+        if (done[i]) continue;
+        const PlanGate &q = g[i];
+        const bool fits = q.diag || in[q.target] || n_bits < m;
+        if (fits && weight + q.weight <= max_weight && slots + q.slots <= max_slots && !held.conflicts(q)) {
+            if (!q.diag && !in[q.target]) in[q.target] = 1, ++n_bits;
+            weight += q.weight;
+            slots += q.slots;
+            done[i] = 1;
+            p.gates.push_back(i);
+            continue;
+        }
+        held.hold(q);
+        if (++left >= kLookahead || held.all()) break;
+    }
+    for (int b = 0; b < n && n_bits < m; ++b)   // a full tile: the lowest free bits
+        if (!in[b]) in[b] = 1, ++n_bits;
+    for (int b = 0; b < n; ++b)
+        if (in[b]) p.bits.push_back(b);
+    while (p.low < (int)p.bits.size() && p.bits[p.low] == p.low) ++p.low;
+    return p;
+}
+
+// Rotations are applied up to a factor of at most sqrt(2), collected per phase; a phase takes
+// at most this many of them (2^8 in the amplitudes, 2^16 in a gradient term).
+constexpr int kMaxScaled = 16;
+
+// The phases of a pass: each takes every gate that commutes with the ones it leaves out and
+// whose non-diagonal target is one of its rb register bits or can become one; then each diagonal
+// gate moves, between the pair gates on its lanes before and after it, to a phase where none of
+// its lanes is a register bit (there it is one factor per thread instead of an update of the
+// registers), if possible one that already has such factors.
+inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const std::vector<int> &gates,
+                                          const int *local, int n, int m, int rb, int wb) {
+    std::vector<PhasePlan> out;
+    std::vector<char> done(gates.size(), 0);
+    size_t first = 0;
+    while (first < gates.size()) {
+        PhasePlan P;
+        HeldLanes held(n);
+        int pairs = 0;
+        for (size_t k = first; k < gates.size(); ++k) {
+            if (done[k]) continue;
+            const PlanGate &q = g[gates[k]];
+            const int lt = local[q.target];
+            const bool known = !q.diag && std::find(P.regs.begin(), P.regs.end(), lt) != P.regs.end();
+            const bool fits = q.diag || (pairs < kMaxScaled && (known || (int)P.regs.size() < rb));
+            if (fits && !held.conflicts(q)) {
+                if (!q.diag) {
+                    if (!known) P.regs.push_back(lt);
+                    ++pairs;
+                }
+                P.order.push_back(gates[k]);
+                done[k] = 1;
+                continue;
+            }
+            held.hold(q);
+            if (held.all()) break;
+        }
+        while (first < gates.size() && done[first]) ++first;
+        // pad with the highest free bits, so that the lane bits are the lowest ones
+        for (int b = m - 1; (int)P.regs.size() < rb && b >= 0; --b)
+            if (std::find(P.regs.begin(), P.regs.end(), b) == P.regs.end()) P.regs.push_back(b);
+        std::sort(P.regs.begin(), P.regs.end());
+        for (int b = 0; b < m; ++b)
+            if (std::find(P.regs.begin(), P.regs.end(), b) == P.regs.end())
+                ((int)P.lanes.size() < 6 ? P.lanes : P.waves).push_back(b);
+        if ((int)P.waves.size() != wb) raise_error("tile layout does not match the workgroup");
+        out.push_back(P);
+    }
+    // diagonal gates: position gp is before pair gate gp (np: after the last)
+    std::vector<int> pairs, phase_of, diags, seen_at;
+    for (size_t ph = 0; ph < out.size(); ++ph)
+        for (int gi : out[ph].order) {
+            if (g[gi].diag) {
+                diags.push_back(gi);
+                seen_at.push_back((int)pairs.size());
+            } else {
+                pairs.push_back(gi);
+                phase_of.push_back((int)ph);
+            }
+        }
+    const int np = (int)pairs.size();
+    if (np == 0 || diags.empty()) return out;
+    const int n_ph = (int)out.size();
+    std::vector<char> has_factor(n_ph, 0);
+    std::vector<std::vector<int>> at(np + 1);   // diagonal gates right before pair gate gp
+    std::vector<std::vector<int>> where(np + 1);   // and the phase each of them runs in
+    for (size_t d = 0; d < diags.size(); ++d) {
+        const PlanGate &q = g[diags[d]];
+        std::vector<int> lanes(*q.ctrl);
+        lanes.push_back(q.target);
+        auto hits = [&](int k) { return std::find(lanes.begin(), lanes.end(), g[pairs[k]].target) != lanes.end(); };
+        int lo = 0, hi = np;
+        for (int k = seen_at[d] - 1; k >= 0; --k)
+            if (hits(k)) {
+                lo = k + 1;
+                break;
+            }
+        for (int k = seen_at[d]; k < np; ++k)
+            if (hits(k)) {
+                hi = k;
+                break;
+            }
+        // phases it may run in: any from that of the pair gate before position lo to that of the
+        // one after position hi
+        const int ph_lo = lo == 0 ? 0 : phase_of[lo - 1], ph_hi = hi == np ? n_ph - 1 : phase_of[hi];
+        auto cost = [&](int ph) {
+            int regs = 0;
+            for (int l : lanes)
+                if (local[l] >= 0 &&
+                    std::find(out[ph].regs.begin(), out[ph].regs.end(), local[l]) != out[ph].regs.end())
+                    ++regs;
+            return regs > 0 ? 4 - (regs > 1) : has_factor[ph] ? 0 : 1;
+        };
+        int best = -1;
+        for (int ph = ph_lo; ph <= ph_hi; ++ph)
+            if (best < 0 || cost(ph) < cost(best)) best = ph;
+        if (cost(best) <= 1) has_factor[best] = 1;
+        // the last position within [lo, hi] that still belongs to that phase
+        int gp = lo;
+        while (gp < hi && phase_of[gp] <= best) ++gp;
+        at[gp].push_back(diags[d]);
+        where[gp].push_back(best);
+    }
+    for (PhasePlan &P : out) P.order.clear();
+    for (int gp = 0; gp <= np; ++gp) {
+        for (size_t k = 0; k < at[gp].size(); ++k) out[where[gp][k]].order.push_back(at[gp][k]);
+        if (gp < np) out[phase_of[gp]].order.push_back(pairs[gp]);
+    }
+    return out;
+}
+
+}  // namespace qg

@@ -1,5 +1,32 @@
-// Register-resident tile passes and their planning, shared by the single-circuit passes
-// (k_tile.hip) and the batched passes (k_batch.hip).
+// Register-resident tile passes: device code shared by the single-circuit passes (k_tile.hip)
+// and the batched ones (k_batch.hip). Their planning is in reg_plan.hpp.
+//
+// A pass keeps its tile in registers: each of the T threads holds A = 2^M / T amplitudes of
+// each state (one state going forward, phi and lambda in the adjoint sweep). It is split into
+// phases; in each phase log2(A) tile bits are register bits (the targets of the phase's
+// non-diagonal gates), 6 are lane bits and the rest wave bits, so the phase's pair updates are
+// register to register, with no LDS traffic and no barrier. Between phases the tile goes
+// through LDS once.
+//
+// What bounds a pass is instruction issue, so the ops are built to be few and short:
+//   * Rotations are applied without their common factor: [[c, -s], [s, c]] is
+//     c [[1, -t], [t, 1]] with t = s / c, or s [[k, -1], [1, k]] with k = c / s where that is
+//     smaller, one FMA a component instead of a multiply and an FMA. The factors of a phase
+//     multiply into one number that is applied at the end of the phase. Uncontrolled general
+//     gates arrive split into diagonals and such a rotation (reg_plan.hpp).
+//   * Register updates are in-place asm statements with tied operands. Written as expressions,
+//     every dispatch arm produced new values and the compiler moved the whole register array at
+//     the joins (32 to 64 moves a gate in the sweep, whose rotations take 48).
+//   * Diagonal gates on no register bit multiply into one factor per thread, applied at the end
+//     of the phase; signs (CZ, Z) into one sign.
+//   * Gradient terms are summed over the wavefront by FP64 matrix-core steps, sixteen slots to
+//     an accumulator tile: a conversion, two moves and one matrix instruction a term, where a
+//     DPP tree took about 20 vector instructions.
+// Together the 24-qubit ansatz's sweep issues 3109 vector instructions per wave and pass, against
+// 5834 before, and its passes take 243 us instead of 353; a forward pass over 30 qubits in
+// complex64 carries 29 gates in 5.36 ms, against 22 in 5.80 ms. Vector and scalar issue still
+// bound both (78% and 54% of the cycles of a sweep pass): a gate costs about 45 scalar
+// instructions to decode and dispatch beside its arithmetic.
 #pragma once
 
 #include <algorithm>
@@ -10,6 +37,7 @@
 
 #include "gate_matrix.hpp"
 #include "qg_runtime.hpp"
+#include "reg_plan.hpp"
 #include "tile_common.hpp"
 
 namespace qg {
@@ -21,26 +49,19 @@ struct TileCfg;
 template <>
 struct TileCfg<float> {
     static constexpr int MaxBits = 12;   // 2^12 x 8 B = 32 KiB of LDS
-    static constexpr int MaxOps = 40;
+    static constexpr int MaxOps = 40;    // LDS passes
+    static constexpr int MaxRegOps = 72; // register passes: 40 B each in the kernel arguments
     static constexpr int Low = 5;        // 32 contiguous amplitudes = 256 B per row
 };
 template <>
 struct TileCfg<double> {
     static constexpr int MaxBits = 11;   // 2^11 x 16 B = 32 KiB
     static constexpr int MaxOps = 24;
+    static constexpr int MaxRegOps = 52; // 56 B each
     static constexpr int Low = 4;        // 16 x 16 B = 256 B per row
 };
 
-// ---- register-resident tile passes ------------------------------------------------------
-//
-// The full-size pass (m == MaxBits) keeps the tile in registers: each of the T threads holds
-// A = 2^m / T amplitudes. A pass is split into phases; in each phase RB = log2(A) tile bits
-// are register bits (the targets of the phase's non-diagonal gates), 6 are lane bits and the
-// rest wave bits, so the phase's pair updates are register-to-register with no LDS traffic
-// or barriers. Between phases the tile goes through LDS once (write, barrier, read in the
-// next phase's layout). A pass of g gates costs about g / RB LDS round trips instead of g.
-
-constexpr int kMaxPhases = 40;
+constexpr int kMaxPhases = 24;
 
 // Bit layout of one register phase, packed in dwords so that a phase read at a runtime
 // index takes scalar loads (a byte array read at a runtime index would be a vector load,
@@ -48,7 +69,7 @@ constexpr int kMaxPhases = 40;
 // register bit k (k < 5), of lane bit k - 5 (5 <= k < 11) or of wave bit k - 11 (k < 14).
 struct PhaseBits {
     unsigned bits[4];
-    int op_begin, n_ops;
+    int op_begin, n_ops;   // ops of the pass
     __host__ __device__ int byte(int k) const { return (int)((bits[k >> 2] >> ((k & 3) * 8)) & 0xffu); }
     __host__ __device__ int rb(int k) const { return byte(k); }
     __host__ __device__ int lb(int k) const { return byte(5 + k); }
@@ -58,46 +79,136 @@ struct PhaseBits {
         bits[k >> 2] = (bits[k >> 2] & ~(0xffu << sh)) | ((unsigned)v << sh);
     }
 };
-typedef PhaseBits RegPhase;
 
-// Local-index bits of register index j in phase P (uniform: a scalar value).
-template <int RB>
-__device__ __forceinline__ unsigned reg_bits(const PhaseBits &P, int j) {
-    unsigned l = 0;
-#pragma unroll
-    for (int k = 0; k < RB; ++k) l |= (((unsigned)j >> k) & 1u) << P.rb(k);
-    return l;
+// Arms of an op. Families of updates on a register position P take codes 4 F + P: rotations
+// about Y and X in their two forms (t, k), controlled swaps, general 2x2, a factor or a sign on
+// the register indices with bit P set, and the gradient term of a Z generator on bit P.
+// kArmPair2 + i: a factor on the register indices with both bits of the i-th pair set
+// (01, 02, 12, 03, 13, 23), kArmSign2 + i a sign; kArmFactorAny: on those with every bit of creg
+// set; kArmZAny: the Z term with controls on register bits. The rest leave the registers alone.
+enum : int {
+    kFamY = 0, kFamYk = 1, kFamX = 2, kFamXk = 3, kFamSwap = 4, kFamAny = 5, kFamFactor = 6, kFamSign = 7, kFamZ = 8,
+    kArmPair2 = 36, kArmSign2 = 42, kArmFactorAny = 48, kArmZAny = 49,
+    kArmThread = 50,       // diag(m00, m11) by a lane or wave bit
+    kArmThreadCtrl = 51,   // the same with controls on lane and wave bits
+    kArmOuter = 52,        // diag(m00, m11) by a bit outside the tile, controls allowed
+    kArmPhase = 53,        // a factor where every control on lane and wave bits is set
+    kArmSign = 54,         // a sign where they are
+    kArmU = 55,            // the thread's sum that the Z terms on bits that are no register bits share
+    kArmFlush = 56,        // 16 gradient slots are complete
+    kArmNone = 57          // the second half of a general 2x2
+};
+
+// One op of a register pass. code: arm | target << 8 | creg << 16 | generator << 24 | first
+// coefficient << 28. Controls are split by where their bits live: outside the tile (gctrl, one
+// test per tile), on lane and wave bits (cthr, one test per thread), on register bits (creg).
+template <class R>
+struct alignas(8) RegOp {
+    unsigned code, cthr;
+    u64 gctrl;
+    int slot;          // gradient slot, -1: none
+    int row;           // batched passes: row of the coefficient table
+    R c[4];            // else the coefficients (a general 2x2 takes the next op's as well)
+};
+
+// An op read whole, as two or three scalar loads: field by field it took five, each with its own
+// address.
+template <class R>
+struct OpWords {
+    typedef unsigned u32x8 __attribute__((ext_vector_type(8), aligned(8)));
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2), aligned(8)));
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4), aligned(8)));
+    u32x8 a;
+    u32x4 b;
+    u32x2 c;
+    __device__ __forceinline__ void load(const RegOp<R> *p) {
+        const unsigned *w = reinterpret_cast<const unsigned *>(p);
+        a = *reinterpret_cast<const u32x8 *>(w);
+        if constexpr (sizeof(R) == 8) {
+            b = *reinterpret_cast<const u32x4 *>(w + 8);
+            c = *reinterpret_cast<const u32x2 *>(w + 12);
+        } else {
+            c = *reinterpret_cast<const u32x2 *>(w + 8);
+        }
+    }
+    // waits for the words: scalar loads return out of order, so a wait for these after the next
+    // op's have been issued would wait for both
+    __device__ __forceinline__ void arrive() {
+        if constexpr (sizeof(R) == 8)
+            asm volatile("; op" : "+s"(a), "+s"(b), "+s"(c));
+        else
+            asm volatile("; op" : "+s"(a), "+s"(c));
+    }
+    __device__ __forceinline__ unsigned code() const { return a[0]; }
+    __device__ __forceinline__ unsigned cthr() const { return a[1]; }
+    __device__ __forceinline__ u64 gctrl() const { return (u64)a[3] << 32 | a[2]; }
+    __device__ __forceinline__ int slot() const { return (int)a[4]; }
+    __device__ __forceinline__ int row() const { return (int)a[5]; }
+    __device__ __forceinline__ R coef(int i) const {
+        if constexpr (sizeof(R) == 8) {
+            const unsigned lo = i == 0 ? a[6] : i == 1 ? b[0] : i == 2 ? b[2] : c[0];
+            const unsigned hi = i == 0 ? a[7] : i == 1 ? b[1] : i == 2 ? b[3] : c[1];
+            return __longlong_as_double((long long)((u64)hi << 32 | lo));
+        } else {
+            return __uint_as_float(i == 0 ? a[6] : i == 1 ? a[7] : i == 2 ? c[0] : c[1]);
+        }
+    }
+};
+static_assert(sizeof(RegOp<float>) == 40 && sizeof(RegOp<double>) == 56, "op words");
+
+// Coefficients of a gate, by kind (a row of a batched pass's table):
+//   rotation   t or k, 1 if it is k, and the factor left out, in FP64 for complex64 (two
+//              entries), as an unevaluated sum of two numbers for complex128
+//   diagonal   m00, m11, m11 / m00 (complex)
+//   general    m00, m01, m10, m11 (complex)
+// The factor is that of the rounded t (or k), which makes good what rounding t does to the norm
+// of the state, and the factors of a phase are multiplied in twice the precision of the state
+// and rounded once. The rounded matrices of the two-multiply form each shift the norm of the
+// whole state; after 530 gates on 30 qubits in complex64 a joint distribution was off by 2.1e-6
+// (2-norm), now 0.57e-6.
+constexpr int kCoefs = 8;
+
+template <class R>
+__host__ __device__ inline void rotation_coefs(R *c, double co, double si) {
+    const bool k = (si < 0. ? -si : si) > (co < 0. ? -co : co);
+    c[0] = (R)(k ? co / si : si / co);
+    c[1] = k ? R(1) : R(0);
+    // f (1 + r / 2) = 1 / sqrt(1 + t^2), r the rest of one Newton step in FMAs
+    const double t = (double)c[0], t2 = t * t, q = 1. + t2, qe = ((1. - q) + t2) + __builtin_fma(t, t, -t2);
+    double f = 1. / sqrt(q);
+    const double f2 = f * f, p = f2 * q;
+    const double r = ((1. - p) - __builtin_fma(f2, q, -p)) - __builtin_fma(__builtin_fma(f, f, -f2), q, f2 * qe);
+    // a matrix that is no rotation but a multiple of one
+    const double mag2 = co * co + si * si;
+    if (mag2 < 1. - 1e-13 || mag2 > 1. + 1e-13) f *= sqrt(mag2);
+    if ((k ? si : co) < 0.) f = -f;
+    if constexpr (sizeof(R) == 8) {
+        c[2] = f;
+        c[3] = 0.5 * f * r;
+    } else {
+        __builtin_memcpy(c + 2, &f, sizeof(double));
+    }
 }
 
-// Register-pass op kinds. Pair updates on a register position (general, swap, real); a
-// diagonal whose target is a register position (every amplitude, or only the |1> half when
-// m00 == 1); a diagonal whose target is a lane/wave bit or a bit outside the tile, which is
-// one factor per thread.
-enum : int {
-    kRegPair = 0, kRegPairSwap = 1, kRegPairReal = 2,
-    kRegDiag = 3, kRegDiagPhase = 4, kRegDiagThread = 5, kRegDiagOuter = 6
-};
-
-// A gate in a register phase. Its controls are split by where their bits live: outside the
-// tile (one test per tile), on lane/wave bits (one test per thread) and on register bits
-// (register positions: tests on the compile-time register indices, made by the scalar unit).
+// The factors of a phase's rotations (uniform): hi + lo for complex128, hi for complex64.
 template <class R>
-struct RegOp {
-    Mat2<R> m;
-    u64 gctrl;         // controls outside the tile (state bits)
-    unsigned cthr;     // controls on lane/wave bits (local bits)
-    int creg;          // controls on register bits (mask of register positions)
-    int target;        // register position (pairs, kRegDiag*), local bit (kRegDiagThread), state bit (kRegDiagOuter)
-    int kind;
-    int gate;          // batched passes: index of the gate in its circuit (m unused)
-};
-
-template <class R>
-struct RegProgram {
-    int n_ops, n_phases, low;
-    alignas(4) signed char pos[kTilePosMax];
-    RegPhase phases[kMaxPhases];
-    RegOp<R> ops[TileCfg<R>::MaxOps];
+struct Scale {
+    double hi, lo;
+    // 1 + carry: what the rounding of the last phase's factor left out
+    __device__ __forceinline__ void init(double carry) {
+        hi = sizeof(R) == 8 ? 1. : 1. + carry;
+        lo = sizeof(R) == 8 ? carry : 0.;
+    }
+    __device__ __forceinline__ void times(R c2, R c3) {
+        if constexpr (sizeof(R) == 8) {
+            const double p = hi * c2;
+            lo = __builtin_fma(lo, c2, __builtin_fma(hi, c3, __builtin_fma(hi, c2, -p)));
+            hi = p;
+        } else {
+            hi *= __longlong_as_double((long long)(((u64)__float_as_uint(c3) << 32) | __float_as_uint(c2)));
+        }
+    }
+    __device__ __forceinline__ double value() const { return sizeof(R) == 8 ? hi + lo : hi; }
 };
 
 template <int A>
@@ -119,21 +230,6 @@ __device__ __forceinline__ void static_for(F &&f) {
     }
 }
 
-// Ends a register-pair update on register bit P. The markers differ per P, so the optimiser
-// cannot merge the updates of different bits (dispatched on a runtime bit) into one block
-// that picks the register elements through pointers, which would move those elements to
-// private (scratch) memory.
-template <int P>
-__device__ __forceinline__ void pair_marker() {
-    asm volatile("; register pair %0" ::"n"(P));
-}
-
-// Im(conj(a) b)
-template <class R>
-__device__ __forceinline__ R im_conj_mul(const Cx<R> &a, const Cx<R> &b) {
-    return a.re * b.im - a.im * b.re;
-}
-
 template <class R>
 __device__ __forceinline__ R fma_r(R a, R b, R c) {
     if constexpr (sizeof(R) == 4)
@@ -148,20 +244,16 @@ __device__ __forceinline__ R add_im_conj_mul(R acc, const Cx<R> &a, const Cx<R> 
     return fma_r(-a.im, b.re, fma_r(a.re, b.im, acc));
 }
 
-// acc + the gradient term of a pair (p0, p1) / (l0, l1) for generator G (1 X, 2 Y, 3 Z):
+// acc + the gradient term of a pair (p0, p1) / (l0, l1) for generator G (1 X, 2 Y):
 // Im<l|G|p> over the pair, four FMAs into the accumulator
 template <class R, int G>
 __device__ __forceinline__ R add_pair_term(R acc, const Cx<R> &p0, const Cx<R> &p1, const Cx<R> &l0,
                                            const Cx<R> &l1) {
     if constexpr (G == 1) return add_im_conj_mul(add_im_conj_mul(acc, l0, p1), l1, p0);
-    if constexpr (G == 2) {
-        acc = fma_r(l1.re, p0.re, acc);
-        acc = fma_r(l1.im, p0.im, acc);
-        acc = fma_r(-l0.re, p1.re, acc);
-        return fma_r(-l0.im, p1.im, acc);
-    }
-    if constexpr (G == 3) return add_im_conj_mul(add_im_conj_mul(acc, l0, p0), p1, l1);
-    return acc;
+    acc = fma_r(l1.re, p0.re, acc);
+    acc = fma_r(l1.im, p0.im, acc);
+    acc = fma_r(-l0.re, p1.re, acc);
+    return fma_r(-l0.im, p1.im, acc);
 }
 
 // c ? a : b, component by component: a select of whole structs can be lowered to a select
@@ -171,700 +263,541 @@ __device__ __forceinline__ Cx<R> csel(bool c, const Cx<R> &a, const Cx<R> &b) {
     return cx<R>(c ? a.re : b.re, c ? a.im : b.im);
 }
 
-// (y0, y1) = M (x0, x1) for a matrix of form F: 0 general, 1 swap, 2 real, 3 real diagonal
-// and imaginary off-diagonal (RX-like: m00, m11 real; m01, m10 imaginary).
-template <class R, int F>
-__device__ __forceinline__ void apply_form(const Mat2<R> &mm, const Cx<R> &x0, const Cx<R> &x1, Cx<R> &y0, Cx<R> &y1) {
-    if constexpr (F == 1) {
-        y0 = x1;
-        y1 = x0;
-    } else if constexpr (F == 2) {
-        const R a = mm.m00.re, b = mm.m01.re, c = mm.m10.re, d = mm.m11.re;
-        y0 = cx<R>(a * x0.re + b * x1.re, a * x0.im + b * x1.im);
-        y1 = cx<R>(c * x0.re + d * x1.re, c * x0.im + d * x1.im);
-    } else if constexpr (F == 3) {
-        const R a = mm.m00.re, b = mm.m01.im, c = mm.m10.im, d = mm.m11.re;
-        y0 = cx<R>(a * x0.re - b * x1.im, a * x0.im + b * x1.re);
-        y1 = cx<R>(d * x1.re - c * x0.im, d * x1.im + c * x0.re);
-    } else {
-        // one multiply and three FMAs per component (a sum of two complex products written
-        // as such takes two multiplies, two FMAs and an add)
-        y0 = cx<R>(fma_r(mm.m00.re, x0.re, fma_r(-mm.m00.im, x0.im, fma_r(mm.m01.re, x1.re, -mm.m01.im * x1.im))),
-                   fma_r(mm.m00.re, x0.im, fma_r(mm.m00.im, x0.re, fma_r(mm.m01.re, x1.im, mm.m01.im * x1.re))));
-        y1 = cx<R>(fma_r(mm.m10.re, x0.re, fma_r(-mm.m10.im, x0.im, fma_r(mm.m11.re, x1.re, -mm.m11.im * x1.im))),
-                   fma_r(mm.m10.re, x0.im, fma_r(mm.m10.im, x0.re, fma_r(mm.m11.re, x1.im, mm.m11.im * x1.re))));
-    }
-}
-
-// ---- register ops between two register arrays ----------------------------------------------
+// ---- in-place register updates ---------------------------------------------------------------
 //
-// The ops of a phase read one register array and write the other, which the next op reads;
-// a uniform flag says which array holds the amplitudes. Every output of an op is a new
-// value, so all dispatch arms of an op leave their results in the same registers and no join
-// needs copies. (An in-place update of one loop-carried array made the compiler keep two
-// copies of it anyway and move the whole array between them on most paths: 36 to 130 moves
-// a gate, against 128 FMAs for a general 2x2.) Ops that change no amplitude (skipped for
-// controls outside the tile, per-thread factors) leave the flag as it is and move nothing.
+// C is a code of its own per dispatch arm, in the statement as a comment, so that the optimiser
+// merges no two arms into one block that would pick register elements through pointers. The
+// statements hold vector instructions only, read and write no memory, and leave every output
+// written; the matrix-core and cross-lane instructions around them, whose operands need wait
+// states after a vector write, take compiler-made values.
 
-// Arm codes of an op: pairs on register bit P of form F (0 general, 1 swap, 2 real) at
-// 4 F + P, with controls on lane, wave or register bits at 12 + 4 F + P; diagonals on
-// register bit P at 24 + P, with m00 == 1 at 28 + P; a diagonal on a register bit with
-// controls 32; a per-thread factor on the register indices with controls creg 33.
-enum : int { kArmPairSel = 12, kArmDiag = 24, kArmDiagPhase = 28, kArmDiagCtrl = 32, kArmFactorReg = 33 };
+// Rotations: (x, y) <- (x + t y, y - t x) for form t, (y + k x, k y - x) for form k. One statement
+// takes both components of a register pair, of every state: the compiler puts an idle
+// instruction between statements that write vector registers.
 
-// Ends an arm. The markers differ per arm and per array, so the optimiser merges no two arms
-// into one block that picks register elements through pointers (which would move them to
-// scratch memory) or through selects.
-template <int H, int C>
-__device__ __forceinline__ void arm_marker() {
-    asm volatile("; register op %0" ::"n"(H * 64 + C));
+template <int C>
+__device__ __forceinline__ void rot_t(float &x0, float &y0, float &x1, float &y1, float c) {
+    float w, z;
+    asm(
+        "v_fma_f32 %4, %6, %1, %0\n\t"
+        "v_fma_f32 %5, %6, %3, %2\n\t"
+        "v_fma_f32 %1, -%6, %0, %1\n\t"
+        "v_fma_f32 %3, -%6, %2, %3\n\t"
+        "v_mov_b32 %0, %4\n\t"
+        "v_mov_b32 %2, %5\n\t"
+        "; arm %7"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
 }
 
-// y = x with the pair update of form F on register bit P applied to every pair (plain), or
-// to the register indices j with (j & creg) == creg in threads with ok set (SEL: selects).
-template <class R, int A, int P, int F, bool SEL>
-__device__ __forceinline__ void op_pair(const Cx<R> (&x)[A], Cx<R> (&y)[A], const Mat2<R> &mm, int creg, bool ok) {
+template <int C>
+__device__ __forceinline__ void rot_t(float &x0, float &y0, float &x1, float &y1, float &x2, float &y2, float &x3, float &y3, float c) {
+    float w, z;
+    asm(
+        "v_fma_f32 %8, %10, %1, %0\n\t"
+        "v_fma_f32 %9, %10, %3, %2\n\t"
+        "v_fma_f32 %1, -%10, %0, %1\n\t"
+        "v_fma_f32 %3, -%10, %2, %3\n\t"
+        "v_mov_b32 %0, %8\n\t"
+        "v_mov_b32 %2, %9\n\t"
+        "v_fma_f32 %8, %10, %5, %4\n\t"
+        "v_fma_f32 %9, %10, %7, %6\n\t"
+        "v_fma_f32 %5, -%10, %4, %5\n\t"
+        "v_fma_f32 %7, -%10, %6, %7\n\t"
+        "v_mov_b32 %4, %8\n\t"
+        "v_mov_b32 %6, %9\n\t"
+        "; arm %11"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "+v"(x2), "+v"(y2), "+v"(x3), "+v"(y3), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
+}
+
+template <int C>
+__device__ __forceinline__ void rot_k(float &x0, float &y0, float &x1, float &y1, float c) {
+    float w, z;
+    asm(
+        "v_fma_f32 %4, %6, %0, %1\n\t"
+        "v_fma_f32 %5, %6, %2, %3\n\t"
+        "v_fma_f32 %1, %6, %1, -%0\n\t"
+        "v_fma_f32 %3, %6, %3, -%2\n\t"
+        "v_mov_b32 %0, %4\n\t"
+        "v_mov_b32 %2, %5\n\t"
+        "; arm %7"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
+}
+
+template <int C>
+__device__ __forceinline__ void rot_k(float &x0, float &y0, float &x1, float &y1, float &x2, float &y2, float &x3, float &y3, float c) {
+    float w, z;
+    asm(
+        "v_fma_f32 %8, %10, %0, %1\n\t"
+        "v_fma_f32 %9, %10, %2, %3\n\t"
+        "v_fma_f32 %1, %10, %1, -%0\n\t"
+        "v_fma_f32 %3, %10, %3, -%2\n\t"
+        "v_mov_b32 %0, %8\n\t"
+        "v_mov_b32 %2, %9\n\t"
+        "v_fma_f32 %8, %10, %4, %5\n\t"
+        "v_fma_f32 %9, %10, %6, %7\n\t"
+        "v_fma_f32 %5, %10, %5, -%4\n\t"
+        "v_fma_f32 %7, %10, %7, -%6\n\t"
+        "v_mov_b32 %4, %8\n\t"
+        "v_mov_b32 %6, %9\n\t"
+        "; arm %11"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "+v"(x2), "+v"(y2), "+v"(x3), "+v"(y3), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
+}
+
+template <int C>
+__device__ __forceinline__ void rot_t(double &x0, double &y0, double &x1, double &y1, double c) {
+    double w, z;
+    asm(
+        "v_fma_f64 %4, %6, %1, %0\n\t"
+        "v_fma_f64 %5, %6, %3, %2\n\t"
+        "v_fma_f64 %1, -%6, %0, %1\n\t"
+        "v_fma_f64 %3, -%6, %2, %3\n\t"
+        "v_mov_b64 %0, %4\n\t"
+        "v_mov_b64 %2, %5\n\t"
+        "; arm %7"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
+}
+
+template <int C>
+__device__ __forceinline__ void rot_t(double &x0, double &y0, double &x1, double &y1, double &x2, double &y2, double &x3, double &y3, double c) {
+    double w, z;
+    asm(
+        "v_fma_f64 %8, %10, %1, %0\n\t"
+        "v_fma_f64 %9, %10, %3, %2\n\t"
+        "v_fma_f64 %1, -%10, %0, %1\n\t"
+        "v_fma_f64 %3, -%10, %2, %3\n\t"
+        "v_mov_b64 %0, %8\n\t"
+        "v_mov_b64 %2, %9\n\t"
+        "v_fma_f64 %8, %10, %5, %4\n\t"
+        "v_fma_f64 %9, %10, %7, %6\n\t"
+        "v_fma_f64 %5, -%10, %4, %5\n\t"
+        "v_fma_f64 %7, -%10, %6, %7\n\t"
+        "v_mov_b64 %4, %8\n\t"
+        "v_mov_b64 %6, %9\n\t"
+        "; arm %11"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "+v"(x2), "+v"(y2), "+v"(x3), "+v"(y3), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
+}
+
+template <int C>
+__device__ __forceinline__ void rot_k(double &x0, double &y0, double &x1, double &y1, double c) {
+    double w, z;
+    asm(
+        "v_fma_f64 %4, %6, %0, %1\n\t"
+        "v_fma_f64 %5, %6, %2, %3\n\t"
+        "v_fma_f64 %1, %6, %1, -%0\n\t"
+        "v_fma_f64 %3, %6, %3, -%2\n\t"
+        "v_mov_b64 %0, %4\n\t"
+        "v_mov_b64 %2, %5\n\t"
+        "; arm %7"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
+}
+
+template <int C>
+__device__ __forceinline__ void rot_k(double &x0, double &y0, double &x1, double &y1, double &x2, double &y2, double &x3, double &y3, double c) {
+    double w, z;
+    asm(
+        "v_fma_f64 %8, %10, %0, %1\n\t"
+        "v_fma_f64 %9, %10, %2, %3\n\t"
+        "v_fma_f64 %1, %10, %1, -%0\n\t"
+        "v_fma_f64 %3, %10, %3, -%2\n\t"
+        "v_mov_b64 %0, %8\n\t"
+        "v_mov_b64 %2, %9\n\t"
+        "v_fma_f64 %8, %10, %4, %5\n\t"
+        "v_fma_f64 %9, %10, %6, %7\n\t"
+        "v_fma_f64 %5, %10, %5, -%4\n\t"
+        "v_fma_f64 %7, %10, %7, -%6\n\t"
+        "v_mov_b64 %4, %8\n\t"
+        "v_mov_b64 %6, %9\n\t"
+        "; arm %11"
+        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "+v"(x2), "+v"(y2), "+v"(x3), "+v"(y3), "=&v"(w), "=&v"(z)
+        : "s"(c), "n"(C));
+}
+
+// x, y <- m ? y, x : x, y (m: lane mask)
+template <int C>
+__device__ __forceinline__ void swap_if(Cx<float> &x, Cx<float> &y, u64 m) {
+    float w, z;
+    asm("v_cndmask_b32 %4, %0, %1, %6\n\tv_cndmask_b32 %5, %2, %3, %6\n\tv_cndmask_b32 %1, %1, %0, %6\n\t"
+        "v_cndmask_b32 %3, %3, %2, %6\n\tv_mov_b32 %0, %4\n\tv_mov_b32 %2, %5 ; arm %7"
+        : "+v"(x.re), "+v"(y.re), "+v"(x.im), "+v"(y.im), "=&v"(w), "=&v"(z) : "s"(m), "n"(C));
+}
+template <int C>
+__device__ __forceinline__ void swap_if(Cx<double> &x, Cx<double> &y, u64 m) {
+    // under a lane mask: a 64-bit value has no select of its own
+    double w, z;
+    u64 saved;
+    asm("s_mov_b64 %6, exec\n\ts_and_b64 exec, exec, %7\n\tv_mov_b64 %4, %0\n\tv_mov_b64 %5, %2\n\t"
+        "v_mov_b64 %0, %1\n\tv_mov_b64 %2, %3\n\tv_mov_b64 %1, %4\n\tv_mov_b64 %3, %5\n\ts_mov_b64 exec, %6 ; arm %8"
+        : "+v"(x.re), "+v"(y.re), "+v"(x.im), "+v"(y.im), "=&v"(w), "=&v"(z), "=&s"(saved)
+        : "s"(m), "n"(C)
+        : "scc");
+}
+
+// (re, im) <- (re, im) (fr, fi)
+template <int C>
+__device__ __forceinline__ void mul_by(Cx<float> &v, const Cx<float> &f) {
+    float w;
+    asm("v_mul_f32 %2, %0, %3\n\tv_fma_f32 %2, -%1, %4, %2\n\tv_mul_f32 %1, %1, %3\n\tv_fma_f32 %1, %0, %4, %1\n\t"
+        "v_mov_b32 %0, %2 ; arm %5"
+        : "+v"(v.re), "+v"(v.im), "=&v"(w) : "v"(f.re), "v"(f.im), "n"(C));
+}
+template <int C>
+__device__ __forceinline__ void mul_by(Cx<double> &v, const Cx<double> &f) {
+    double w;
+    asm("v_mul_f64 %2, %0, %3\n\tv_fma_f64 %2, -%1, %4, %2\n\tv_mul_f64 %1, %1, %3\n\tv_fma_f64 %1, %0, %4, %1\n\t"
+        "v_mov_b64 %0, %2 ; arm %5"
+        : "+v"(v.re), "+v"(v.im), "=&v"(w) : "v"(f.re), "v"(f.im), "n"(C));
+}
+
+// v <- v s
+template <int C>
+__device__ __forceinline__ void scale_by(Cx<float> &v, float s) {
+    asm("v_mul_f32 %0, %0, %2\n\tv_mul_f32 %1, %1, %2 ; arm %3" : "+v"(v.re), "+v"(v.im) : "v"(s), "n"(C));
+}
+template <int C>
+__device__ __forceinline__ void scale_by(Cx<double> &v, double s) {
+    asm("v_mul_f64 %0, %0, %2\n\tv_mul_f64 %1, %1, %2 ; arm %3" : "+v"(v.re), "+v"(v.im) : "v"(s), "n"(C));
+}
+
+// (x0, x1) <- M (x0, x1) where c, in place; general 2x2
+template <class R, int C>
+__device__ __forceinline__ void mix(Cx<R> &x0, Cx<R> &x1, const R (&m)[8], bool c) {
+    const Cx<R> y0 = cx<R>(fma_r(m[0], x0.re, fma_r(-m[1], x0.im, fma_r(m[2], x1.re, -m[3] * x1.im))),
+                           fma_r(m[0], x0.im, fma_r(m[1], x0.re, fma_r(m[2], x1.im, m[3] * x1.re))));
+    const Cx<R> y1 = cx<R>(fma_r(m[4], x0.re, fma_r(-m[5], x0.im, fma_r(m[6], x1.re, -m[7] * x1.im))),
+                           fma_r(m[4], x0.im, fma_r(m[5], x0.re, fma_r(m[6], x1.im, m[7] * x1.re))));
+    x0 = csel(c, y0, x0);
+    x1 = csel(c, y1, x1);
+    asm volatile("; arm %0" ::"n"(C));
+}
+
+// Every component in a register of its own: LDS reads and stores take register pairs, and a pair
+// that stayed one through the phase could be no operand of the updates above, so that each of
+// them copied it out and back. These statements keep the copies at the two ends of the phase.
+template <class R>
+__device__ __forceinline__ void own_register(R &x) {
+    asm("; own register" : "+v"(x));
+}
+
+template <class R, int A>
+__device__ __forceinline__ void apart(Cx<R> (&v)[A]) {
     static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
         constexpr int j = decltype(jc)::value;
-        if constexpr (((j >> P) & 1) == 0) {
-            constexpr int j1 = j + (1 << P);
-            if constexpr (SEL) {
-                Cx<R> y0, y1;
-                apply_form<R, F>(mm, x[j], x[j1], y0, y1);
-                const bool c = ok && (j & creg) == creg;
-                y[j] = csel(c, y0, x[j]);
-                y[j1] = csel(c, y1, x[j1]);
-            } else {
-                apply_form<R, F>(mm, x[j], x[j1], y[j], y[j1]);
-            }
-            __builtin_amdgcn_sched_barrier(0);   // one pair at a time: bounded register use
-        }
+        own_register(v[j].re);
+        own_register(v[j].im);
     });
 }
 
-// y = x times m11 where bit P of the register index is set, else m00 (PHASE: m00 == 1, those
-// indices copied), the choice made at compile time.
-template <class R, int A, int P, bool PHASE>
-__device__ __forceinline__ void op_diag(const Cx<R> (&x)[A], Cx<R> (&y)[A], const Mat2<R> &mm) {
-    static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-        constexpr int j = decltype(jc)::value;
-        if constexpr (((j >> P) & 1) != 0)
-            y[j] = cmul(mm.m11, x[j]);
-        else if constexpr (PHASE)
-            y[j] = x[j];
-        else
-            y[j] = cmul(mm.m00, x[j]);
-        __builtin_amdgcn_sched_barrier(0);
-    });
+// The register bits of the i-th pair of kArmPair2 / kArmSign2.
+__host__ __device__ constexpr int pair2_mask(int i) {
+    return i == 0 ? 3 : i == 1 ? 5 : i == 2 ? 6 : i == 3 ? 9 : i == 4 ? 10 : 12;
 }
 
-template <class R, int A, int H, int C>
-__device__ __forceinline__ void arm_body(const Cx<R> (&x)[A], Cx<R> (&y)[A], const Mat2<R> &mm, int creg, bool ok,
-                                         int tgt, const Cx<R> &f) {
-    constexpr int RB = Log2<A>::v;
-    // Complex64: each arm takes its own copy of the matrix entries (scalar registers, through
-    // an empty asm statement). A product of an entry and an amplitude that two arms share
-    // would otherwise be computed once above their branch and be live through either arm,
-    // which raised the kernel above 128 VGPRs (3 workgroups per CU instead of 4).
-    const Cx<R>(&xl)[A] = x;
-    Mat2<R> ml = mm;
-    if constexpr (sizeof(R) == 4)
-        asm volatile("; register op matrix %8"
-                     : "+s"(ml.m00.re), "+s"(ml.m00.im), "+s"(ml.m01.re), "+s"(ml.m01.im), "+s"(ml.m10.re),
-                       "+s"(ml.m10.im), "+s"(ml.m11.re), "+s"(ml.m11.im)
-                     : "n"(H * 64 + C));
-    if constexpr (C < kArmDiag) {
-        constexpr int F = (C % kArmPairSel) / 4, P = C % 4;
-        if constexpr (P < RB)
-            op_pair<R, A, P, F, (C >= kArmPairSel)>(xl, y, ml, creg, ok);
-        else
-            __builtin_unreachable();
-    } else if constexpr (C < kArmDiagCtrl) {
-        constexpr int P = C % 4;
-        if constexpr (P < RB)
-            op_diag<R, A, P, (C >= kArmDiagPhase)>(xl, y, ml);
-        else
-            __builtin_unreachable();
-    } else if constexpr (C == kArmDiagCtrl) {
-        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            const Cx<R> u = cmul(csel(((j >> tgt) & 1) != 0, ml.m11, ml.m00), xl[j]);
-            y[j] = csel(ok && (j & creg) == creg, u, xl[j]);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    } else {
-        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            y[j] = csel((j & creg) == creg, cmul(f, xl[j]), xl[j]);
-            __builtin_amdgcn_sched_barrier(0);
-        });
+// ---- gradient terms --------------------------------------------------------------------------
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// Sums over the wavefront of up to 16 consecutive slots: one v_mfma_f64_16x16x4f64 per term
+// multiplies the 64 lanes' values, as a 16 x 4 matrix, by a 4 x 16 matrix whose column `slot` is
+// one, so column slot of the accumulator collects the sums over groups of four lanes; flush
+// adds the accumulator's rows, in a fixed order, and leaves them in red[slot].
+template <int NW>
+struct SlotSums {
+    f64x4 acc;
+    __device__ __forceinline__ void init() { acc = f64x4{0., 0., 0., 0.}; }
+    __device__ __forceinline__ void flush(int group, double (*red)[NW], int n_slots, unsigned lane, unsigned wave) {
+        double s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        const int slot = group * 16 + (int)lane;
+        if (lane < 16 && slot < n_slots) red[slot][wave] = s;
+        acc = f64x4{0., 0., 0., 0.};
     }
-    arm_marker<H, C>();
-}
-
-// One op from x into y (H: 0 when x is the phase's first array, 1 for the second), one
-// switch: every arm ends at one join.
-template <class R, int A, int H>
-__device__ __forceinline__ void reg_op(const Cx<R> (&x)[A], Cx<R> (&y)[A], const Mat2<R> &mm, int arm, int creg,
-                                       bool ok, int tgt, const Cx<R> &f) {
-#define QG_REG_ARM(c)                                          \
-    case c:                                                    \
-        arm_body<R, A, H, c>(x, y, mm, creg, ok, tgt, f);      \
-        break;
-    switch (arm) {
-        QG_REG_ARM(0) QG_REG_ARM(1) QG_REG_ARM(2) QG_REG_ARM(3) QG_REG_ARM(4) QG_REG_ARM(5) QG_REG_ARM(6)
-        QG_REG_ARM(7) QG_REG_ARM(8) QG_REG_ARM(9) QG_REG_ARM(10) QG_REG_ARM(11) QG_REG_ARM(12) QG_REG_ARM(13)
-        QG_REG_ARM(14) QG_REG_ARM(15) QG_REG_ARM(16) QG_REG_ARM(17) QG_REG_ARM(18) QG_REG_ARM(19)
-        QG_REG_ARM(20) QG_REG_ARM(21) QG_REG_ARM(22) QG_REG_ARM(23) QG_REG_ARM(24) QG_REG_ARM(25)
-        QG_REG_ARM(26) QG_REG_ARM(27) QG_REG_ARM(28) QG_REG_ARM(29) QG_REG_ARM(30) QG_REG_ARM(31)
-        QG_REG_ARM(32) QG_REG_ARM(33)
-        default: __builtin_unreachable();
+    __device__ __forceinline__ void add(double v, int slot, unsigned lane) {
+        const double b = (lane & 15u) == (unsigned)(slot & 15) ? 1. : 0.;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, b, acc, 0, 0, 0);
     }
-#undef QG_REG_ARM
-}
-
-// The phase's amplitudes back to LDS, times the collected per-thread factor if there is one.
-template <class R, int A, int H>
-__device__ __forceinline__ void phase_store(Cx<R> *t, const Cx<R> (&v)[A], const PhaseBits &P, unsigned off,
-                                            const Cx<R> &tf, bool pending) {
-    constexpr int RB = Log2<A>::v;
-    // the store addresses are formed here again (one OR each) from an opaque copy of off: the
-    // compiler would otherwise keep the phase load's A addresses live through every op
-    asm volatile("; phase store %1" : "+v"(off) : "n"(H));
-    if (pending) {
-        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            t[off | reg_bits<RB>(P, j)] = cmul(tf, v[j]);
-        });
-    } else {
-        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            t[off | reg_bits<RB>(P, j)] = v[j];
-        });
-    }
-    arm_marker<H, 63>();
-}
-
-__host__ __device__ constexpr bool is_pair_kind(int k) { return k == kOpPair || k == kOpPairSwap || k == kOpPairReal; }
-
-// One op of a register phase, decoded for reg_op.
-template <class R>
-struct RegStep {
-    Mat2<R> mm;
-    Cx<R> f;          // kArmFactorReg: the factor
-    int arm, creg, tgt;
-    bool ok;          // the thread passes the op's controls on lane and wave bits
 };
 
-// The first op of phase P at index k or later that changes amplitudes (P.n_ops if none),
-// decoded into d. Ops skipped on the way: those whose controls outside the tile fail (the
-// same for the whole workgroup), and per-thread factors on every register index, which are
-// multiplied into tf.
-template <class R, bool B>
-__device__ __forceinline__ int next_reg_op(const RegProgram<R> &prog, const RegPhase &P, int k, u64 base,
-                                           unsigned off, const Mat2<R> *tm, Cx<R> &tf, bool &pending,
-                                           RegStep<R> &d) {
-    const Cx<R> one = cx<R>(R(1), R(0));
-    for (; k < P.n_ops; ++k) {
-        const int oi = P.op_begin + k;
-        const u64 gctrl = prog.ops[oi].gctrl;
-        if ((base & gctrl) != gctrl) continue;
-        if constexpr (B)
-            d.mm = tm[2 * prog.ops[oi].gate];
-        else
-            d.mm = prog.ops[oi].m;
-        const unsigned cthr = prog.ops[oi].cthr;
-        const int creg = prog.ops[oi].creg, tgt = prog.ops[oi].target, kind = prog.ops[oi].kind;
-        // no controls on lane, wave or register bits: straight-line updates, no tests
-        const bool plain = cthr == 0 && creg == 0;
-        d.ok = (off & cthr) == cthr;
-        d.creg = creg;
-        d.tgt = tgt;
-        d.f = one;
-        if (kind <= kRegPairReal) {
-            d.arm = (plain ? 0 : kArmPairSel) + 4 * kind + tgt;
-        } else if (kind <= kRegDiagPhase) {
-            d.arm = plain ? (kind == kRegDiag ? kArmDiag : kArmDiagPhase) + tgt : kArmDiagCtrl;
-        } else {
-            const u64 src = kind == kRegDiagThread ? (u64)off : base;
-            Cx<R> f = csel(((src >> tgt) & 1) != 0, d.mm.m11, d.mm.m00);
-            f = csel(cthr == 0 || d.ok, f, one);
-            if (creg == 0) {
-                tf = cmul(tf, f);
-                pending = true;
-                continue;
-            }
-            d.f = f;
-            d.arm = kArmFactorReg;
-        }
-        return k;
-    }
-    return P.n_ops;
-}
-
-// Batched passes (B): the state vector holds many circuits of one gate structure, item i's
-// amplitudes at [i << item_shift, (i + 1) << item_shift), and no tile spans two items. Gate g
-// then takes its matrix from the tile item's table, imats[2 (item n_gates + g)] (tables hold U
-// and U^dagger per gate; imats points at the one the pass applies), instead of from the op.
-// One tile per workgroup: persistent workgroups that load the next tile into registers while
-// they work on the current one need 32 more VGPRs (3 workgroups per CU instead of 4) and
-// measured slower (30-qubit complex64 step 610 ms against 507 ms).
-template <class R, int M, int T, bool B>
-__global__ __launch_bounds__(T) void k_tile_reg(Cx<R> *__restrict__ a, const RegProgram<R> prog, u64 first,
-                                                const Mat2<R> *__restrict__ imats, int n_gates, int item_shift) {
-    constexpr int A = (1 << M) / T, RB = Log2<A>::v, WB = Log2<T / 64>::v;
-    constexpr int W = Unit<R>::W, lw = W == 2 ? 1 : 0;
-    __shared__ Cx<R> t[1 << M];
-    const u64 base = tile_base(first + blockIdx.x, prog.pos, M);
-    const Mat2<R> *tm = nullptr;
-    if constexpr (B) tm = imats + 2 * (base >> item_shift) * (u64)n_gates;
-    tile_to_lds<R, T, (1 << (M - lw)) / T>(t, a, base, prog.pos, M, prog.low);
-    __syncthreads();
-    const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const Cx<R> one = cx<R>(R(1), R(0));
-    Cx<R> va[A], vb[A];
-    for (int ph = 0; ph < prog.n_phases; ++ph) {
-        const RegPhase P = prog.phases[ph];
-        unsigned off = 0;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) off |= ((lane >> k) & 1u) << P.lb(k);
-#pragma unroll
-        for (int k = 0; k < WB; ++k) off |= ((wave >> k) & 1u) << P.wb(k);
-        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            va[j] = t[off | reg_bits<RB>(P, j)];
-        });
-        // Diagonal gates with no register bit among their bits multiply all of a thread's
-        // amplitudes by one factor. They are collected in tf and applied once at the end of
-        // the phase: tf commutes with every other gate of the phase, which mixes or scales
-        // amplitudes of one thread only.
-        Cx<R> tf = one;
-        bool pending = false;
-        // ops in twos, va -> vb then vb -> va: only va is carried round the loop
-        int k = 0;
-        for (;;) {
-            RegStep<R> d;
-            k = next_reg_op<R, B>(prog, P, k, base, off, tm, tf, pending, d);
-            if (k >= P.n_ops) {
-                phase_store<R, A, 0>(t, va, P, off, tf, pending);
-                break;
-            }
-            reg_op<R, A, 0>(va, vb, d.mm, d.arm, d.creg, d.ok, d.tgt, d.f);
-            k = next_reg_op<R, B>(prog, P, k + 1, base, off, tm, tf, pending, d);
-            if (k >= P.n_ops) {
-                phase_store<R, A, 1>(t, vb, P, off, tf, pending);
-                break;
-            }
-            reg_op<R, A, 1>(vb, va, d.mm, d.arm, d.creg, d.ok, d.tgt, d.f);
-            ++k;
-        }
-        __syncthreads();
-    }
-    lds_to_tile<R, T, (1 << (M - lw)) / T>(a, t, base, prog.pos, M, prog.low);
-}
-
-// Phases of a pass: consecutive gates whose pair targets (pair[k] >= 0: local bit of a
-// non-diagonal gate) fit rb_count register bits. Each phase also fixes its lane bits (the
-// lowest 6 other tile bits) and wave bits (the rest).
-struct PhaseLayout {
-    std::vector<int> regs, lanes, waves;
-    int begin, end;
-};
-
-inline std::vector<PhaseLayout> plan_phase_layouts(const std::vector<int> &pair, int m, int rb_count, int wb_count) {
-    std::vector<PhaseLayout> out;
-    int k = 0;
-    const int n = (int)pair.size();
-    while (k < n) {
-        PhaseLayout P;
-        P.begin = k;
-        for (; k < n; ++k) {
-            if (pair[k] < 0) continue;
-            if (std::find(P.regs.begin(), P.regs.end(), pair[k]) != P.regs.end()) continue;
-            if ((int)P.regs.size() == rb_count) break;
-            P.regs.push_back(pair[k]);
-        }
-        P.end = k;
-        // pad with the highest free bits, so that the lane bits are the lowest ones: a
-        // wavefront then reads and writes LDS at consecutive addresses (no bank conflicts)
-        for (int b = m - 1; (int)P.regs.size() < rb_count && b >= 0; --b)
-            if (std::find(P.regs.begin(), P.regs.end(), b) == P.regs.end()) P.regs.push_back(b);
-        std::sort(P.regs.begin(), P.regs.end());
-        for (int b = 0; b < m; ++b)
-            if (std::find(P.regs.begin(), P.regs.end(), b) == P.regs.end()) {
-                if ((int)P.lanes.size() < 6)
-                    P.lanes.push_back(b);
-                else
-                    P.waves.push_back(b);
-            }
-        QG_REQUIRE((int)P.waves.size() == wb_count, "tile layout does not match the workgroup");
-        out.push_back(P);
-    }
-    return out;
-}
-
-// A register pass keeps its pair updates in order and puts each diagonal gate at a position,
-// between the pair updates on its lanes before and after it, whose phase has none of its tile
-// lanes as a register bit: there it is a per-thread factor, not an update of the register
-// arrays. (A pass that takes the gates of several layers otherwise meets a layer's RZ and CZ
-// right after the RY that made their lanes register bits.) Diagonal gates commute with each
-// other and with every pair update whose target is none of their lanes, as do the generators
-// of diagonal rotations, so the states and gradient terms are unchanged. order[begin, end) are
-// the pass's gates; is_diag(g), target_of(g) and lanes_of(g) (target and controls) describe
-// gate g; local maps a state lane to its tile bit (-1 outside the tile).
-template <class IsDiag, class TargetOf, class LanesOf>
-inline void place_diagonals(std::vector<int> &order, int begin, int end, const int *local, int m, int rb_count,
-                            int wb_count, IsDiag is_diag, TargetOf target_of, LanesOf lanes_of) {
-    std::vector<int> pairs, pair_local;
-    for (int i = begin; i < end; ++i)
-        if (!is_diag(order[i])) {
-            pairs.push_back(order[i]);
-            pair_local.push_back(local[target_of(order[i])]);
-        }
-    const int np = (int)pairs.size();
-    if (np == 0) return;
-    const std::vector<PhaseLayout> L = plan_phase_layouts(pair_local, m, rb_count, wb_count);
-    std::vector<int> phase_of(np, 0);
-    for (int ph = 0; ph < (int)L.size(); ++ph)
-        for (int k = L[ph].begin; k < L[ph].end; ++k) phase_of[k] = ph;
-    // a gate after pair update gp - 1 (before the first: gp = 0) runs in its phase
-    auto gap_phase = [&](int gp) { return gp >= 1 ? phase_of[gp - 1] : 0; };
-    std::vector<std::vector<int>> at(np + 1);
-    int seen = 0;
-    for (int i = begin; i < end; ++i) {
-        const int gi = order[i];
-        if (!is_diag(gi)) {
-            ++seen;
-            continue;
-        }
-        const std::vector<int> lanes = lanes_of(gi);
-        auto hits = [&](int k) { return std::find(lanes.begin(), lanes.end(), target_of(pairs[k])) != lanes.end(); };
-        int lo = 0, hi = np;
-        for (int k = seen - 1; k >= 0; --k)
-            if (hits(k)) {
-                lo = k + 1;
-                break;
-            }
-        for (int k = seen; k < np; ++k)
-            if (hits(k)) {
-                hi = k;
-                break;
-            }
-        auto bad = [&](int gp) {
-            const std::vector<int> &rg = L[gap_phase(gp)].regs;
-            for (int l : lanes)
-                if (local[l] >= 0 && std::find(rg.begin(), rg.end(), local[l]) != rg.end()) return true;
-            return false;
-        };
-        int best = seen;
-        for (int d = 1; bad(best) && (seen - d >= lo || seen + d <= hi); ++d) {
-            if (seen - d >= lo && !bad(seen - d))
-                best = seen - d;
-            else if (seen + d <= hi && !bad(seen + d))
-                best = seen + d;
-        }
-        at[best].push_back(gi);
-    }
-    int w = begin;
-    for (int gp = 0; gp <= np; ++gp) {
-        for (int gi : at[gp]) order[w++] = gi;
-        if (gp < np) order[w++] = pairs[gp];
-    }
-}
-
-// Packed form of a phase layout (ops [begin, end) of its pass).
-inline PhaseBits phase_bits(const PhaseLayout &P) {
-    PhaseBits h;
-    std::memset(&h, 0, sizeof(h));
-    for (int b = 0; b < (int)P.regs.size(); ++b) h.set(b, P.regs[b]);
-    for (int b = 0; b < (int)P.lanes.size(); ++b) h.set(5 + b, P.lanes[b]);
-    for (int b = 0; b < (int)P.waves.size(); ++b) h.set(11 + b, P.waves[b]);
-    h.op_begin = P.begin;
-    h.n_ops = P.end - P.begin;
-    return h;
-}
-
-inline int reg_position(const PhaseLayout &P, int bit) {
-    return (int)(std::find(P.regs.begin(), P.regs.end(), bit) - P.regs.begin());
-}
-
-// Register-pass encoding of a gate in phase P: kind (tile-pass kind, local bits: kOpPair*,
-// kOpDiag*), target (local bit, or state bit for kOpDiagOuter) and local controls lctrl.
-struct RegSplit {
-    int kind, target, creg;
-    unsigned cthr;
-};
-
-inline RegSplit split_for_phase(const PhaseLayout &P, int kind, int target, unsigned lctrl) {
-    RegSplit r;
-    r.creg = 0;
-    r.cthr = 0;
-    const int rb = (int)P.regs.size();
-    for (int b = 0; b < 32; ++b) {
-        if (((lctrl >> b) & 1u) == 0) continue;
-        const int p = reg_position(P, b);
-        if (p < rb)
-            r.creg |= 1 << p;
-        else
-            r.cthr |= 1u << b;
-    }
-    if (kind == kOpPair || kind == kOpPairSwap || kind == kOpPairReal) {
-        r.kind = kind == kOpPair ? kRegPair : kind == kOpPairSwap ? kRegPairSwap : kRegPairReal;
-        r.target = reg_position(P, target);
-        QG_REQUIRE(r.target < rb, "register phase: pair target is not a register bit");
-    } else if (kind == kOpDiagOuter) {
-        r.kind = kRegDiagOuter;
-        r.target = target;
-    } else {
-        const int p = reg_position(P, target);
-        if (p < rb) {
-            r.kind = kind == kOpDiagPhase ? kRegDiagPhase : kRegDiag;
-            r.target = p;
-        } else {
-            r.kind = kRegDiagThread;
-            r.target = target;
-        }
-    }
-    return r;
-}
-
-// Phase layouts of a register program built from tile-pass ops (local bits; an Op has m,
-// gctrl, lctrl, target and kind as TileOp does): false if the pass needs more phases than a
-// program holds.
-template <class R, class Op>
-bool plan_phases(RegProgram<R> &prog, const Op *ops, int m, int rb_count, int wb_count) {
-    std::vector<int> pair(prog.n_ops);
-    for (int k = 0; k < prog.n_ops; ++k) pair[k] = is_pair_kind(ops[k].kind) ? ops[k].target : -1;
-    const std::vector<PhaseLayout> L = plan_phase_layouts(pair, m, rb_count, wb_count);
-    if ((int)L.size() > kMaxPhases) return false;
-    prog.n_phases = (int)L.size();
-    for (int i = 0; i < prog.n_phases; ++i) {
-        prog.phases[i] = phase_bits(L[i]);
-        for (int k = L[i].begin; k < L[i].end; ++k) {
-            const RegSplit r = split_for_phase(L[i], ops[k].kind, ops[k].target, ops[k].lctrl);
-            RegOp<R> &op = prog.ops[k];
-            op.m = ops[k].m;
-            op.gctrl = ops[k].gctrl;
-            op.cthr = r.cthr;
-            op.creg = r.creg;
-            op.target = r.target;
-            op.kind = r.kind;
-            op.gate = 0;
-        }
-    }
-    return true;
-}
-
-// ---- register-resident adjoint sweep ------------------------------------------------------
-
-// Form code of a sweep op for the register passes: 4 * matrix form + generator (0 none, 1 X,
-// 2 Y, 3 Z). Pair ops: matrix form 1 swap, 2 real, 3 real diagonal with imaginary
-// off-diagonal, 0 anything else. Diagonal ops: 1 if m00 == 1 (only the |1> half changes),
-// else 0. The forms are exact properties of the entries, which rounding to the state
-// precision keeps.
-inline int sweep_form(const GateMatrix &u, int pauli, bool diagonal) {
-    const std::complex<double> m00 = u.m[0][0], m01 = u.m[0][1], m10 = u.m[1][0], m11 = u.m[1][1];
-    int f = 0;
-    if (diagonal) {
-        f = m00 == 1. ? 1 : 0;
-    } else if (m00 == 0. && m11 == 0. && m01 == 1. && m10 == 1.) {
-        f = 1;
-    } else if (m00.imag() == 0. && m01.imag() == 0. && m10.imag() == 0. && m11.imag() == 0.) {
-        f = 2;
-    } else if (m00.imag() == 0. && m11.imag() == 0. && m01.real() == 0. && m10.real() == 0.) {
-        f = 3;
-    }
-    return 4 * f + pauli;
-}
-
-template <class R>
-struct SweepOp {
-    Mat2<R> udag;       // applied to phi and lambda
-    Mat2<R> gen;        // generator of a rotation (entries 0, +-1, +-i)
-    u64 gctrl;
-    unsigned lctrl;
-    int target;         // local bit (pair, diag-local) or state bit (diag-outer)
-    int kind;           // (dwords: a uniform dword field is one scalar load)
-    int slot;           // gradient slot within the pass, -1 for fixed gates
-    int form;           // register passes: 4 * matrix form + generator (sweep_form)
-    int rkind, rtarget; // register passes: kind and target in the phase (RegOp)
-    int creg;           // register passes: controls on register bits (register positions)
-    unsigned cthr;      // register passes: controls on lane/wave bits (local bits)
-    int gate;           // batched passes: index of the gate in its circuit (udag unused)
-};
-
-struct SweepPass {
-    int m, low;
-    int op_begin, n_ops;
-    int phase_begin, n_phases, n_slots;
-    alignas(4) signed char pos[kTilePosMax];
-};
-
-// Register-resident sweep pass (m == SweepBits): phi and lambda tiles in registers, one LDS
-// round trip per phase; each rotation's tile term is reduced over the wavefront at once and
-// over the workgroup at the end of the pass.
 constexpr int kMaxSweepSlots = 96;
 
-typedef PhaseBits SweepPhase;   // op_begin relative to the pass
+// ---- register ops ----------------------------------------------------------------------------
 
-// One DPP step on a double: lane l receives v of the lane that control CTRL names, in the rows
-// enabled by ROWS (other rows receive 0). DPP moves run on the vector ALU, with no LDS
-// round trip.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_double(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-
-// Sum of v over the 64 lanes of a wavefront in a fixed order, valid in lane 63: butterflies
-// within quads (quad_perm [1,0,3,2], [2,3,0,1]) and rows (row_ror 4, 8) give every lane its
-// 16-lane row sum; row_bcast 15 then adds row 0 into row 1 and row 2 into row 3, and
-// row_bcast 31 adds rows 0+1 into row 3.
-__device__ __forceinline__ double wave_sum_lane63(double v) {
-    v += dpp_double<0xb1, 0xf>(v);
-    v += dpp_double<0x4e, 0xf>(v);
-    v += dpp_double<0x124, 0xf>(v);
-    v += dpp_double<0x128, 0xf>(v);
-    v += dpp_double<0x142, 0xa>(v);
-    v += dpp_double<0x143, 0xc>(v);
-    return v;
-}
-
-// Register sweep pair update on register bit P: the gradient term Im<lambda|G|phi> over the
-// pair for generator G (0 none, 1 X, 2 Y, 3 Z), accumulated in `acc` (state precision; the
-// caller widens each thread's sum to FP64), then U^dagger of form F on phi and lambda.
-// SEL: controls present; a pair changes (and contributes) only if ok && (j & creg) == creg,
-// written as selects so that no masked region needs copies of the registers.
-template <class R, int A, int P, int F, int G, bool SEL>
-__device__ __forceinline__ void reg_sweep_pair(Cx<R> (&vp)[A], Cx<R> (&vl)[A], const Mat2<R> &ud, int creg, bool ok,
-                                               R &acc) {
-    static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-        constexpr int j = decltype(jc)::value;
-        if constexpr (((j >> P) & 1) == 0) {
-            constexpr int j1 = j + (1 << P);
-            const Cx<R> p0 = vp[j], p1 = vp[j1], l0 = vl[j], l1 = vl[j1];
-            Cx<R> q0, q1, m0, m1;
-            apply_form<R, F>(ud, p0, p1, q0, q1);
-            apply_form<R, F>(ud, l0, l1, m0, m1);
-            if constexpr (SEL) {
-                const bool c = ok && (j & creg) == creg;
-                if constexpr (G != 0) acc += c ? add_pair_term<R, G>(R(0), p0, p1, l0, l1) : R(0);
-                vp[j] = csel(c, q0, p0);
-                vp[j1] = csel(c, q1, p1);
-                vl[j] = csel(c, m0, l0);
-                vl[j1] = csel(c, m1, l1);
-            } else {
-                acc = add_pair_term<R, G>(acc, p0, p1, l0, l1);
-                vp[j] = q0;
-                vp[j1] = q1;
-                vl[j] = m0;
-                vl[j1] = m1;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    });
-    pair_marker<64 + ((P * 4 + F) * 4 + G) * 2 + (SEL ? 1 : 0)>();
-}
-
-template <class R, int A, int F, int G, bool SEL>
-__device__ __forceinline__ void reg_sweep_pair_pos(Cx<R> (&vp)[A], Cx<R> (&vl)[A], const Mat2<R> &ud, int creg, bool ok,
-                                                   int p, R &acc) {
-    constexpr int RB = Log2<A>::v;
-    if constexpr (sizeof(R) == 8) {
-        // complex128: one-armed ifs keep the kernel's register count (and occupancy) lower
-        if constexpr (RB > 0) {
-            if (p == 0) reg_sweep_pair<R, A, 0, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-        }
-        if constexpr (RB > 1) {
-            if (p == 1) reg_sweep_pair<R, A, 1, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-        }
-        if constexpr (RB > 2) {
-            if (p == 2) reg_sweep_pair<R, A, 2, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-        }
-        if constexpr (RB > 3) {
-            if (p == 3) reg_sweep_pair<R, A, 3, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-        }
-        return;
-    }
-    switch (p) {
-        case 0:
-            if constexpr (RB > 0) {
-                reg_sweep_pair<R, A, 0, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-                break;
-            }
-            [[fallthrough]];
-        case 1:
-            if constexpr (RB > 1) {
-                reg_sweep_pair<R, A, 1, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-                break;
-            }
-            [[fallthrough]];
-        case 2:
-            if constexpr (RB > 2) {
-                reg_sweep_pair<R, A, 2, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-                break;
-            }
-            [[fallthrough]];
-        case 3:
-            if constexpr (RB > 3) {
-                reg_sweep_pair<R, A, 3, F, G, SEL>(vp, vl, ud, creg, ok, acc);
-                break;
-            }
-            [[fallthrough]];
-        default: __builtin_unreachable();
-    }
-}
-
-// Pair op of form code 4 F + G (see sweep_form): fixed gates in the general, swap and real
-// forms, RY (real, Y) and RX (form 3, X); any other combination takes the general matrix with
-// the op's own generator G (an RX whose matrix happens to be real, RX(0) = 1, keeps its X
-// term).
-template <class R, int A>
-__device__ __forceinline__ void reg_sweep_pair_at(Cx<R> (&vp)[A], Cx<R> (&vl)[A], const Mat2<R> &ud, int creg, bool ok,
-                                                  bool plain, int p, int form, R &acc) {
-    if (plain) {
-        switch (form) {
-            case 4 * 2 + 2: reg_sweep_pair_pos<R, A, 2, 2, false>(vp, vl, ud, 0, true, p, acc); break;
-            case 4 * 3 + 1: reg_sweep_pair_pos<R, A, 3, 1, false>(vp, vl, ud, 0, true, p, acc); break;
-            case 4 * 1 + 0: reg_sweep_pair_pos<R, A, 1, 0, false>(vp, vl, ud, 0, true, p, acc); break;
-            case 4 * 2 + 0: reg_sweep_pair_pos<R, A, 2, 0, false>(vp, vl, ud, 0, true, p, acc); break;
-            default:
-                switch (form & 3) {
-                    case 1: reg_sweep_pair_pos<R, A, 0, 1, false>(vp, vl, ud, 0, true, p, acc); break;
-                    case 2: reg_sweep_pair_pos<R, A, 0, 2, false>(vp, vl, ud, 0, true, p, acc); break;
-                    case 3: reg_sweep_pair_pos<R, A, 0, 3, false>(vp, vl, ud, 0, true, p, acc); break;
-                    default: reg_sweep_pair_pos<R, A, 0, 0, false>(vp, vl, ud, 0, true, p, acc); break;
+// The op of code C on the registers. m: coefficients; f: its factor in this thread (1 where its
+// controls on lane and wave bits fail, ok); acc receives the gradient term (NS == 2).
+template <int C, class R, int A, int NS>
+__device__ __forceinline__ void reg_arm(Cx<R> (&v)[NS][A], const R (&m)[8], const Cx<R> &f, int creg, bool ok,
+                                        int pauli, int tgt, u64 zsrc, R &acc) {
+    constexpr int RB = Log2<A>::v, F = C / 4, P = C % 4;
+    constexpr bool subset = F == kFamFactor || F == kFamSign || (C >= kArmPair2 && C < kArmFactorAny);
+    constexpr int mask = F == kFamFactor || F == kFamSign ? 1 << P
+                         : C >= kArmSign2                 ? pair2_mask(C - kArmSign2)
+                                                          : pair2_mask(C - kArmPair2);
+    constexpr bool sign = F == kFamSign || (C >= kArmSign2 && C < kArmFactorAny);
+    if constexpr (F <= kFamAny) {
+        if constexpr (P >= RB) {
+            __builtin_unreachable();
+        } else {
+            const R t = m[0];
+            const u64 okm = F == kFamSwap ? __ballot(ok) : 0;
+            static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                if constexpr (((j >> P) & 1) == 0) {
+                    constexpr int j1 = j + (1 << P);
+                    const bool c = ok && (j & creg) == creg;
+                    if constexpr (NS == 2 && F <= kFamXk)
+                        acc = add_pair_term<R, (F <= kFamYk ? 2 : 1)>(acc, v[0][j], v[0][j1], v[NS - 1][j],
+                                                                      v[NS - 1][j1]);
+                    if constexpr (NS == 2 && F == kFamAny) {
+                        R w = R(0);
+                        if (pauli == 1) w = add_pair_term<R, 1>(w, v[0][j], v[0][j1], v[NS - 1][j], v[NS - 1][j1]);
+                        if (pauli == 2) w = add_pair_term<R, 2>(w, v[0][j], v[0][j1], v[NS - 1][j], v[NS - 1][j1]);
+                        acc += c ? w : R(0);
+                    }
+                    if constexpr (F <= kFamXk) {
+                        constexpr bool X = F >= kFamX, K = F == kFamYk || F == kFamXk;
+                        Cx<R> &a0 = v[0][j], &a1 = v[0][j1], &b0 = v[NS - 1][j], &b1 = v[NS - 1][j1];
+                        if constexpr (NS == 1 && !X && !K) rot_t<C>(a0.re, a1.re, a0.im, a1.im, t);
+                        if constexpr (NS == 1 && !X && K) rot_k<C>(a0.re, a1.re, a0.im, a1.im, t);
+                        if constexpr (NS == 1 && X && !K) rot_t<C>(a0.re, a1.im, a1.re, a0.im, t);
+                        if constexpr (NS == 1 && X && K) rot_k<C>(a0.re, a1.im, a1.re, a0.im, t);
+                        if constexpr (NS == 2 && !X && !K)
+                            rot_t<C>(a0.re, a1.re, a0.im, a1.im, b0.re, b1.re, b0.im, b1.im, t);
+                        if constexpr (NS == 2 && !X && K)
+                            rot_k<C>(a0.re, a1.re, a0.im, a1.im, b0.re, b1.re, b0.im, b1.im, t);
+                        if constexpr (NS == 2 && X && !K)
+                            rot_t<C>(a0.re, a1.im, a1.re, a0.im, b0.re, b1.im, b1.re, b0.im, t);
+                        if constexpr (NS == 2 && X && K)
+                            rot_k<C>(a0.re, a1.im, a1.re, a0.im, b0.re, b1.im, b1.re, b0.im, t);
+                    } else {
+#pragma unroll
+                        for (int s = 0; s < NS; ++s) {
+                            Cx<R> &x0 = v[s][j], &x1 = v[s][j1];
+                            if constexpr (F == kFamSwap) {
+                                const u64 mk = (j & creg) == creg ? okm : 0;
+                                swap_if<C>(x0, x1, mk);
+                            } else {
+                                mix<R, C>(x0, x1, m, c);
+                            }
+                        }
+                    }
                 }
-                break;
+            });
         }
-        return;
-    }
-    // controlled gates: general matrix, any generator
-    switch (form & 3) {
-        case 1: reg_sweep_pair_pos<R, A, 0, 1, true>(vp, vl, ud, creg, ok, p, acc); break;
-        case 2: reg_sweep_pair_pos<R, A, 0, 2, true>(vp, vl, ud, creg, ok, p, acc); break;
-        case 3: reg_sweep_pair_pos<R, A, 0, 3, true>(vp, vl, ud, creg, ok, p, acc); break;
-        default: reg_sweep_pair_pos<R, A, 0, 0, true>(vp, vl, ud, creg, ok, p, acc); break;
+    } else if constexpr (subset) {
+        if constexpr (mask >= A) {
+            __builtin_unreachable();
+        } else {
+            const R sg = ok ? R(-1) : R(1);
+            static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                if constexpr ((j & mask) == mask) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) {
+                        if constexpr (sign) {
+                            scale_by<C>(v[s][j], sg);
+                        } else {
+                            mul_by<C>(v[s][j], f);
+                        }
+                    }
+                }
+            });
+        }
+    } else if constexpr (F == kFamZ) {
+        if constexpr (NS == 1 || P >= RB) {
+            __builtin_unreachable();
+        } else {
+            static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                if constexpr (((j >> P) & 1) == 0)
+                    acc = add_im_conj_mul(acc, v[1][j], v[0][j]);
+                else
+                    acc = add_im_conj_mul(acc, v[0][j], v[1][j]);
+            });
+            acc = ok ? acc : R(0);
+        }
+    } else if constexpr (C == kArmFactorAny) {
+        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            const Cx<R> fj = csel((j & creg) == creg, f, cx<R>(R(1), R(0)));
+#pragma unroll
+            for (int s = 0; s < NS; ++s) mul_by<C>(v[s][j], fj);
+        });
+    } else {   // Z term with controls on register bits; target: register position, or RB + bit
+        if constexpr (NS == 1) {
+            __builtin_unreachable();
+        } else {
+            const bool reg = tgt < RB, tb = !reg && ((zsrc >> ((tgt & 0x7f) - RB)) & 1) != 0;
+            static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                const R w = add_im_conj_mul(R(0), v[1][j], v[0][j]);
+                const bool b = reg ? ((j >> tgt) & 1) != 0 : tb;
+                acc += ok && (j & creg) == creg ? (b ? -w : w) : R(0);
+            });
+        }
     }
 }
 
-// Registers of one state in phase layout (off, P) <-> LDS tile t.
-template <class R, int A, int RB>
-__device__ __forceinline__ void regs_from_lds(Cx<R> (&v)[A], const Cx<R> *t, unsigned off, const PhaseBits &P) {
-    static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-        constexpr int j = decltype(jc)::value;
-        v[j] = t[off | reg_bits<RB>(P, j)];
-    });
+// ---- one phase -------------------------------------------------------------------------------
+
+// What a thread carries through a phase besides its amplitudes.
+template <class R>
+struct PhaseState {
+    Cx<R> tf;          // factor per thread, pending: there is one
+    Scale<R> sc;       // factor left out of the rotations, scaled: there is one
+    unsigned sign;     // sign bit of the factor per thread
+    bool pending, scaled;
+    __device__ __forceinline__ void init(double carry) {
+        tf = cx<R>(R(1), R(0));
+        sc.init(carry);
+        sign = 0;
+        pending = scaled = false;
+    }
+    // At the end of the phase: f is the factor to apply (its imaginary part only if pending), and
+    // carry what rounding it left out, for the next phase (the norm of the whole state would
+    // otherwise be off by up to half a unit in the last place per phase).
+    __device__ __forceinline__ Cx<R> finish(double &carry) const {
+        if (!pending && !scaled) return cx<R>(R(1), R(0));
+        const double s = sizeof(R) == 8 ? sc.value() : pending ? sc.hi : (double)(R)sc.hi;
+        carry = ((sc.hi - s) + sc.lo) * __builtin_amdgcn_rcp(s);
+        if (!pending) return cx<R>((R)s, R(0));
+        const double t = __longlong_as_double(__double_as_longlong(s) ^ (long long)((u64)sign << 32));
+        return cx<R>((R)((double)tf.re * t), (R)((double)tf.im * t));
+    }
+};
+
+// The ops of a phase on NS states in registers. ops: the pass's ops (one more is read than there
+// are); tm: the item's coefficient table (B), kCoefs to a row; sums, red: the gradient terms of
+// the sweep (NS == 2). One loop with one exit: with two, or with a loop inside for the ops that
+// leave the registers alone, the compiler kept the registers of several iterations alive and
+// copied them.
+template <class R, int A, int NS, bool B, int NW>
+__device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops, int op_begin, int n_ops, u64 base,
+                                          unsigned off, const R *tm, PhaseState<R> &st, SlotSums<NW> &sums,
+                                          double (*red)[NW], int n_slots, unsigned lane, unsigned wave) {
+    const Cx<R> one = cx<R>(R(1), R(0));
+#pragma unroll
+    for (int s = 0; s < NS; ++s) apart(v[s]);
+    double u = 0.;   // sum of Im(conj(lambda) phi), true scale
+    OpWords<R> op, next;
+    op.load(ops + op_begin);
+    for (int k = op_begin; k < op_begin + n_ops; ++k) {
+        op.arrive();
+        next.load(ops + k + 1);   // read while this op runs
+        const int slot = op.slot();
+        if ((base & op.gctrl()) == op.gctrl()) {
+            const unsigned code = op.code(), cthr = op.cthr();
+            const bool ok = (off & cthr) == cthr;
+            const int tgt = (int)((code >> 8) & 0xffu), creg = (int)((code >> 16) & 0xffu);
+            R m[8];
+            if constexpr (B) {
+                const R *row = tm + (size_t)op.row() * kCoefs + (code >> 28);
+                for (int i = 0; i < 4; ++i) m[i] = row[i];
+            } else {
+                for (int i = 0; i < 4; ++i) m[i] = op.coef(i);
+            }
+            double term = 0.;
+            R acc = R(0);
+            int arm = (int)(code & 0xffu);
+            if (arm < 16) arm += m[1] != R(0) ? 4 : 0;   // rotations: the form comes with the coefficients
+            const u64 zsrc = (tgt & 0x80) ? base : (u64)off;
+#define QG_ARM(C_)                                                                                  \
+    case C_: {                                                                                      \
+        const Cx<R> f = csel(ok, cx<R>(m[0], m[1]), one);                                          \
+        if constexpr ((C_) / 4 == kFamAny) {   /* the second half of the matrix */                    \
+            if constexpr (B) {                                                                     \
+                for (int i = 4; i < 8; ++i) m[i] = tm[(size_t)op.row() * kCoefs + i];                 \
+            } else {                                                                               \
+                for (int i = 4; i < 8; ++i) m[i] = next.coef(i - 4);                                \
+            }                                                                                      \
+        }                                                                                          \
+        reg_arm<(C_), R, A, NS>(v, m, f, creg, ok, (int)((code >> 24) & 0xfu), tgt, zsrc, acc);          \
+        if constexpr (NS == 2) term = (double)acc * (st.sc.hi * st.sc.hi);                               \
+        if constexpr ((C_) < 16) {                                                                    \
+            st.sc.times(m[2], m[3]);                                                               \
+            st.scaled = true;                                                                      \
+        }                                                                                          \
+        break;                                                                                     \
+    }
+#define QG_ARMS(C_) QG_ARM(C_) QG_ARM(C_ + 1) QG_ARM(C_ + 2) QG_ARM(C_ + 3)
+            switch (arm) {
+                QG_ARMS(0) QG_ARMS(4) QG_ARMS(8) QG_ARMS(12) QG_ARMS(16) QG_ARMS(20) QG_ARMS(24) QG_ARMS(28)
+                QG_ARMS(32) QG_ARMS(36) QG_ARMS(40) QG_ARMS(44) QG_ARM(48) QG_ARM(49)
+                case kArmThread:
+                case kArmThreadCtrl: {
+                    const bool b = ((off >> tgt) & 1u) != 0;
+                    Cx<R> f = csel(b, cx<R>(m[2], m[3]), cx<R>(m[0], m[1]));
+                    if (arm == kArmThreadCtrl) f = csel(ok, f, one);
+                    st.tf = cmul(st.tf, f);
+                    st.pending = true;
+                    if constexpr (NS == 2) {
+                        term = b ? -u : u;
+                        if (arm == kArmThreadCtrl) term = ok ? term : 0.;
+                    }
+                    break;
+                }
+                case kArmOuter: {
+                    const bool b = ((base >> tgt) & 1u) != 0;
+                    const Cx<R> f = csel(ok, csel(b, cx<R>(m[2], m[3]), cx<R>(m[0], m[1])), one);
+                    st.tf = cmul(st.tf, f);
+                    st.pending = true;
+                    if constexpr (NS == 2) term = ok ? (b ? -u : u) : 0.;
+                    break;
+                }
+                case kArmPhase:
+                    st.tf = cmul(st.tf, csel(ok, cx<R>(m[0], m[1]), one));
+                    st.pending = true;
+                    break;
+                case kArmSign:
+                    st.sign ^= ok ? 0x80000000u : 0u;
+                    st.pending = true;
+                    break;
+                case kArmU:
+                    if constexpr (NS == 2) {
+                        R w = R(0);
+                        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+                            constexpr int j = decltype(jc)::value;
+                            w = add_im_conj_mul(w, v[1][j], v[0][j]);
+                        });
+                        u = (double)w * (st.sc.hi * st.sc.hi);
+                    }
+                    break;
+                case kArmFlush:
+                    if constexpr (NS == 2) sums.flush(tgt, red, n_slots, lane, wave);
+                    break;
+                default: break;
+            }
+#undef QG_ARM
+#undef QG_ARMS
+            if constexpr (NS == 2)
+                if (slot >= 0) sums.add(term, slot, lane);
+        }
+        op = next;
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) apart(v[s]);
 }
 
-template <class R, int A, int RB>
-__device__ __forceinline__ void regs_to_lds(Cx<R> *t, const Cx<R> (&v)[A], unsigned off, const PhaseBits &P) {
-    static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-        constexpr int j = decltype(jc)::value;
-        t[off | reg_bits<RB>(P, j)] = v[j];
-    });
+// ---- layouts ---------------------------------------------------------------------------------
+
+// LDS index of local tile index l: bits 5 to 9 and 10 to 12 folded onto the low five, so that a
+// wavefront whose lane bits start above bit 0 still spreads over the banks. Linear over XOR:
+// swizzle(a ^ b) = swizzle(a) ^ swizzle(b).
+__host__ __device__ __forceinline__ unsigned swizzle(unsigned l) { return l ^ ((l >> 5) & 31u) ^ ((l >> 10) & 31u); }
+
+// Local-index bits of register index j in phase P (uniform: a scalar value).
+template <int RB>
+__device__ __forceinline__ unsigned reg_bits(const PhaseBits &P, int j) {
+    unsigned l = 0;
+#pragma unroll
+    for (int k = 0; k < RB; ++k) l |= (((unsigned)j >> k) & 1u) << P.rb(k);
+    return l;
 }
 
 template <int WB>
@@ -877,184 +810,392 @@ __device__ __forceinline__ unsigned phase_offset(const PhaseBits &P, unsigned la
     return off;
 }
 
+// Registers of one state in phase layout (off, P) <- LDS tile t.
+template <class R, int A, int RB>
+__device__ __forceinline__ void regs_from_lds(Cx<R> (&v)[A], const Cx<R> *t, unsigned soff, const PhaseBits &P) {
+    static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value;
+        v[j] = t[soff ^ swizzle(reg_bits<RB>(P, j))];
+    });
+}
+
+// LDS tile t <- registers, times the factor f of the phase.
+template <class R, int A, int RB>
+__device__ __forceinline__ void regs_to_lds(Cx<R> *t, const Cx<R> (&v)[A], unsigned soff, const PhaseBits &P,
+                                            const PhaseState<R> &st, const Cx<R> &f) {
+    // an opaque copy of soff: the addresses are formed here again (one XOR each) instead of being
+    // kept from the phase's load through every op
+    asm volatile("; phase store" : "+v"(soff));
+    if (st.pending) {
+        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            t[soff ^ swizzle(reg_bits<RB>(P, j))] = cmul(f, v[j]);
+        });
+    } else if (st.scaled) {
+        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            t[soff ^ swizzle(reg_bits<RB>(P, j))] = cx<R>(v[j].re * f.re, v[j].im * f.re);
+        });
+    } else {
+        static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            t[soff ^ swizzle(reg_bits<RB>(P, j))] = v[j];
+        });
+    }
+}
+
+// HBM <-> swizzled LDS tile of 2^M amplitudes, all of a thread's 16-byte accesses in flight at
+// once. Unit c T + tid has local index (c T + tid) << lw, whose two parts occupy disjoint bits:
+// one deposit per thread and one per chunk (the same for the whole workgroup).
+template <class R, int T, int M>
+__device__ __forceinline__ void tile_in(Cx<R> *t, const Cx<R> *a, u64 base, const signed char *pos, int low) {
+    constexpr int W = Unit<R>::W, lw = W == 2 ? 1 : 0, N = (1 << (M - lw)) / T;
+    const u64 dt = base | deposit((unsigned)threadIdx.x << lw, pos, M, low);
+    Amps<R> x[N];
+#pragma unroll
+    for (int c = 0; c < N; ++c) x[c] = load_unit(a, (dt | deposit((unsigned)(c * T) << lw, pos, M, low)) >> lw);
+    const unsigned s = swizzle((unsigned)threadIdx.x << lw);
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+#pragma unroll
+        for (int j = 0; j < W; ++j) t[s ^ swizzle(((unsigned)(c * T) << lw) | (unsigned)j)] = x[c].v[j];
+}
+
+template <class R, int T, int M>
+__device__ __forceinline__ void tile_out(Cx<R> *a, const Cx<R> *t, u64 base, const signed char *pos, int low) {
+    constexpr int W = Unit<R>::W, lw = W == 2 ? 1 : 0, N = (1 << (M - lw)) / T;
+    const u64 dt = base | deposit((unsigned)threadIdx.x << lw, pos, M, low);
+    const unsigned s = swizzle((unsigned)threadIdx.x << lw);
+    Amps<R> x[N];
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+#pragma unroll
+        for (int j = 0; j < W; ++j) x[c].v[j] = t[s ^ swizzle(((unsigned)(c * T) << lw) | (unsigned)j)];
+#pragma unroll
+    for (int c = 0; c < N; ++c) store_unit(a, (dt | deposit((unsigned)(c * T) << lw, pos, M, low)) >> lw, x[c]);
+}
+
+// ---- forward pass ----------------------------------------------------------------------------
+
+// The program of a forward pass travels in the kernel arguments (under 4 KiB).
+template <class R>
+struct RegProgram {
+    int n_ops, n_phases, low;
+    alignas(4) signed char pos[kTilePosMax];
+    PhaseBits phases[kMaxPhases];
+    RegOp<R> ops[TileCfg<R>::MaxRegOps + 1];   // one more is read than there are
+};
+static_assert(sizeof(RegProgram<float>) <= 3584 && sizeof(RegProgram<double>) <= 3584, "kernel argument size");
+
+// Batched passes (B): the state vector holds many circuits of one gate structure, item i's
+// amplitudes at [i << item_shift, (i + 1) << item_shift), and no tile spans two items. An op
+// then takes its coefficients from the tile item's table of n_rows rows of kCoefs.
+// One tile per workgroup: persistent workgroups that load the next tile into registers while
+// they work on the current one need 32 more VGPRs (3 workgroups per CU instead of 4) and
+// measured slower.
+template <class R, int M, int T, bool B>
+__global__ __launch_bounds__(T) void k_tile_reg(Cx<R> *__restrict__ a, const RegProgram<R> prog, u64 first,
+                                                const R *__restrict__ coefs, int n_rows, int item_shift) {
+    constexpr int A = (1 << M) / T, RB = Log2<A>::v, WB = Log2<T / 64>::v;
+    __shared__ Cx<R> t[1 << M];
+    const u64 base = tile_base(first + blockIdx.x, prog.pos, M);
+    const R *tm = nullptr;
+    if constexpr (B) tm = coefs + (base >> item_shift) * (u64)n_rows * kCoefs;
+    tile_in<R, T, M>(t, a, base, prog.pos, prog.low);
+    __syncthreads();
+    const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    Cx<R> v[1][A];
+    SlotSums<1> none;
+    double carry = 0.;
+    for (int ph = 0; ph < prog.n_phases; ++ph) {
+        const PhaseBits P = prog.phases[ph];
+        const unsigned off = phase_offset<WB>(P, lane, wave);
+        regs_from_lds<R, A, RB>(v[0], t, swizzle(off), P);
+        PhaseState<R> st;
+        st.init(carry);
+        run_phase<R, A, 1, B, 1>(v, prog.ops, P.op_begin, P.n_ops, base, off, tm, st, none, nullptr, 0, lane, wave);
+        const Cx<R> f = st.finish(carry);
+        regs_to_lds<R, A, RB>(t, v[0], swizzle(off), P, st, f);
+        __syncthreads();
+    }
+    tile_out<R, T, M>(a, t, base, prog.pos, prog.low);
+}
+
+// ---- adjoint sweep ---------------------------------------------------------------------------
+
+struct SweepPass {
+    int low;
+    int op_begin;          // ops of the pass in the op table; its phases count from there
+    int phase_begin, n_phases, n_slots;
+    alignas(4) signed char pos[kTilePosMax];
+};
+
 // phi and lambda tiles in registers, one LDS tile each for the layout changes. Every LDS
 // location written at the end of a phase is the one the same thread read at its start, so
-// only the hand-overs between layouts need barriers.
-// B: batched passes, as in k_tile_reg (imats points at the U^dagger entries).
+// only the hand-overs between layouts need barriers. Each rotation's tile term is left in
+// partial[slot * n_tiles + tile].
 template <class R, int M, int T, bool B>
 __global__ __launch_bounds__(T) void k_tile_sweep_reg(Cx<R> *__restrict__ phi, Cx<R> *__restrict__ lam,
-                                                      const SweepPass pass, const SweepOp<R> *__restrict__ ops,
-                                                      const SweepPhase *__restrict__ phases,
+                                                      const SweepPass pass, const RegOp<R> *__restrict__ ops,
+                                                      const PhaseBits *__restrict__ phases,
                                                       double *__restrict__ partial, u64 n_tiles, u64 first,
-                                                      const Mat2<R> *__restrict__ imats, int n_gates,
-                                                      int item_shift) {
+                                                      const R *__restrict__ coefs, int n_rows, int item_shift) {
     constexpr int A = (1 << M) / T, RB = Log2<A>::v, WB = Log2<T / 64>::v, NW = T / 64;
-    constexpr int W = Unit<R>::W, lw = W == 2 ? 1 : 0;
     __shared__ Cx<R> tp[1 << M];
     __shared__ Cx<R> tl[1 << M];
     __shared__ double red[kMaxSweepSlots][NW];
     const u64 tile = first + blockIdx.x;
     const u64 base = tile_base(tile, pass.pos, M);
-    const Mat2<R> *tm = nullptr;
-    if constexpr (B) tm = imats + 2 * (base >> item_shift) * (u64)n_gates;
-    // U^dagger of an op: from the op, or from the tile item's table
-    auto udag_of = [&](const SweepOp<R> &op) __attribute__((always_inline)) -> Mat2<R> {
-        if constexpr (B)
-            return tm[2 * op.gate];
-        else
-            return op.udag;
-    };
-    constexpr int upt = (1 << (M - lw)) / T;   // units per thread
+    const R *tm = nullptr;
+    if constexpr (B) tm = coefs + (base >> item_shift) * (u64)n_rows * kCoefs;
     const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    Cx<R> vp[A], vl[A];
-    SweepPhase P = phases[pass.phase_begin];
-    unsigned off = phase_offset<WB>(P, lane, wave);
-    tile_to_lds<R, T, upt>(tp, phi, base, pass.pos, M, pass.low);
-    tile_to_lds<R, T, upt>(tl, lam, base, pass.pos, M, pass.low);
+    Cx<R> v[2][A];
+    tile_in<R, T, M>(tp, phi, base, pass.pos, pass.low);
+    tile_in<R, T, M>(tl, lam, base, pass.pos, pass.low);
+    for (int k = threadIdx.x; k < pass.n_slots * NW; k += T) red[k / NW][k % NW] = 0.;   // slots off in this tile
     __syncthreads();
-    regs_from_lds<R, A, RB>(vp, tp, off, P);
-    regs_from_lds<R, A, RB>(vl, tl, off, P);
+    SlotSums<NW> sums;
+    sums.init();
+    double carry = 0.;
     for (int ph = 0; ph < pass.n_phases; ++ph) {
-        if (ph > 0) {   // registers from phase ph - 1's layout to phase ph's
-            const SweepPhase Q = phases[pass.phase_begin + ph];
-            const unsigned qoff = phase_offset<WB>(Q, lane, wave);
-            regs_to_lds<R, A, RB>(tp, vp, off, P);
-            regs_to_lds<R, A, RB>(tl, vl, off, P);
-            __syncthreads();
-            regs_from_lds<R, A, RB>(vp, tp, qoff, Q);
-            regs_from_lds<R, A, RB>(vl, tl, qoff, Q);
-            P = Q;
-            off = qoff;
-        }
-        // As in the forward register pass, diagonal gates on no register bit are one factor per
-        // thread (tf), applied to phi and lambda at the end of the phase. Diagonal gates
-        // leave w_j = Im(conj(lambda_j) phi_j) unchanged (|factor| = 1), so the generator-Z
-        // terms of a run of diagonal gates all use the same w: an RZ on a lane, wave or outer
-        // bit contributes +-U with U = sum_j w_j, computed once per run (have_u).
-        // Runs of gates that leave the registers alone (fused diagonals, gates whose controls
-        // outside the tile are not all set here) go through an inner loop that carries only
-        // tf, U and the slot terms: the register arrays cross a loop back-edge (where the
-        // compiler inserts copies of them) once per register-changing gate, not once per gate.
-        Cx<R> tf = cx<R>(R(1), R(0));
-        bool pending = false, have_u = false;
-        R u_sum = R(0);
-        int k = 0;
-        while (k < P.n_ops) {
-            for (; k < P.n_ops; ++k) {
-                const SweepOp<R> &op = ops[pass.op_begin + P.op_begin + k];
-                const bool on = (base & op.gctrl) == op.gctrl;
-                const int kind = op.rkind, creg = op.creg, form = op.form;
-                if (on && (kind < kRegDiagThread || creg != 0)) break;   // changes the registers
-                R acc = R(0);
-                if (on) {
-                    const unsigned cthr = op.cthr;
-                    const bool ok = (off & cthr) == cthr;
-                    const u64 src = kind == kRegDiagThread ? (u64)off : base;
-                    const bool one = ((src >> op.rtarget) & 1) != 0;
-                    const Mat2<R> ud = udag_of(op);
-                    Cx<R> f = csel(one, ud.m11, ud.m00);
-                    f = csel(cthr == 0 || ok, f, cx<R>(R(1), R(0)));
-                    if ((form & 3) == 3) {
-                        if (!have_u) {
-                            u_sum = R(0);
-                            static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-                                constexpr int j = decltype(jc)::value;
-                                u_sum = add_im_conj_mul(u_sum, vl[j], vp[j]);
-                            });
-                            have_u = true;
-                        }
-                        acc = ok ? (one ? -u_sum : u_sum) : R(0);
-                    }
-                    tf = cmul(tf, f);
-                    pending = true;
-                }
-                if (op.slot >= 0) {
-                    const double s = wave_sum_lane63((double)acc);
-                    if (lane == 63) red[op.slot][wave] = s;
-                }
-            }
-            if (k == P.n_ops) break;
-            // one gate that changes the registers (it is on)
-            const SweepOp<R> &op = ops[pass.op_begin + P.op_begin + k];
-            ++k;
-            const unsigned cthr = op.cthr;
-            const int creg = op.creg, tgt = op.rtarget, kind = op.rkind, form = op.form;
-            const bool ok = (off & cthr) == cthr;
-            const bool plain = cthr == 0 && creg == 0;
-            R acc = R(0);
-            if (kind <= kRegPairReal) {
-                // tf (pending diagonal factor) commutes with the pair update, and the pair's
-                // gradient term is unchanged by a common unit-modulus factor of phi and lambda
-                reg_sweep_pair_at<R, A>(vp, vl, udag_of(op), creg, ok, plain, tgt, form, acc);
-                have_u = false;
-            } else {
-                const bool zgen = (form & 3) == 3;
-                const Mat2<R> ud = udag_of(op);
-                const Cx<R> f0 = ud.m00, f1 = ud.m11;
-                if (kind <= kRegDiagPhase) {
-                    // target on register position tgt: the factor of index j is a scalar choice
-                    static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-                        constexpr int j = decltype(jc)::value;
-                        const bool one = ((j >> tgt) & 1) != 0;
-                        const Cx<R> f = csel(one, f1, f0);
-                        const Cx<R> x = vp[j], y = vl[j];
-                        const R w = zgen ? im_conj_mul(y, x) : R(0);
-                        const Cx<R> nx = cmul(f, x), ny = cmul(f, y);
-                        if (plain) {
-                            acc += one ? -w : w;
-                            vp[j] = nx;
-                            vl[j] = ny;
-                        } else {
-                            const bool c = ok && (j & creg) == creg;
-                            acc += c ? (one ? -w : w) : R(0);
-                            vp[j] = csel(c, nx, x);
-                            vl[j] = csel(c, ny, y);
-                        }
-                    });
-                } else {   // lane, wave or outer target with controls on register bits
-                    const u64 src = kind == kRegDiagThread ? (u64)off : base;
-                    const bool one = ((src >> tgt) & 1) != 0;
-                    Cx<R> f = csel(one, f1, f0);
-                    f = csel(cthr == 0 || ok, f, cx<R>(R(1), R(0)));
-                    static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-                        constexpr int j = decltype(jc)::value;
-                        const bool c = (j & creg) == creg;   // scalar
-                        const Cx<R> x = vp[j], y = vl[j];
-                        if (zgen) {
-                            const R w = im_conj_mul(y, x);
-                            acc += (c && ok) ? (one ? -w : w) : R(0);
-                        }
-                        if (c) {
-                            vp[j] = cmul(f, x);
-                            vl[j] = cmul(f, y);
-                        }
-                    });
-                }
-            }
-            if (op.slot >= 0) {
-                const double s = wave_sum_lane63((double)acc);
-                if (lane == 63) red[op.slot][wave] = s;
-            }
-        }
-        if (pending) {
-            static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
-                constexpr int j = decltype(jc)::value;
-                vp[j] = cmul(tf, vp[j]);
-                vl[j] = cmul(tf, vl[j]);
-            });
-        }
+        const PhaseBits P = phases[pass.phase_begin + ph];
+        const unsigned off = phase_offset<WB>(P, lane, wave);
+        const unsigned soff = swizzle(off);
+        regs_from_lds<R, A, RB>(v[0], tp, soff, P);
+        regs_from_lds<R, A, RB>(v[1], tl, soff, P);
+        PhaseState<R> st;
+        st.init(carry);
+        run_phase<R, A, 2, B, NW>(v, ops, pass.op_begin + P.op_begin, P.n_ops, base, off, tm, st, sums, red,
+                                  pass.n_slots, lane, wave);
+        const Cx<R> f = st.finish(carry);
+        regs_to_lds<R, A, RB>(tp, v[0], soff, P, st, f);
+        regs_to_lds<R, A, RB>(tl, v[1], soff, P, st, f);
+        __syncthreads();
     }
-    regs_to_lds<R, A, RB>(tp, vp, off, P);
-    regs_to_lds<R, A, RB>(tl, vl, off, P);
-    __syncthreads();
-    lds_to_tile<R, T, upt>(phi, tp, base, pass.pos, M, pass.low);
-    lds_to_tile<R, T, upt>(lam, tl, base, pass.pos, M, pass.low);
+    tile_out<R, T, M>(phi, tp, base, pass.pos, pass.low);
+    tile_out<R, T, M>(lam, tl, base, pass.pos, pass.low);
     for (int k = threadIdx.x; k < pass.n_slots; k += T) {
-        double t = 0.;
+        double s = 0.;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) t += red[k][w];
-        partial[(u64)k * n_tiles + tile] = t;
+        for (int w = 0; w < NW; ++w) s += red[k][w];
+        partial[(u64)k * n_tiles + tile] = s;
     }
+}
+
+// ---- ops of a planned phase (host) -------------------------------------------------------------
+
+// Packed form of a phase layout (ops [begin, begin + n) of its pass).
+inline PhaseBits phase_bits(const PhasePlan &P, int begin, int n) {
+    PhaseBits h;
+    std::memset(&h, 0, sizeof(h));
+    for (int b = 0; b < (int)P.regs.size(); ++b) h.set(b, P.regs[b]);
+    for (int b = 0; b < (int)P.lanes.size(); ++b) h.set(5 + b, P.lanes[b]);
+    for (int b = 0; b < (int)P.waves.size(); ++b) h.set(11 + b, P.waves[b]);
+    h.op_begin = begin;
+    h.n_ops = n;
+    return h;
+}
+
+// Coefficients of a gate (kCoefs of them), as the ops read them.
+template <class R>
+void gate_coefs(const RegGate &g, R *c) {
+    for (int i = 0; i < kCoefs; ++i) c[i] = R(0);
+    if (g.kind == kGateY) {
+        rotation_coefs(c, g.m.m[0][0].real(), g.m.m[0][1].real());
+    } else if (g.kind == kGateX) {
+        rotation_coefs(c, g.m.m[0][0].real(), -g.m.m[0][1].imag());
+    } else if (g.kind == kGateDiag) {
+        const std::complex<double> r = g.m.m[1][1] / g.m.m[0][0];
+        c[0] = (R)g.m.m[0][0].real(); c[1] = (R)g.m.m[0][0].imag();
+        c[2] = (R)g.m.m[1][1].real(); c[3] = (R)g.m.m[1][1].imag();
+        c[4] = (R)r.real(); c[5] = (R)r.imag();
+    } else if (g.kind == kGateAny) {
+        double a[8];
+        gate_matrix_to_array(g.m, a);
+        for (int i = 0; i < 8; ++i) c[i] = (R)a[i];
+    }
+}
+
+template <class R>
+void append_flush(std::vector<RegOp<R>> &out, int group) {
+    RegOp<R> op;
+    std::memset(&op, 0, sizeof(op));
+    op.code = (unsigned)kArmFlush | (unsigned)group << 8;
+    op.slot = -1;
+    out.push_back(op);
+}
+
+// Appends the ops of gate g (index `row` in the coefficient table) in phase P. local: tile bit
+// of a state lane, -1 outside the tile. n_slots counts the gradient slots given out; have_u: the
+// sum of kArmU is that of the registers as they are.
+template <class R>
+void append_ops(std::vector<RegOp<R>> &out, const RegGate &g, int row, const PhasePlan &P, const int *local,
+                int &n_slots, bool &have_u) {
+    if (g.pauli != 0 && n_slots > 0 && n_slots % 16 == 0) append_flush(out, n_slots / 16 - 1);
+    const int rb = (int)P.regs.size();
+    auto position = [&](int bit) { return (int)(std::find(P.regs.begin(), P.regs.end(), bit) - P.regs.begin()); };
+    RegOp<R> op;
+    std::memset(&op, 0, sizeof(op));
+    op.row = row;
+    op.slot = -1;
+    int creg = 0;
+    for (int c : g.ctrl) {
+        if (local[c] < 0)
+            op.gctrl |= u64(1) << c;
+        else if (position(local[c]) < rb)
+            creg |= 1 << position(local[c]);
+        else
+            op.cthr |= 1u << local[c];
+    }
+    R c[kCoefs];
+    gate_coefs<R>(g, c);
+    auto push = [&](int arm, int tgt, int regs, int coff, int slot, const RegOp<R> &base) {
+        RegOp<R> o = base;
+        o.code = (unsigned)arm | (unsigned)tgt << 8 | (unsigned)regs << 16 |
+                 (unsigned)(slot >= 0 ? g.pauli : 0) << 24 | (unsigned)coff << 28;
+        o.slot = slot;
+        for (int i = 0; i < 4; ++i) o.c[i] = c[coff + i];
+        out.push_back(o);
+    };
+    const int lt = local[g.target];
+    const int tp = lt < 0 ? rb : position(lt);
+    if (g.kind != kGateDiag) {
+        QG_REQUIRE(tp < rb, "register phase: pair target is not a register bit");
+        const int fam = g.kind == kGateY ? kFamY : g.kind == kGateX ? kFamX : g.kind == kGateSwap ? kFamSwap : kFamAny;
+        QG_REQUIRE((fam != kFamY && fam != kFamX) || g.ctrl.empty(), "register phase: controlled rotation");
+        push(4 * fam + tp, 0, creg, 0, g.pauli != 0 ? n_slots++ : -1, op);
+        if (fam == kFamAny) push(kArmNone, 0, 0, 4, -1, op);   // m10, m11
+        have_u = false;
+        return;
+    }
+    const std::complex<double> d0 = g.m.m[0][0], d1 = g.m.m[1][1];
+    int slot = g.pauli != 0 ? n_slots++ : -1;
+    // factor on the amplitudes whose bits (masks of o, regs) are all set
+    auto factor = [&](RegOp<R> o, int regs, int coff, std::complex<double> f) {
+        const bool sign = f == -1. && g.pauli == 0;
+        const int n = __builtin_popcount((unsigned)regs);
+        if (n == 0) {
+            push(sign ? kArmSign : kArmPhase, 0, 0, coff, -1, o);
+        } else if (n == 1) {
+            push(4 * (sign ? kFamSign : kFamFactor) + __builtin_ctz((unsigned)regs), 0, regs, coff, -1, o);
+        } else if (n == 2) {
+            int i = 0;
+            while (pair2_mask(i) != regs) ++i;
+            push((sign ? kArmSign2 : kArmPair2) + i, 0, regs, coff, -1, o);
+        } else {
+            push(kArmFactorAny, 0, regs, coff, -1, o);
+        }
+    };
+    const bool one0 = d0 == 1. && g.pauli == 0;   // m00 == 1 whatever the parameter
+    if (tp < rb || creg != 0 || one0) {
+        RegOp<R> t = op;   // the controls and the target
+        int treg = creg;
+        if (lt < 0)
+            t.gctrl |= u64(1) << g.target;
+        else if (tp < rb)
+            treg |= 1 << tp;
+        else
+            t.cthr |= 1u << lt;
+        if (slot >= 0) {
+            if (creg == 0 && tp < rb)
+                push(4 * kFamZ + tp, 0, 0, 0, slot, op);
+            else   // target: register position, or RB + local bit, or 0x80 | RB + state bit
+                push(kArmZAny, tp < rb ? tp : lt >= 0 ? rb + lt : 0x80 | (rb + g.target), creg, 0, slot, op);
+        }
+        if (!one0) factor(op, creg, 0, d0);
+        factor(t, treg, one0 ? 2 : 4, one0 ? d1 : d1 / d0);
+        return;
+    }
+    if (slot >= 0 && !have_u) {
+        RegOp<R> u;
+        std::memset(&u, 0, sizeof(u));
+        push(kArmU, 0, 0, 0, -1, u);
+        have_u = true;
+    }
+    push(lt < 0 ? kArmOuter : op.cthr != 0 ? kArmThreadCtrl : kArmThread, lt >= 0 ? lt : g.target, 0, 0, slot, op);
+}
+
+// A planned register pass: phases (op_begin from 0) and ops.
+template <class R>
+struct BuiltPass {
+    std::vector<int> bits;
+    int low = 0;
+    std::vector<PhaseBits> phases;
+    std::vector<RegOp<R>> ops;
+    std::vector<int> slot_gate;    // gate of each gradient slot
+    std::vector<int> gates;        // gates of the pass
+};
+
+// Passes over a gate list: tiles of m of n lanes that hold the lowest `low`, rb register and wb
+// wave bits, at most max_gates gates, max_ops ops and max_phases phases a pass. Gates whose tile has no bit left
+// for them (tile bits == low bits) are refused by the caller's choice of m > low.
+template <class R>
+std::vector<BuiltPass<R>> build_passes(const std::vector<RegGate> &gates, int n, int m, int low, int rb, int wb,
+                                       int max_gates, int max_ops, int max_phases) {
+    QG_REQUIRE(low < m && m <= n, "register pass: %d tile bits, %d low, %d lanes", m, low, n);
+    const int ng = (int)gates.size();
+    std::vector<PlanGate> pg(ng);
+    for (int i = 0; i < ng; ++i)
+        pg[i] = PlanGate{gates[i].target, &gates[i].ctrl, gates[i].kind == kGateDiag,
+                         gates[i].kind == kGateAny ? 2 : 1, gates[i].pauli != 0 ? 1 : 0};
+    std::vector<char> done(ng, 0);
+    std::vector<BuiltPass<R>> out;
+    for (int first = 0; first < ng;) {
+        // a diagonal gate on a register bit can take two ops (three with a gradient): a pass
+        // that comes out too long is planned again with fewer gates
+        for (int limit = std::min(max_gates, max_ops);; limit = limit * 3 / 4) {
+            std::vector<char> now(done);
+            const PassBits pb = next_pass(pg, now, first, n, m, low, limit, kMaxSweepSlots);
+            QG_REQUIRE(!pb.gates.empty(), "register pass takes no gate");
+            int local[64];
+            for (int b = 0; b < 64; ++b) local[b] = -1;
+            for (int j = 0; j < m; ++j) local[pb.bits[j]] = j;
+            BuiltPass<R> bp;
+            bp.bits = pb.bits;
+            bp.low = pb.low;
+            bp.gates = pb.gates;
+            int slots = 0;
+            for (const PhasePlan &P : plan_phases(pg, pb.gates, local, n, m, rb, wb)) {
+                const int begin = (int)bp.ops.size();
+                bool have_u = false;
+                for (int gi : P.order) {
+                    append_ops<R>(bp.ops, gates[gi], gi, P, local, slots, have_u);
+                    if (gates[gi].pauli != 0) bp.slot_gate.push_back(gi);
+                }
+                bp.phases.push_back(phase_bits(P, begin, (int)bp.ops.size() - begin));
+            }
+            if (slots > 0) {   // the last slots
+                append_flush(bp.ops, (slots - 1) / 16);
+                bp.phases.back().n_ops += 1;
+            }
+            if ((int)bp.ops.size() > max_ops || (int)bp.phases.size() > max_phases) {
+                QG_REQUIRE(limit > 2, "register pass: a gate takes too many ops");
+                continue;
+            }
+            done.swap(now);
+            out.push_back(bp);
+            break;
+        }
+        while (first < ng && done[first]) ++first;
+    }
+    return out;
+}
+
+inline void set_positions(signed char *pos, const std::vector<int> &bits) {
+    for (int j = 0; j < kTilePosMax; ++j) pos[j] = j < (int)bits.size() ? (signed char)bits[j] : (signed char)0;
+}
+
+template <class R>
+RegProgram<R> reg_program(const BuiltPass<R> &bp) {
+    RegProgram<R> rp;
+    std::memset(&rp, 0, sizeof(rp));
+    rp.n_ops = (int)bp.ops.size();
+    rp.n_phases = (int)bp.phases.size();
+    rp.low = bp.low;
+    set_positions(rp.pos, bp.bits);
+    std::copy(bp.phases.begin(), bp.phases.end(), rp.phases);
+    std::copy(bp.ops.begin(), bp.ops.end(), rp.ops);
+    return rp;
 }
 
 }  // namespace
