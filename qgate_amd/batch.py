@@ -8,7 +8,8 @@ of uneven qubit counts in one replayed HIP graph (csrc/k_batch.hip).
 
 Circuits built from the same ParametricCircuit object with observables of the same terms
 share a group: their state vectors are stacked into one array and every tile-pass kernel
-covers the whole group. The first run times the tile shape (register-resident or LDS passes,
+covers the whole group; circuits that fit one workgroup (13 qubits in complex64, 12 in complex128)
+run there from |0...0> to the gradient, a workgroup each. The first run times the tile shape (register-resident or LDS passes,
 tile size) and the LDS passes' workgroup and grid size per group and keeps the fastest
 (`tuning` shows the choice), then captures the launch sequence of all groups into a graph
 that later runs replay.

@@ -13,7 +13,7 @@ CSRC = os.path.join(HERE, 'csrc')
 LIBDIR = os.path.join(HERE, 'lib')
 LIBNAME = 'libqgate_hip.so'
 SOURCES = ['qg_runtime.hip', 'gate_matrix.hip', 'k_gates.hip', 'k_state.hip', 'k_getter.hip',
-           'capi.hip', 'adjoint.hip', 'k_tile.hip', 'k_batch.hip', 'k_marginal.hip']
+           'capi.hip', 'adjoint.hip', 'k_tile.hip', 'k_batch.hip', 'k_small.hip', 'k_marginal.hip']
 ARCH = os.environ.get('QGATE_HIP_ARCH', 'gfx950')
 
 # -packed-fp32-ops: no v_pk_*_f32 instructions are generated.
@@ -22,7 +22,7 @@ HIPFLAGS = ['-std=c++17', '-O3', '-fPIC', '--offload-arch=' + ARCH, '-munsafe-fp
             '-Wall', '-Wno-unused-function', '-Wno-unused-command-line-argument']
 # Register tile passes (csrc/tile_reg.hpp) dispatch their ops by uniform branches. Structurized
 # like divergent ones, every arm of the dispatch copied the whole register array.
-EXTRA_FLAGS = {src: ['-mllvm', '-structurizecfg-skip-uniform-regions=true'] for src in ('k_tile.hip', 'k_batch.hip')}
+EXTRA_FLAGS = {src: ['-mllvm', '-structurizecfg-skip-uniform-regions=true'] for src in ('k_tile.hip', 'k_batch.hip', 'k_small.hip')}
 
 
 def lib_path():

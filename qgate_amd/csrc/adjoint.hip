@@ -24,6 +24,7 @@
 #include "gate_matrix.hpp"
 #include "kernels.hpp"
 #include "qg_runtime.hpp"
+#include "small.hpp"
 
 using namespace qg;
 
@@ -252,22 +253,22 @@ double forward_impl(qghip_circuit *c, const double *params, const Observable &ob
     ensure_states(c);
     Cx<R> *psi = static_cast<Cx<R> *>(c->psi), *lam = static_cast<Cx<R> *>(c->lam);
     hipStream_t s = stream();
-    launch_set_zero_state<R>(psi, c->n_qubits);
     if (c->fusion == QGHIP_FUSION_TILE) {
         std::vector<QueuedGate> gates;
         gates.reserve(c->ops.size());
         for (const Op &op : c->ops) gates.push_back(QueuedGate{op_matrix(op, params), op.ctrl, op.target});
-        apply_gate_sequence<R>(psi, c->n_qubits, gates, 0, -1);
-    } else {
-        for (const Op &op : c->ops) launch_gate<R>(psi, c->n_qubits, op_matrix(op, params), op.ctrl, op.target);
-    }
-    if (c->fusion == QGHIP_FUSION_TILE) {
         std::vector<PauliGroup> groups;
         std::vector<PauliTerm> terms;
         for (const GroupDev &g : obs.groups) groups.push_back(PauliGroup{g.xmask, g.first, g.count, 0u});
         for (const TermDev &t : obs.terms) terms.push_back(PauliTerm{t.cre, t.cim, t.zmask});
+        if (fits_workgroup<R>(c->n_qubits, groups))
+            return small_expectation<R>(psi, lam, c->n_qubits, gates, groups, terms);
+        launch_set_zero_state<R>(psi, c->n_qubits);
+        apply_gate_sequence<R>(psi, c->n_qubits, gates, 0, -1);
         return pauli_expectation<R>(psi, lam, c->n_qubits, groups, terms);
     }
+    launch_set_zero_state<R>(psi, c->n_qubits);
+    for (const Op &op : c->ops) launch_gate<R>(psi, c->n_qubits, op_matrix(op, params), op.ctrl, op.target);
     const u64 n = u64(1) << c->n_qubits;
     const size_t obs_bytes = sizeof(GroupDev) * obs.groups.size() + sizeof(TermDev) * obs.terms.size();
     char *d_obs = static_cast<char *>(dev_alloc(obs_bytes + 16));
@@ -301,6 +302,24 @@ double forward_impl(qghip_circuit *c, const double *params, const Observable &ob
 }
 
 template <class R>
+void sweep_terms(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<SweepGate> &gates,
+                 std::vector<double> &terms) {
+    const size_t bytes = sizeof(double) * terms.size();
+    double *d_terms = static_cast<double *>(dev_alloc(bytes));
+    hipError_t e = hipSuccess;
+    try {
+        adjoint_sweep<R>(phi, lam, n_lanes, gates, d_terms, 0, -1);
+        e = hipMemcpyAsync(terms.data(), d_terms, bytes, hipMemcpyDeviceToHost, stream());
+        if (e == hipSuccess) e = hipStreamSynchronize(stream());
+    } catch (...) {
+        dev_free(d_terms, bytes);
+        throw;
+    }
+    dev_free(d_terms, bytes);
+    QG_HIP(e);
+}
+
+template <class R>
 void backward_tiles(qghip_circuit *c, const double *params, double *grad) {
     Cx<R> *phi = static_cast<Cx<R> *>(c->psi), *lam = static_cast<Cx<R> *>(c->lam);
     const int n_ops = (int)c->ops.size();
@@ -310,20 +329,11 @@ void backward_tiles(qghip_circuit *c, const double *params, double *grad) {
         const Op &op = c->ops[k];
         gates.push_back(SweepGate{dagger(op_matrix(op, params)), op.kind == 1 ? op.pauli : 0, op.ctrl, op.target});
     }
-    const size_t bytes = sizeof(double) * (size_t)std::max(1, n_ops);
-    double *d_terms = static_cast<double *>(dev_alloc(bytes));
     std::vector<double> terms(std::max(1, n_ops));
-    hipError_t e = hipSuccess;
-    try {
-        adjoint_sweep<R>(phi, lam, c->n_qubits, gates, d_terms, 0, -1);
-        e = hipMemcpyAsync(terms.data(), d_terms, bytes, hipMemcpyDeviceToHost, stream());
-        if (e == hipSuccess) e = hipStreamSynchronize(stream());
-    } catch (...) {
-        dev_free(d_terms, bytes);
-        throw;
-    }
-    dev_free(d_terms, bytes);
-    QG_HIP(e);
+    if (fits_workgroup<R>(c->n_qubits) && n_ops <= small_max_gates())
+        small_sweep<R>(phi, lam, c->n_qubits, gates, terms.data());
+    else
+        sweep_terms<R>(phi, lam, c->n_qubits, gates, terms);
     for (int i = 0; i < c->n_params; ++i) grad[i] = 0.;
     for (int i = 0; i < n_ops; ++i) {   // sweep order: last gate first
         const Op &op = c->ops[n_ops - 1 - i];

@@ -6,7 +6,8 @@
 // (i << n) | x: the group is one state vector of n + log2(items) bits whose top bits select
 // the circuit. Tiles never take those top bits, so every tile belongs to one circuit, and
 // the per-circuit gate matrices (computed on the device from each circuit's parameters) and
-// observable coefficients are picked by the tile's item index. A group then runs as:
+// observable coefficients are picked by the tile's item index. Groups whose circuits fit one
+// workgroup run there whole (k_small.hip). Any other group runs as:
 //   k_batch_mats     U and U^dagger of every (item, gate), from the parameters (FP64 sincos)
 //   k_batch_zero     |0...0> in every item
 //   k_batch_pass     forward tile passes (gates applied in LDS, many per pass)
@@ -29,8 +30,10 @@
 
 #include "../../include/qgate_hip.h"
 #include "circuit.hpp"
+#include "circuit_rows.hpp"
 #include "kernels.hpp"
 #include "qg_runtime.hpp"
+#include "small.hpp"
 #include "tile_common.hpp"
 #include "tile_pauli.hpp"
 #include "tile_reg.hpp"
@@ -48,15 +51,6 @@ struct BGate {          // one gate of a group's structure
 template <class R>
 struct BMats {
     Mat2<R> fwd, bwd;
-};
-
-template <class R>
-struct BRow {           // one row of a register-pass coefficient table (kCoefs numbers per item)
-    R c[8];             // fixed gates: the coefficients
-    int kind;           // RegGate kind
-    int pauli;          // rotations: 1 X, 2 Y, 3 Z; 0: fixed
-    int param;
-    int back;           // the inverse (sweep)
 };
 
 struct BOp {            // a gate inside a pass
@@ -116,37 +110,14 @@ __global__ __launch_bounds__(256) void k_batch_mats(const BGate *__restrict__ ga
     mats[i] = out;
 }
 
-// Coefficients of the register passes' rows for every item, in FP64 and rounded once.
+// The coefficient rows of every item.
 template <class R>
-__global__ __launch_bounds__(256) void k_batch_coefs(const BRow<R> *__restrict__ rows, int n_rows,
-                                                     const double *__restrict__ params, int n_params, u64 n_items,
-                                                     R *__restrict__ coefs) {
+__global__ __launch_bounds__(256) void k_row_coefs(const BRow<R> *__restrict__ rows, int n_rows,
+                                                   const double *__restrict__ params, int n_params, u64 n_items,
+                                                   R *__restrict__ coefs) {
     const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
     if (i >= n_items * (u64)n_rows) return;
-    const u64 item = i / (u64)n_rows;
-    const BRow<R> row = rows[i % (u64)n_rows];
-    R c[kCoefs];
-    for (int k = 0; k < kCoefs; ++k) c[k] = row.c[k];
-    if (row.pauli != 0) {
-        const double th = params[item * (u64)n_params + (u64)row.param];
-        const double co = cos(0.5 * th), si = row.back ? -sin(0.5 * th) : sin(0.5 * th);
-        if (row.kind == kGateY) {          // m00 = co, m01 = -si
-            rotation_coefs(c, co, -si);
-        } else if (row.kind == kGateX) {   // m00 = co, m01 = -i si
-            rotation_coefs(c, co, si);
-        } else if (row.kind == kGateDiag) {   // co - i si, co + i si and their ratio
-            c[0] = (R)co;  c[1] = (R)-si;
-            c[2] = (R)co;  c[3] = (R)si;
-            c[4] = (R)(co * co - si * si);  c[5] = (R)(2. * co * si);
-        } else {                           // controlled RX, RY: the whole matrix
-            const double isx = row.pauli == 1 ? 1. : 0., isy = row.pauli == 2 ? 1. : 0.;
-            c[0] = (R)co;  c[1] = R(0);
-            c[2] = (R)(-si * isy);  c[3] = (R)(-si * isx);
-            c[4] = (R)(si * isy);   c[5] = (R)(-si * isx);
-            c[6] = (R)co;  c[7] = R(0);
-        }
-    }
-    for (int k = 0; k < kCoefs; ++k) coefs[i * kCoefs + k] = c[k];
+    row_coefs(rows[i % (u64)n_rows], params + i / (u64)n_rows * (u64)n_params, coefs + i * kCoefs);
 }
 
 // every item to |0...0>
@@ -614,6 +585,7 @@ struct Group {
     std::vector<SweepPass> rspasses;
     void *d_rsops = nullptr;                // RegOp<R>[]
     PhaseBits *d_rphases = nullptr;
+    int small = -1;                         // index in the batch's one-workgroup groups, -1: tile passes
     int n_frows = 0, n_srows = 0;           // rows of the coefficient tables
     void *d_frows = nullptr, *d_srows = nullptr;   // BRow<R>[]
     void *d_fcoefs = nullptr, *d_scoefs = nullptr;
@@ -626,6 +598,7 @@ struct qghip_batch {
     Prec prec;
     std::vector<std::pair<int, int>> items;   // (group, index in group)
     std::vector<Group> groups;
+    SmallBatch small;                         // the groups whose circuits each take one workgroup
     bool built = false;
     bool tuned = false;
     hipGraph_t graph = nullptr;
@@ -679,45 +652,6 @@ std::vector<RegProgram<float>> &reg_programs<float>(Group &g) {
 template <>
 std::vector<RegProgram<double>> &reg_programs<double>(Group &g) {
     return g.rprog64;
-}
-
-// The register gates of a group's structure, forward or (back) inverted in sweep order, and the
-// row of each in the coefficient table. Rotations keep their form at every angle; fixed gates
-// are split as in the single-circuit passes. RegGate::source is the gate of the structure.
-template <class R>
-std::vector<RegGate> group_gates(const std::vector<CircuitOp> &ops, bool back, std::vector<BRow<R>> &rows) {
-    std::vector<RegGate> out;
-    const int n = (int)ops.size();
-    for (int k = 0; k < n; ++k) {
-        const int i = back ? n - 1 - k : k;
-        const CircuitOp &op = ops[i];
-        if (op.kind == 0) {
-            append_fixed(out, back ? dagger(op.mat) : op.mat, op.ctrl, op.target, i);
-            continue;
-        }
-        RegGate g;
-        g.kind = op.pauli == 3 ? kGateDiag : !op.ctrl.empty() ? kGateAny : op.pauli == 1 ? kGateX : kGateY;
-        g.target = op.target;
-        g.pauli = back ? op.pauli : 0;
-        g.source = i;
-        g.ctrl = op.ctrl;
-        g.m = rotation(op.pauli, back ? -1. : 1.);   // its form; the angle is each item's own
-        out.push_back(g);
-    }
-    rows.clear();
-    for (const RegGate &g : out) {
-        BRow<R> r;
-        std::memset(&r, 0, sizeof(r));
-        gate_coefs<R>(g, r.c);
-        r.kind = g.kind;
-        if (ops[g.source].kind == 1) {
-            r.pauli = ops[g.source].pauli;
-            r.param = ops[g.source].param;
-        }
-        r.back = back ? 1 : 0;
-        rows.push_back(r);
-    }
-    return out;
 }
 
 // Plans and device tables of a group for a tuning (allocates; not during capture).
@@ -783,7 +717,7 @@ void build_group(Group &g, const Tuning &t) {
     }
     std::vector<BRow<R>> frows, srows;
     if (fregs)
-        for (const BuiltPass<R> &bp : build_passes<R>(group_gates<R>(g.ops, false, frows), n, TC::MaxBits, lowf,
+        for (const BuiltPass<R> &bp : build_passes<R>(row_gates<R>(g.ops, false, frows), n, TC::MaxBits, lowf,
                                                       Log2<kFA>::v, kWB, TC::MaxOps, TC::MaxRegOps, kMaxPhases))
             progs.push_back(reg_program(bp));
     // sweep passes: the gates in reverse order
@@ -832,7 +766,7 @@ void build_group(Group &g, const Tuning &t) {
         g.spasses.push_back(p);
     }
     if (sregs) {
-        const std::vector<RegGate> gates = group_gates<R>(g.ops, true, srows);
+        const std::vector<RegGate> gates = row_gates<R>(g.ops, true, srows);
         slot_out.clear();
         g.spass_slot_begin.clear();
         max_slots = 1;
@@ -885,7 +819,7 @@ void build_group(Group &g, const Tuning &t) {
         for (size_t k = 0; k < pl.size(); ++k) {
             const int begin = (int)pworks.size();
             plan_pauli_pass<R>(pgroups, pl[k].begin, pl[k].end - pl[k].begin, g.zmask, [&](int t) { return ny[t]; },
-                               pl[k].bits, pworks, pzs);
+                               pl[k].bits, kPauliThreads<R>, pworks, pzs);
             g.ppasses[k].op_begin = begin;
         }
     }
@@ -1032,11 +966,11 @@ void launch_group_t(Group &g) {
                            g.n_params, ni, mats);
     R *fcoefs = static_cast<R *>(g.d_fcoefs), *scoefs = static_cast<R *>(g.d_scoefs);
     if (g.n_frows > 0)
-        hipLaunchKernelGGL((k_batch_coefs<R>), (unsigned)((ni * (u64)g.n_frows + 255) / 256), 256, 0, s,
+        hipLaunchKernelGGL((k_row_coefs<R>), (unsigned)((ni * (u64)g.n_frows + 255) / 256), 256, 0, s,
                            static_cast<const BRow<R> *>(g.d_frows),
                            g.n_frows, g.d_params, g.n_params, ni, fcoefs);
     if (g.n_srows > 0)
-        hipLaunchKernelGGL((k_batch_coefs<R>), (unsigned)((ni * (u64)g.n_srows + 255) / 256), 256, 0, s,
+        hipLaunchKernelGGL((k_row_coefs<R>), (unsigned)((ni * (u64)g.n_srows + 255) / 256), 256, 0, s,
                            static_cast<const BRow<R> *>(g.d_srows),
                            g.n_srows, g.d_params, g.n_params, ni, scoefs);
     const u64 n_units = (ni << n) / W;
@@ -1212,23 +1146,52 @@ void tune_group(qghip_batch *b, Group &g) {
     g.tune = best;
 }
 
+// Groups whose circuits fit a workgroup take one each (k_small.hip) unless a knob of the tile
+// passes is fixed. The line is where a circuit stops fitting: below it the tile passes were slower for
+// few items and for many (13 lanes in complex64, 6 layers: 16 items 428 us against 370, 512 items 2.41 ms
+// against 2.28; 9 lanes, 512 items 1.90 ms against 1.71).
+template <class R>
+bool one_workgroup(const qghip_batch *b, const Group &g) {
+    return b->fixed_registers < 0 && b->fixed_tile_bits == 0 && b->fixed_threads == 0 && b->fixed_grid == 0 &&
+           fits_workgroup<R>(g.n, g.pgroups);
+}
+
+template <class R>
+void launch_all(qghip_batch *b) {
+    if (!b->small.empty()) b->small.launch<R>(stream());
+    for (Group &g : b->groups)
+        if (g.small < 0) launch_group<R>(g);
+}
+
 template <class R>
 void prepare(qghip_batch *b) {
     if (b->built) return;
     drop_graph(b);
+    b->small.clear();
+    std::vector<SmallGroupIn> small;
     for (Group &g : b->groups) {
-        if (!b->tuned || g.tune.tile_bits == 0)   // new settings, or a group added since tuning
+        if (one_workgroup<R>(b, g)) {
+            g.small = (int)small.size();
+            free_group(g);
+            g.tune = Tuning();
+            small.push_back(SmallGroupIn{g.n, g.n_params, (int)g.n_items(), &g.ops, &g.pgroups, &g.xmask, &g.zmask,
+                                         &g.coefs});
+            continue;
+        }
+        if (!b->tuned || g.small >= 0 || g.tune.tile_bits == 0)   // new settings, or a group added since tuning
             tune_group<R>(b, g);
         else
             build_group<R>(g, g.tune);
+        g.small = -1;
     }
+    b->small.build<R>(small);
     b->tuned = true;
     // capture every group's launch sequence into one graph
     hipStream_t s = stream();
     QG_HIP(hipStreamSynchronize(s));
     QG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
     try {
-        for (Group &g : b->groups) launch_group<R>(g);
+        launch_all<R>(b);
     } catch (...) {
         hipGraph_t tmp = nullptr;
         hipStreamEndCapture(s, &tmp);
@@ -1380,38 +1343,43 @@ int qghip_batch_run(qghip_batch *b, int use_graph, double *values, double *grads
         else
             prepare<double>(b);
         hipStream_t s = stream();
-        for (Group &g : b->groups) upload_params(g);
-        if (use_graph) {
-            QG_HIP(hipGraphLaunch(b->exec, s));
-        } else {
-            for (Group &g : b->groups) {
-                if (b->prec == precFP32)
-                    launch_group<float>(g);
-                else
-                    launch_group<double>(g);
-            }
+        std::vector<const std::vector<double> *> small_params;
+        for (Group &g : b->groups) {
+            if (g.small >= 0)
+                small_params.push_back(&g.params);
+            else
+                upload_params(g);
         }
+        if (!b->small.empty()) b->small.upload(small_params);
+        if (use_graph)
+            QG_HIP(hipGraphLaunch(b->exec, s));
+        else if (b->prec == precFP32)
+            launch_all<float>(b);
+        else
+            launch_all<double>(b);
         // results, item by item in batch order
         std::vector<std::vector<double>> gv(b->groups.size()), gg(b->groups.size());
         for (size_t k = 0; k < b->groups.size(); ++k) {
             Group &g = b->groups[k];
+            if (g.small >= 0) continue;
             gv[k].resize(g.n_items());
             gg[k].resize(g.n_items() * (size_t)g.n_params);
             QG_HIP(hipMemcpyAsync(gv[k].data(), g.d_values, sizeof(double) * gv[k].size(), hipMemcpyDeviceToHost, s));
             if (!gg[k].empty())
                 QG_HIP(hipMemcpyAsync(gg[k].data(), g.d_grads, sizeof(double) * gg[k].size(), hipMemcpyDeviceToHost, s));
         }
+        if (!b->small.empty()) b->small.download();
         QG_HIP(hipStreamSynchronize(s));
+        table_buffer_done();
         // grads are laid out per item in batch order, each item with its circuit's n_params entries
         int64_t off = 0;
         for (size_t i = 0; i < b->items.size(); ++i) {
             const int gi = b->items[i].first, k = b->items[i].second;
             const Group &g = b->groups[gi];
-            values[i] = gv[gi][k];
-            if (grads) {
-                std::copy(gg[gi].begin() + (size_t)k * g.n_params, gg[gi].begin() + (size_t)(k + 1) * g.n_params,
-                          grads + off);
-            }
+            const double *v = g.small >= 0 ? b->small.values(g.small) : gv[gi].data();
+            const double *gr = g.small >= 0 ? b->small.grads(g.small) : gg[gi].data();
+            values[i] = v[k];
+            if (grads) std::copy(gr + (size_t)k * g.n_params, gr + (size_t)(k + 1) * g.n_params, grads + off);
             off += g.n_params;
         }
     });
@@ -1424,15 +1392,23 @@ int qghip_batch_describe(const qghip_batch *b, char *buf, int size) {
         for (size_t k = 0; k < b->groups.size(); ++k) {
             const Group &g = b->groups[k];
             char line[512];
+            const bool f32 = b->prec == precFP32, sm = g.small >= 0;
+            const int sb = !sm ? 0 : f32 ? small_bits<float>(g.n) : small_bits<double>(g.n);
             snprintf(line, sizeof(line),
                      "%s{\"qubits\": %d, \"items\": %zu, \"gates\": %zu, \"tile_bits\": %d, \"threads\": %d, "
                      "\"grid_per_cu\": %d, \"registers\": %d, \"forward_in_registers\": %d, "
                      "\"sweep_in_registers\": %d, \"tuned_ms\": %.4f, \"forward_passes\": %zu, "
                      "\"sweep_passes\": %zu}",
-                     k ? ", " : "", g.n, g.n_items(), g.ops.size(), g.tune.tile_bits, g.tune.threads,
-                     g.tune.grid_per_cu, g.tune.registers, g.fregs ? 1 : 0, g.sregs ? 1 : 0, g.tune.ms,
-                     !g.fregs ? g.fpasses.size() : b->prec == precFP32 ? g.rprog32.size() : g.rprog64.size(),
-                     g.sregs ? g.rspasses.size() : g.spasses.size());
+                     k ? ", " : "", g.n, g.n_items(), g.ops.size(), sm ? sb : g.tune.tile_bits,
+                     sm ? (1 << sb) / kPauliPatterns : g.tune.threads, sm ? 1 : g.tune.grid_per_cu,
+                     sm ? 1 : g.tune.registers, sm || g.fregs ? 1 : 0, sm || g.sregs ? 1 : 0, g.tune.ms,
+                     sm         ? (size_t)1
+                     : !g.fregs ? g.fpasses.size()
+                     : f32      ? g.rprog32.size()
+                                : g.rprog64.size(),
+                     sm        ? (size_t)b->small.sweep_passes(g.small)
+                     : g.sregs ? g.rspasses.size()
+                               : g.spasses.size());
             out += line;
         }
         out += "]";

@@ -20,6 +20,7 @@
 
 #include "kernels.hpp"
 #include "qg_runtime.hpp"
+#include "table_layout.hpp"
 #include "tile_common.hpp"
 #include "tile_pauli.hpp"
 #include "tile_reg.hpp"
@@ -609,29 +610,6 @@ void apply_gate_sequence(Cx<R> *a, int n_lanes, const std::vector<QueuedGate> &g
 template void apply_gate_sequence<float>(Cx<float> *, int, const std::vector<QueuedGate> &, int, int);
 template void apply_gate_sequence<double>(Cx<double> *, int, const std::vector<QueuedGate> &, int, int);
 
-// The register gates of the gate list of a sweep: rotations whole (their gradient terms are
-// taken right before them), fixed gates split as in the forward pass.
-static std::vector<RegGate> sweep_gates(const std::vector<SweepGate> &gates) {
-    std::vector<RegGate> out;
-    out.reserve(gates.size() + gates.size() / 4);
-    for (int i = 0; i < (int)gates.size(); ++i) {
-        const SweepGate &g = gates[i];
-        if (g.pauli == 0) {
-            append_fixed(out, g.udag, g.ctrl, g.target, i);
-            continue;
-        }
-        RegGate r;
-        r.kind = g.pauli == 3 ? kGateDiag : !g.ctrl.empty() ? kGateAny : g.pauli == 1 ? kGateX : kGateY;
-        r.target = g.target;
-        r.pauli = g.pauli;
-        r.source = i;
-        r.ctrl = g.ctrl;
-        r.m = g.udag;
-        out.push_back(r);
-    }
-    return out;
-}
-
 // Gradient terms of consecutive passes: their partial rows (one per slot, one entry per tile)
 // accumulate in one device buffer, up to kSweepPartialBytes, and are summed by one launch when
 // it is full or the sweep ends, not by a small launch after each pass.
@@ -674,31 +652,6 @@ class SweepRows {
     int cap_ = 0, pending_ = 0, begin_ = 0;
     size_t o_part_ = 0, bytes_ = 0;
     char *buf_ = nullptr;
-};
-
-// Copies host tables one after another (each 256-byte aligned) to device memory.
-class TableLayout {
-  public:
-    template <class T>
-    size_t add(const std::vector<T> &v) {
-        const size_t at = (bytes_ + 255) & ~size_t(255);
-        bytes_ = at + sizeof(T) * v.size();
-        parts_.push_back(Part{at, sizeof(T) * v.size(), v.data()});
-        return at;
-    }
-    size_t bytes() const { return bytes_; }
-    void upload(char *dst) const {
-        for (const Part &p : parts_)
-            if (p.bytes > 0) QG_HIP(hipMemcpyAsync(dst + p.at, p.src, p.bytes, hipMemcpyHostToDevice, stream()));
-    }
-
-  private:
-    struct Part {
-        size_t at, bytes;
-        const void *src;
-    };
-    std::vector<Part> parts_;
-    size_t bytes_ = 0;
 };
 
 template <class R>
@@ -752,6 +705,7 @@ static void sweep_in_registers(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::v
     rows.sum(d_sg, d_terms);
     QG_HIP(hipGetLastError());
     QG_HIP(hipStreamSynchronize(s));   // the tables are host temporaries
+    table_buffer_done();
 }
 
 template <class R>
@@ -838,6 +792,7 @@ static void sweep_in_lds(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<
     rows.sum(d_sg, d_terms);
     QG_HIP(hipGetLastError());
     QG_HIP(hipStreamSynchronize(s));   // the tables are host temporaries
+    table_buffer_done();
 }
 
 template <class R>
@@ -959,7 +914,8 @@ double pauli_expectation(const Cx<R> *psi, Cx<R> *lam, int n_lanes, const std::v
         for (PauliPass &ps : passes) {
             const std::vector<int> bits(ps.pos, ps.pos + ps.m);
             const int begin = (int)works.size();
-            plan_pauli_pass<R>(groups, ps.g_begin, ps.n_groups, zmask, [&](int k) { return ny[k]; }, bits, works, zs);
+            plan_pauli_pass<R>(groups, ps.g_begin, ps.n_groups, zmask, [&](int k) { return ny[k]; }, bits,
+                               kPauliThreads<R>, works, zs);
             ps.g_begin = begin;
         }
     }
@@ -1002,6 +958,7 @@ double pauli_expectation(const Cx<R> *psi, Cx<R> *lam, int n_lanes, const std::v
     }
     dev_free(buf, bytes);
     QG_HIP(e);
+    table_buffer_done();
     return rt.h_pinned[0];
 }
 

@@ -156,6 +156,18 @@ void release_staging() {
     }
 }
 
+char *g_table = nullptr;
+bool g_table_busy = false;
+double *g_result = nullptr;
+
+void release_tables() {
+    if (g_table != nullptr) hipHostFree(g_table);
+    if (g_result != nullptr) hipHostFree(g_result);
+    g_table = nullptr;
+    g_result = nullptr;
+    g_table_busy = false;
+}
+
 // memcpy split over up to 8 host threads (first touch of fresh pages included)
 void parallel_memcpy(char *dst, const char *src, size_t bytes) {
     constexpr size_t kMinPerThread = size_t(4) << 20;
@@ -178,6 +190,25 @@ void parallel_memcpy(char *dst, const char *src, size_t bytes) {
 }
 
 }  // namespace
+
+char *table_buffer() {
+    hipStream_t s = stream();
+    if (g_table == nullptr)
+        QG_HIP(hipHostMalloc(reinterpret_cast<void **>(&g_table), kTableBytes, hipHostMallocDefault));
+    if (g_table_busy) QG_HIP(hipStreamSynchronize(s));
+    g_table_busy = true;
+    return g_table;
+}
+
+void table_buffer_done() { g_table_busy = false; }
+
+double *result_buffer() {
+    stream();
+    if (g_result == nullptr)
+        QG_HIP(hipHostMalloc(reinterpret_cast<void **>(&g_result), sizeof(double) * kResultDoubles,
+                             hipHostMallocDefault));
+    return g_result;
+}
 
 HostStager::HostStager() { staging(); }
 
@@ -230,6 +261,7 @@ void runtime_clear() {
     if (!rt.initialized) return;
     hipStreamSynchronize(rt.stream);
     release_staging();
+    release_tables();
     release_cache();
     hipFree(rt.d_partials);
     hipHostFree(rt.h_pinned);

@@ -89,6 +89,15 @@ class HostStager {
     int next_ = 0;
 };
 
+// Pinned host memory for one call's tables on their way up, and for results that kernels write
+// directly, each of one call at a time (under the runtime's lock; the call synchronises the stream
+// before it returns). table_buffer() waits for a copy that a failed call may have left behind.
+constexpr size_t kTableBytes = size_t(1) << 20;
+constexpr int kResultDoubles = 1 << 16;
+char *table_buffer();
+void table_buffer_done();   // its copy has completed
+double *result_buffer();
+
 // Copy `bytes` of device memory to pageable host memory through the stager; synchronises.
 void copy_to_host(void *dst, const void *src, size_t bytes);
 

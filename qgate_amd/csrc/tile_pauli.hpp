@@ -67,6 +67,50 @@ __device__ __forceinline__ void pauli_coefs(double (&c)[E], const int *begin, co
             }
 }
 
+// H psi of a thread's E amplitudes, added to (ar, ai). l0: local index of the first one (the others
+// differ from it by the constant bits at(e)); dt: its state index; psi(l, c): the tile's amplitude of
+// local index l ^ c, c constant.
+template <class R, int E, class At, class Psi>
+__device__ __forceinline__ void pauli_apply(double (&ar)[E], double (&ai)[E], unsigned l0, u64 dt, At at, Psi psi,
+                                            const PauliWork *__restrict__ works, int n_groups,
+                                            const PauliZ *__restrict__ zs, const double *__restrict__ coefs) {
+    for (int g = 0; g < n_groups; ++g) {
+        const PauliWork &w = works[g];
+        const unsigned lx = l0 ^ w.xlocal;
+        if (w.plain) {
+            double s = 0.;
+            for (int k = w.begin[0]; k < w.begin[1]; ++k) {
+                const PauliZ z = zs[k];
+                s = __builtin_fma((__popcll(dt & z.zmask) & 1) ? -1. : 1., coefs[z.coef], s);
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const Cx<R> v = psi(lx, at(e));
+                ar[e] = __builtin_fma(s, (double)v.re, ar[e]);
+                ai[e] = __builtin_fma(s, (double)v.im, ai[e]);
+            }
+            continue;
+        }
+        double c[E];
+        pauli_coefs<E>(c, w.begin, zs, coefs, dt);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const Cx<R> v = psi(lx, at(e));
+            ar[e] = __builtin_fma(c[e], (double)v.re, ar[e]);
+            ai[e] = __builtin_fma(c[e], (double)v.im, ai[e]);
+        }
+        if (w.imag) {
+            pauli_coefs<E>(c, w.ibegin, zs, coefs, dt);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const Cx<R> v = psi(lx, at(e));
+                ar[e] = __builtin_fma(-c[e], (double)v.im, ar[e]);
+                ai[e] = __builtin_fma(c[e], (double)v.re, ai[e]);
+            }
+        }
+    }
+}
+
 // One full-size tile (2^MB amplitudes, kPauliThreads<R> threads); returns the thread's part of
 // Re<psi|lambda> if `dot` is set. tp: the psi tile, in the order of its local index.
 template <class R, int MB>
@@ -96,41 +140,9 @@ __device__ __forceinline__ double pauli_full_tile(const Cx<R> *tp, Cx<R> *__rest
     }
     // local index of amplitude e: unit (e / W) T + tid, amplitude e % W of it
     const unsigned l0 = (unsigned)threadIdx.x << lw;
-    for (int g = 0; g < n_groups; ++g) {
-        const PauliWork &w = works[g];
-        const unsigned lx = l0 ^ w.xlocal;
-        if (w.plain) {
-            double s = 0.;
-            for (int k = w.begin[0]; k < w.begin[1]; ++k) {
-                const PauliZ z = zs[k];
-                s = __builtin_fma((__popcll(dt & z.zmask) & 1) ? -1. : 1., coefs[z.coef], s);
-            }
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const Cx<R> v = tp[lx ^ (((unsigned)(e / W * T) << lw) | (unsigned)(e % W))];
-                ar[e] = __builtin_fma(s, (double)v.re, ar[e]);
-                ai[e] = __builtin_fma(s, (double)v.im, ai[e]);
-            }
-            continue;
-        }
-        double c[E];
-        pauli_coefs<E>(c, w.begin, zs, coefs, dt);
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const Cx<R> v = tp[lx ^ (((unsigned)(e / W * T) << lw) | (unsigned)(e % W))];
-            ar[e] = __builtin_fma(c[e], (double)v.re, ar[e]);
-            ai[e] = __builtin_fma(c[e], (double)v.im, ai[e]);
-        }
-        if (w.imag) {
-            pauli_coefs<E>(c, w.ibegin, zs, coefs, dt);
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const Cx<R> v = tp[lx ^ (((unsigned)(e / W * T) << lw) | (unsigned)(e % W))];
-                ar[e] = __builtin_fma(-c[e], (double)v.im, ar[e]);
-                ai[e] = __builtin_fma(c[e], (double)v.re, ai[e]);
-            }
-        }
-    }
+    const auto at = [](int e) { return ((unsigned)(e / W * T) << lw) | (unsigned)(e % W); };
+    pauli_apply<R, E>(ar, ai, l0, dt, at, [&](unsigned l, unsigned c) { return tp[l ^ c]; }, works, n_groups, zs,
+                      coefs);
     double sum = 0.;
 #pragma unroll
     for (int q = 0; q < N; ++q) {
@@ -140,7 +152,7 @@ __device__ __forceinline__ double pauli_full_tile(const Cx<R> *tp, Cx<R> *__rest
             const int e = q * W + j;
             out.v[j] = cx<R>((R)ar[e], (R)ai[e]);
             if (dot) {
-                const Cx<R> v = tp[l0 | (((unsigned)(q * T) << lw) | (unsigned)j)];
+                const Cx<R> v = tp[l0 | at(e)];
                 sum += (double)v.re * (double)out.v[j].re + (double)v.im * (double)out.v[j].im;
             }
         }
@@ -149,18 +161,20 @@ __device__ __forceinline__ double pauli_full_tile(const Cx<R> *tp, Cx<R> *__rest
     return sum;
 }
 
-// The groups [first, first + n) of a pass on full-size tiles whose bits are `bits` (ascending):
-// their works and sorted terms. n_y(k): number of Y factors of term k.
+// The groups [first, first + n) of a pass on tiles whose bits are `bits` (ascending), in workgroups
+// of `threads` with kPauliPatterns amplitudes a thread: their works and sorted terms. n_y(k): number
+// of Y factors of term k.
 template <class R, class NY>
 void plan_pauli_pass(const std::vector<PauliGroup> &groups, int first, int n, const std::vector<u64> &zmask, NY n_y,
-                     const std::vector<int> &bits, std::vector<PauliWork> &works, std::vector<PauliZ> &zs) {
+                     const std::vector<int> &bits, int threads, std::vector<PauliWork> &works,
+                     std::vector<PauliZ> &zs) {
     constexpr int W = Unit<R>::W, lw = W == 2 ? 1 : 0;
     // state bits in which a thread's amplitudes differ: unit bits above the workgroup's, and (W ==
     // 2) the amplitude inside the unit
     std::vector<int> own;
     if (W == 2) own.push_back(bits[0]);
     int tb = 0;
-    while ((1 << tb) < kPauliThreads<R>) ++tb;
+    while ((1 << tb) < threads) ++tb;
     for (int j = lw + tb; j < (int)bits.size(); ++j) own.push_back(bits[j]);
     auto pattern = [&](u64 z) {
         int p = 0;

@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "gate_matrix.hpp"
+#include "kernels.hpp"
 #include "qg_runtime.hpp"
 #include "reg_plan.hpp"
 #include "tile_common.hpp"
@@ -1113,6 +1114,29 @@ void append_ops(std::vector<RegOp<R>> &out, const RegGate &g, int row, const Pha
         have_u = true;
     }
     push(lt < 0 ? kArmOuter : op.cthr != 0 ? kArmThreadCtrl : kArmThread, lt >= 0 ? lt : g.target, 0, 0, slot, op);
+}
+
+// The register gates of the gate list of a sweep: rotations whole (their gradient terms are
+// taken right before them), fixed gates split as in the forward pass.
+inline std::vector<RegGate> sweep_gates(const std::vector<SweepGate> &gates) {
+    std::vector<RegGate> out;
+    out.reserve(gates.size() + gates.size() / 4);
+    for (int i = 0; i < (int)gates.size(); ++i) {
+        const SweepGate &g = gates[i];
+        if (g.pauli == 0) {
+            append_fixed(out, g.udag, g.ctrl, g.target, i);
+            continue;
+        }
+        RegGate r;
+        r.kind = g.pauli == 3 ? kGateDiag : !g.ctrl.empty() ? kGateAny : g.pauli == 1 ? kGateX : kGateY;
+        r.target = g.target;
+        r.pauli = g.pauli;
+        r.source = i;
+        r.ctrl = g.ctrl;
+        r.m = g.udag;
+        out.push_back(r);
+    }
+    return out;
 }
 
 // A planned register pass: phases (op_begin from 0) and ops.
