@@ -38,7 +38,7 @@ __device__ __forceinline__ void row_coefs(const BRow<R> &row, const double *__re
         } else if (row.kind == kGateDiag) {   // co - i si, co + i si and their ratio
             c[0] = (R)co;  c[1] = (R)-si;
             c[2] = (R)co;  c[3] = (R)si;
-            c[4] = (R)(co * co - si * si);  c[5] = (R)(2. * co * si);
+            c[4] = (R)cos(th);  c[5] = (R)(row.back ? -sin(th) : sin(th));
         } else {                           // controlled RX, RY: the whole matrix
             const double isx = row.pauli == 1 ? 1. : 0., isy = row.pauli == 2 ? 1. : 0.;
             c[0] = (R)co;  c[1] = R(0);

@@ -380,13 +380,13 @@ template <>
 struct BCfg<float> {
     static constexpr int MaxBits = 12;       // forward / Pauli tiles: 32 KiB
     static constexpr int SweepBits = 11;     // sweep: two tiles, 32 KiB
-    static constexpr int Low = 5;
+    static constexpr int Low = 4;
 };
 template <>
 struct BCfg<double> {
     static constexpr int MaxBits = 11;
     static constexpr int SweepBits = 10;
-    static constexpr int Low = 4;
+    static constexpr int Low = 3;
 };
 // Register-resident passes (tile_reg.hpp): 256 threads, 2^12 / 2^11 amplitudes per forward tile
 // (16 / 8 per thread) and 2^11 / 2^10 per sweep tile (8 / 4 per thread and state), as in the
@@ -718,7 +718,7 @@ void build_group(Group &g, const Tuning &t) {
     std::vector<BRow<R>> frows, srows;
     if (fregs)
         for (const BuiltPass<R> &bp : build_passes<R>(row_gates<R>(g.ops, false, frows), n, TC::MaxBits, lowf,
-                                                      Log2<kFA>::v, kWB, TC::MaxOps, TC::MaxRegOps, kMaxPhases))
+                                                      Log2<kFA>::v, kWB, TC::MaxOps, TC::MaxRegOps, kMaxPhases, kNoGlobalPhase))
             progs.push_back(reg_program(bp));
     // sweep passes: the gates in reverse order
     std::vector<u64> sneed(n_gates), sdl(n_gates);
@@ -771,7 +771,8 @@ void build_group(Group &g, const Tuning &t) {
         g.spass_slot_begin.clear();
         max_slots = 1;
         for (const BuiltPass<R> &bp :
-             build_passes<R>(gates, n, C::SweepBits, lows, Log2<kSA>::v, kWB, 1 << 30, 1 << 30, 1 << 30)) {
+             build_passes<R>(gates, n, C::SweepBits, lows, Log2<kSA>::v, kWB, 1 << 30, 1 << 30, 1 << 30,
+                             kNoGlobalPhase)) {
             SweepPass rp;
             rp.low = bp.low;
             rp.op_begin = (int)rsops.size();

@@ -311,10 +311,10 @@ struct SmallTables {
 };
 
 template <class R>
-void plan_small(SmallTables<R> &t, const std::vector<RegGate> &gates, int m) {
+void plan_small(SmallTables<R> &t, const std::vector<RegGate> &gates, int m, GlobalPhases keep) {
     constexpr int RB = Log2<kSmallAmps>::v;
     for (const BuiltPass<R> &bp :
-         build_passes<R>(gates, m, m, TileCfg<R>::Low, RB, m - RB - 6, 1 << 30, 1 << 30, 1 << 30)) {
+         build_passes<R>(gates, m, m, TileCfg<R>::Low, RB, m - RB - 6, 1 << 30, 1 << 30, 1 << 30, keep)) {
         SmallPass ps;
         ps.op_begin = (int)t.ops.size();
         ps.phase_begin = (int)t.phases.size();
@@ -330,9 +330,9 @@ void plan_small(SmallTables<R> &t, const std::vector<RegGate> &gates, int m) {
 
 // The forward passes as one: phases whose ops count from the first one's.
 template <class R>
-void plan_small_forward(SmallTables<R> &t, const std::vector<RegGate> &gates, int m) {
+void plan_small_forward(SmallTables<R> &t, const std::vector<RegGate> &gates, int m, GlobalPhases keep) {
     const size_t pass0 = t.passes.size(), op0 = t.ops.size();
-    plan_small(t, gates, m);
+    plan_small(t, gates, m, keep);
     for (size_t p = pass0; p < t.passes.size(); ++p)
         for (int k = 0; k < t.passes[p].n_phases; ++k)
             t.phases[t.passes[p].phase_begin + k].op_begin += t.passes[p].op_begin - (int)op0;
@@ -401,7 +401,8 @@ double small_expectation(Cx<R> *psi, Cx<R> *lam, int n_lanes, const std::vector<
     const int m = small_bits<R>(n_lanes);
     SmallTables<R> t;
     plan_small_forward(
-        t, merged_gates((int)gates.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates[i]; }), m);
+        t, merged_gates((int)gates.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates[i]; }), m,
+        kGlobalPhase);
     t.ops.push_back(RegOp<R>());   // one more is read than there are
     std::vector<u64> xmask, zmask;
     std::vector<double> coefs;
@@ -456,7 +457,7 @@ void small_sweep(const Cx<R> *phi, const Cx<R> *lam, int n_lanes, const std::vec
     QG_REQUIRE((int)gates.size() <= small_max_gates(), "sweep in one workgroup: %d gates", (int)gates.size());
     for (size_t i = 0; i < gates.size(); ++i) out[i] = 0.;
     SmallTables<R> t;
-    plan_small(t, sweep_gates(gates), m);
+    plan_small(t, sweep_gates(gates), m, kNoGlobalPhase);
     if (t.passes.empty()) return;
     t.ops.push_back(RegOp<R>());   // one more is read than there are
     TableLayout tab;
@@ -524,10 +525,10 @@ void SmallBatch::build(const std::vector<SmallGroupIn> &in) {
         std::vector<BRow<R>> fr, sr;
         g.f_op = (int)t.ops.size();
         g.f_phase = (int)t.phases.size();
-        plan_small_forward(t, row_gates<R>(*gi.ops, false, fr), m);
+        plan_small_forward(t, row_gates<R>(*gi.ops, false, fr), m, kNoGlobalPhase);
         g.f_phases = (int)t.phases.size() - g.f_phase;
         g.pass = (int)t.passes.size();
-        plan_small(t, row_gates<R>(*gi.ops, true, sr), m);
+        plan_small(t, row_gates<R>(*gi.ops, true, sr), m, kNoGlobalPhase);
         g.n_passes = (int)t.passes.size() - g.pass;
         g.n_ops = (int)t.ops.size() - g.f_op;
         passes_.push_back(g.n_passes);

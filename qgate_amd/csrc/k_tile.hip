@@ -12,7 +12,8 @@
 //     predicate per tile, so they never use a tile bit.
 // Gates are applied in program order with the reference's pair update
 // (CPUQubitProcessor.cpp:307-362): a[i0] <- m00 a[i0] + m01 a[i1], a[i1] <- m10 a[i0] + m11 a[i1].
-// The gate list of a pass travels in the kernel arguments (at most 40 / 24 gates).
+// Full-size tiles take the register engine (tile_reg.hpp), the rest work in LDS. The gates of a pass
+// travel in the kernel arguments: at most 72 / 52 register ops, 40 / 24 gates of an LDS pass.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -430,22 +431,23 @@ __global__ __launch_bounds__((kPauliThreads<R>)) void k_tile_pauli_full(const Cx
 template <class R>
 struct SweepCfg;
 // Sweep tiles: register passes (RegBits, RegThreads) and LDS passes for smaller tiles or with
-// register tiles off (LdsBits), both holding a phi and a lambda tile. 12-bit complex64 tiles
-// (512 threads, 64 KiB of LDS) cut the 24-qubit ansatz's backward from 38 passes to 33 but
-// measured no faster: the sweep is bound by its per-gate instruction work, not by passes.
-// 128 threads on 11-bit tiles (16 amplitudes per state and thread, 203 VGPRs, two waves per
-// SIMD) made that backward slower, 7.4 -> 8.6 ms.
+// register tiles off (LdsBits), both holding a phi and a lambda tile. The sweep is bound by its
+// per-gate instruction work more than by passes: 12-bit complex64 tiles (512 threads, 64 KiB of LDS)
+// take the 24-qubit ansatz's backward in 14 passes instead of 15 and measured slower, 4.08 -> 4.23 ms;
+// 11-bit complex128 tiles (512 threads) take that of 19 qubits and 8 layers in 5 instead of 8 and
+// measured faster than 10-bit ones, 268 -> 253 us. One LDS tile for both states in turn and five
+// waves per SIMD instead of four gave nothing (242 -> 239 us a pass).
 template <>
 struct SweepCfg<float> {
     static constexpr int RegBits = 11, RegThreads = 256;   // 8 amplitudes per state and thread
     static constexpr int LdsBits = 11;                     // two 2^11 x 8 B tiles = 32 KiB
-    static constexpr int Low = 5;
+    static constexpr int Low = 4;
 };
 template <>
 struct SweepCfg<double> {
-    static constexpr int RegBits = 10, RegThreads = 256;   // 4 amplitudes per state and thread
+    static constexpr int RegBits = 11, RegThreads = 512;   // 4 amplitudes per state and thread
     static constexpr int LdsBits = 10;                     // two 2^10 x 16 B tiles = 32 KiB
-    static constexpr int Low = 4;
+    static constexpr int Low = 3;
 };
 
 }  // namespace
@@ -501,12 +503,10 @@ static void run_register_passes(Cx<R> *a, int n_lanes, const std::vector<QueuedG
     constexpr int A = (1 << M) / T;
     const std::vector<RegGate> gates =
         merged_gates((int)gates_in.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates_in[i]; });
-    const std::vector<BuiltPass<R>> passes = build_passes<R>(gates, n_lanes, M, low, Log2<A>::v, Log2<T / 64>::v,
-                                                             TileCfg<R>::MaxRegOps, TileCfg<R>::MaxRegOps, kMaxPhases);
     hipStream_t s = stream();
     const u64 n_tiles = u64(1) << (n_lanes - M);
     const u64 piece = launch_piece_items() / T;   // keeps every grid within launch_piece_items() threads
-    for (const BuiltPass<R> &bp : passes) {
+    const auto run = [&](const BuiltPass<R> &bp) {
         // a pass that comes to one gate streams faster than through a tile
         const RegGate &g0 = gates[bp.gates[0]];
         bool lone = bp.gates.size() == 1;
@@ -524,7 +524,7 @@ static void run_register_passes(Cx<R> *a, int n_lanes, const std::vector<QueuedG
         }
         if (lone) {
             launch_gate<R>(a, n_lanes, m, g0.ctrl, g0.target);
-            continue;
+            return;
         }
         const RegProgram<R> rp = reg_program(bp);
         for (u64 first = 0; first < n_tiles; first += piece) {
@@ -532,7 +532,9 @@ static void run_register_passes(Cx<R> *a, int n_lanes, const std::vector<QueuedG
             hipLaunchKernelGGL((k_tile_reg<R, M, T, false>), (unsigned)count, T, 0, s, a, rp, first,
                                (const R *)nullptr, 0, 0);
         }
-    }
+    };
+    for_each_pass<R>(gates, n_lanes, M, low, Log2<A>::v, Log2<T / 64>::v, TileCfg<R>::MaxRegOps,
+                     TileCfg<R>::MaxRegOps, kMaxPhases, kGlobalPhase, run);
     QG_HIP(hipGetLastError());
 }
 
@@ -662,7 +664,7 @@ static void sweep_in_registers(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::v
     const std::vector<RegGate> rg = sweep_gates(gates);
     const std::vector<BuiltPass<R>> passes = build_passes<R>(
         rg, n_lanes, C::RegBits, low, Log2<A>::v, Log2<C::RegThreads / 64>::v, 1 << 30, 1 << 30,
-        1 << 30);
+        1 << 30, kNoGlobalPhase);
     if (passes.empty()) return;
     std::vector<RegOp<R>> ops;
     std::vector<PhaseBits> phases;

@@ -66,11 +66,13 @@ inline bool split_unitary(const GateMatrix &u, std::complex<double> &a0, std::co
     const long double tol = 4e-15L;
     if (!(std::abs(std::norm(m00) + std::norm(m01) - 1.L) < tol &&
           std::abs(std::norm(m10) + std::norm(m11) - 1.L) < tol &&
-          std::abs(m00 * std::conj(m10) + m01 * std::conj(m11)) < tol))
+          std::norm(m00 * std::conj(m10) + m01 * std::conj(m11)) < tol * tol))
         return false;
-    const long double r0 = std::abs(m00), r1 = std::abs(m10), r = std::sqrt(r0 * r0 + r1 * r1);
-    auto phase = [](const cl &v) {
-        const long double n = std::abs(v);
+    // (moduli at most 1 and squared without harm: no std::abs, whose hypot guards against more)
+    auto modulus = [](const cl &v) { return std::sqrt(std::norm(v)); };
+    const long double r0 = modulus(m00), r1 = modulus(m10), r = std::sqrt(r0 * r0 + r1 * r1);
+    auto phase = [&](const cl &v) {
+        const long double n = modulus(v);
         return n > 0.L ? v / n : cl(1.L);
     };
     const cl p0 = phase(m00), p1 = phase(m10);
@@ -290,21 +292,23 @@ constexpr int kMaxScaled = 16;
 inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const std::vector<int> &gates,
                                           const int *local, int n, int m, int rb, int wb) {
     std::vector<PhasePlan> out;
+    std::vector<unsigned> regs;              // register bits of each phase
     std::vector<char> done(gates.size(), 0);
     size_t first = 0;
     while (first < gates.size()) {
         PhasePlan P;
+        unsigned in = 0;
         HeldLanes held(n);
-        int pairs = 0;
+        int pairs = 0, free_regs = rb;
         for (size_t k = first; k < gates.size(); ++k) {
             if (done[k]) continue;
             const PlanGate &q = g[gates[k]];
-            const int lt = local[q.target];
-            const bool known = !q.diag && std::find(P.regs.begin(), P.regs.end(), lt) != P.regs.end();
-            const bool fits = q.diag || (pairs < kMaxScaled && (known || (int)P.regs.size() < rb));
+            const unsigned bit = q.diag ? 0u : 1u << local[q.target];
+            const bool fits = q.diag || (pairs < kMaxScaled && ((in & bit) || free_regs > 0));
             if (fits && !held.conflicts(q)) {
                 if (!q.diag) {
-                    if (!known) P.regs.push_back(lt);
+                    if (!(in & bit)) --free_regs;
+                    in |= bit;
                     ++pairs;
                 }
                 P.order.push_back(gates[k]);
@@ -316,73 +320,71 @@ inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const 
         }
         while (first < gates.size() && done[first]) ++first;
         // pad with the highest free bits, so that the lane bits are the lowest ones
-        for (int b = m - 1; (int)P.regs.size() < rb && b >= 0; --b)
-            if (std::find(P.regs.begin(), P.regs.end(), b) == P.regs.end()) P.regs.push_back(b);
-        std::sort(P.regs.begin(), P.regs.end());
+        for (int b = m - 1; free_regs > 0 && b >= 0; --b)
+            if (!((in >> b) & 1)) in |= 1u << b, --free_regs;
         for (int b = 0; b < m; ++b)
-            if (std::find(P.regs.begin(), P.regs.end(), b) == P.regs.end())
-                ((int)P.lanes.size() < 6 ? P.lanes : P.waves).push_back(b);
+            ((in >> b) & 1 ? P.regs : (int)P.lanes.size() < 6 ? P.lanes : P.waves).push_back(b);
         if ((int)P.waves.size() != wb) raise_error("tile layout does not match the workgroup");
-        out.push_back(P);
+        regs.push_back(in);
+        out.push_back(std::move(P));
     }
-    // diagonal gates: position gp is before pair gate gp (np: after the last)
-    std::vector<int> pairs, phase_of, diags, seen_at;
+    // diagonal gates: position gp is before pair gate gp (np: after the last); lo and hi: right
+    // after the last pair gate on one of its lanes before it, right before the first one after it
+    struct Diag {
+        int gate, lo, hi, at, phase;
+    };
+    std::vector<int> pairs, phase_of;
+    std::vector<Diag> diags;
+    std::vector<int> seen(n, 0);   // position after the last pair gate on a lane
     for (size_t ph = 0; ph < out.size(); ++ph)
         for (int gi : out[ph].order) {
             if (g[gi].diag) {
-                diags.push_back(gi);
-                seen_at.push_back((int)pairs.size());
+                int lo = seen[g[gi].target];
+                for (int c : *g[gi].ctrl) lo = std::max(lo, seen[c]);
+                diags.push_back(Diag{gi, lo, (int)pairs.size(), 0, 0});
             } else {
                 pairs.push_back(gi);
                 phase_of.push_back((int)ph);
+                seen[g[gi].target] = (int)pairs.size();
             }
         }
-    const int np = (int)pairs.size();
+    const int np = (int)pairs.size(), n_ph = (int)out.size();
     if (np == 0 || diags.empty()) return out;
-    const int n_ph = (int)out.size();
+    std::fill(seen.begin(), seen.end(), np);   // position of the next pair gate on a lane
+    for (int d = (int)diags.size() - 1, k = np; d >= 0; --d) {
+        Diag &q = diags[d];
+        for (; k > q.hi; --k) seen[g[pairs[k - 1]].target] = k - 1;
+        q.hi = seen[g[q.gate].target];
+        for (int c : *g[q.gate].ctrl) q.hi = std::min(q.hi, seen[c]);
+    }
     std::vector<char> has_factor(n_ph, 0);
-    std::vector<std::vector<int>> at(np + 1);   // diagonal gates right before pair gate gp
-    std::vector<std::vector<int>> where(np + 1);   // and the phase each of them runs in
-    for (size_t d = 0; d < diags.size(); ++d) {
-        const PlanGate &q = g[diags[d]];
-        std::vector<int> lanes(*q.ctrl);
-        lanes.push_back(q.target);
-        auto hits = [&](int k) { return std::find(lanes.begin(), lanes.end(), g[pairs[k]].target) != lanes.end(); };
-        int lo = 0, hi = np;
-        for (int k = seen_at[d] - 1; k >= 0; --k)
-            if (hits(k)) {
-                lo = k + 1;
-                break;
-            }
-        for (int k = seen_at[d]; k < np; ++k)
-            if (hits(k)) {
-                hi = k;
-                break;
-            }
+    std::vector<int> count(np + 2, 0);
+    for (Diag &d : diags) {
+        const PlanGate &q = g[d.gate];
+        const auto bit = [&](int lane) { return local[lane] >= 0 ? 1u << local[lane] : 0u; };
+        unsigned mask = bit(q.target);
+        for (int c : *q.ctrl) mask |= bit(c);
         // phases it may run in: any from that of the pair gate before position lo to that of the
         // one after position hi
-        const int ph_lo = lo == 0 ? 0 : phase_of[lo - 1], ph_hi = hi == np ? n_ph - 1 : phase_of[hi];
+        const int ph_lo = d.lo == 0 ? 0 : phase_of[d.lo - 1], ph_hi = d.hi == np ? n_ph - 1 : phase_of[d.hi];
         auto cost = [&](int ph) {
-            int regs = 0;
-            for (int l : lanes)
-                if (local[l] >= 0 &&
-                    std::find(out[ph].regs.begin(), out[ph].regs.end(), local[l]) != out[ph].regs.end())
-                    ++regs;
-            return regs > 0 ? 4 - (regs > 1) : has_factor[ph] ? 0 : 1;
+            const unsigned on = mask & regs[ph];
+            return on != 0 ? 4 - ((on & (on - 1)) != 0) : has_factor[ph] ? 0 : 1;
         };
-        int best = -1;
-        for (int ph = ph_lo; ph <= ph_hi; ++ph)
-            if (best < 0 || cost(ph) < cost(best)) best = ph;
-        if (cost(best) <= 1) has_factor[best] = 1;
+        d.phase = ph_lo;
+        for (int ph = ph_lo + 1; ph <= ph_hi; ++ph)
+            if (cost(ph) < cost(d.phase)) d.phase = ph;
+        if (cost(d.phase) <= 1) has_factor[d.phase] = 1;
         // the last position within [lo, hi] that still belongs to that phase
-        int gp = lo;
-        while (gp < hi && phase_of[gp] <= best) ++gp;
-        at[gp].push_back(diags[d]);
-        where[gp].push_back(best);
+        d.at = (int)(std::upper_bound(phase_of.begin() + d.lo, phase_of.begin() + d.hi, d.phase) - phase_of.begin());
+        ++count[d.at + 1];
     }
+    for (int gp = 0; gp <= np; ++gp) count[gp + 1] += count[gp];
+    std::vector<int> by(diags.size()), next(count);   // diagonal gates by position
+    for (size_t d = 0; d < diags.size(); ++d) by[next[diags[d].at]++] = (int)d;
     for (PhasePlan &P : out) P.order.clear();
     for (int gp = 0; gp <= np; ++gp) {
-        for (size_t k = 0; k < at[gp].size(); ++k) out[where[gp][k]].order.push_back(at[gp][k]);
+        for (int k = count[gp]; k < count[gp + 1]; ++k) out[diags[by[k]].phase].order.push_back(diags[by[k]].gate);
         if (gp < np) out[phase_of[gp]].order.push_back(pairs[gp]);
     }
     return out;

@@ -22,11 +22,12 @@
 //   * Gradient terms are summed over the wavefront by FP64 matrix-core steps, sixteen slots to
 //     an accumulator tile: a conversion, two moves and one matrix instruction a term, where a
 //     DPP tree took about 20 vector instructions.
-// Together the 24-qubit ansatz's sweep issues 3109 vector instructions per wave and pass, against
-// 5834 before, and its passes take 243 us instead of 353; a forward pass over 30 qubits in
-// complex64 carries 29 gates in 5.36 ms, against 22 in 5.80 ms. Vector and scalar issue still
-// bound both (78% and 54% of the cycles of a sweep pass): a gate costs about 45 scalar
-// instructions to decode and dispatch beside its arithmetic.
+//   * A diagonal gate is its first entry, which without controls is a phase of the whole state (one
+//     factor per pass, none where only <H> and gradients are wanted), and a ratio.
+// Against passes without these steps, the backward sweep of the 24-qubit, 12-layer ansatz takes 15
+// passes of 272 us instead of 19 of 353, its forward part 15 of 106 us instead of 22 of 129, and 500
+// random gates on 30 qubits 16 of 5.5 ms instead of 20 of 5.8. Vector and scalar issue bound all of
+// them: a gate costs about 45 scalar instructions to decode and dispatch beside its arithmetic.
 #pragma once
 
 #include <algorithm>
@@ -45,6 +46,9 @@ namespace qg {
 
 namespace {
 
+// Low: the lowest bits that every tile holds, one 128-byte cache line. Each bit less frees one for a
+// gate's target: with 256-byte rows the 24-qubit ansatz took 19 sweep and 16 forward passes instead of
+// 15 and 15 (sweep 4.36 -> 4.08 ms, forward 1.63 -> 1.59), 500 gates on 30 qubits 17 instead of 16.
 template <class R>
 struct TileCfg;
 template <>
@@ -52,14 +56,14 @@ struct TileCfg<float> {
     static constexpr int MaxBits = 12;   // 2^12 x 8 B = 32 KiB of LDS
     static constexpr int MaxOps = 40;    // LDS passes
     static constexpr int MaxRegOps = 72; // register passes: 40 B each in the kernel arguments
-    static constexpr int Low = 5;        // 32 contiguous amplitudes = 256 B per row
+    static constexpr int Low = 4;        // 16 contiguous amplitudes = 128 B per row
 };
 template <>
 struct TileCfg<double> {
     static constexpr int MaxBits = 11;   // 2^11 x 16 B = 32 KiB
     static constexpr int MaxOps = 24;
     static constexpr int MaxRegOps = 52; // 56 B each
-    static constexpr int Low = 4;        // 16 x 16 B = 256 B per row
+    static constexpr int Low = 3;        // 8 x 16 B = 128 B per row
 };
 
 constexpr int kMaxPhases = 24;
@@ -83,16 +87,17 @@ struct PhaseBits {
 
 // Arms of an op. Families of updates on a register position P take codes 4 F + P: rotations
 // about Y and X in their two forms (t, k), controlled swaps, general 2x2, a factor or a sign on
-// the register indices with bit P set, and the gradient term of a Z generator on bit P.
+// the register indices with bit P set, and a Z rotation on bit P with its gradient term (the term,
+// then the factor on the indices with the bit set).
 // kArmPair2 + i: a factor on the register indices with both bits of the i-th pair set
 // (01, 02, 12, 03, 13, 23), kArmSign2 + i a sign; kArmFactorAny: on those with every bit of creg
 // set; kArmZAny: the Z term with controls on register bits. The rest leave the registers alone.
 enum : int {
     kFamY = 0, kFamYk = 1, kFamX = 2, kFamXk = 3, kFamSwap = 4, kFamAny = 5, kFamFactor = 6, kFamSign = 7, kFamZ = 8,
     kArmPair2 = 36, kArmSign2 = 42, kArmFactorAny = 48, kArmZAny = 49,
-    kArmThread = 50,       // diag(m00, m11) by a lane or wave bit
+    kArmThread = 50,       // a Z rotation on a lane or wave bit with its gradient term
     kArmThreadCtrl = 51,   // the same with controls on lane and wave bits
-    kArmOuter = 52,        // diag(m00, m11) by a bit outside the tile, controls allowed
+    kArmOuter = 52,        // the same on a bit outside the tile, controls allowed
     kArmPhase = 53,        // a factor where every control on lane and wave bits is set
     kArmSign = 54,         // a sign where they are
     kArmU = 55,            // the thread's sum that the Z terms on bits that are no register bits share
@@ -506,7 +511,7 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 // Sums over the wavefront of up to 16 consecutive slots: one v_mfma_f64_16x16x4f64 per term
 // multiplies the 64 lanes' values, as a 16 x 4 matrix, by a 4 x 16 matrix whose column `slot` is
-// one, so column slot of the accumulator collects the sums over groups of four lanes; flush
+// their scale, so column slot of the accumulator collects the sums over groups of four lanes; flush
 // adds the accumulator's rows, in a fixed order, and leaves them in red[slot].
 template <int NW>
 struct SlotSums {
@@ -520,8 +525,8 @@ struct SlotSums {
         if (lane < 16 && slot < n_slots) red[slot][wave] = s;
         acc = f64x4{0., 0., 0., 0.};
     }
-    __device__ __forceinline__ void add(double v, int slot, unsigned lane) {
-        const double b = (lane & 15u) == (unsigned)(slot & 15) ? 1. : 0.;
+    __device__ __forceinline__ void add(double v, double scale, int slot, unsigned lane) {
+        const double b = (lane & 15u) == (unsigned)(slot & 15) ? scale : 0.;
         acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, b, acc, 0, 0, 0);
     }
 };
@@ -622,6 +627,13 @@ __device__ __forceinline__ void reg_arm(Cx<R> (&v)[NS][A], const R (&m)[8], cons
                     acc = add_im_conj_mul(acc, v[0][j], v[1][j]);
             });
             acc = ok ? acc : R(0);
+            static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                if constexpr (((j >> P) & 1) != 0) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) mul_by<C>(v[s][j], f);
+                }
+            });
         }
     } else if constexpr (C == kArmFactorAny) {
         static_for<0, A>([&](auto jc) __attribute__((always_inline)) {
@@ -653,7 +665,7 @@ struct PhaseState {
     Cx<R> tf;          // factor per thread, pending: there is one
     Scale<R> sc;       // factor left out of the rotations, scaled: there is one
     unsigned sign;     // sign bit of the factor per thread
-    bool pending, scaled;
+    bool pending, scaled;   // scaled: there is a real factor, the one left out or a sign
     __device__ __forceinline__ void init(double carry) {
         tf = cx<R>(R(1), R(0));
         sc.init(carry);
@@ -667,8 +679,8 @@ struct PhaseState {
         if (!pending && !scaled) return cx<R>(R(1), R(0));
         const double s = sizeof(R) == 8 ? sc.value() : pending ? sc.hi : (double)(R)sc.hi;
         carry = ((sc.hi - s) + sc.lo) * __builtin_amdgcn_rcp(s);
-        if (!pending) return cx<R>((R)s, R(0));
         const double t = __longlong_as_double(__double_as_longlong(s) ^ (long long)((u64)sign << 32));
+        if (!pending) return cx<R>((R)t, R(0));
         return cx<R>((R)((double)tf.re * t), (R)((double)tf.im * t));
     }
 };
@@ -685,7 +697,7 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
     const Cx<R> one = cx<R>(R(1), R(0));
 #pragma unroll
     for (int s = 0; s < NS; ++s) apart(v[s]);
-    double u = 0.;   // sum of Im(conj(lambda) phi), true scale
+    R u = R(0);   // sum of Im(conj(lambda) phi), in the registers' scale
     OpWords<R> op, next;
     op.load(ops + op_begin);
     for (int k = op_begin; k < op_begin + n_ops; ++k) {
@@ -694,7 +706,7 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
         const int slot = op.slot();
         if ((base & op.gctrl()) == op.gctrl()) {
             const unsigned code = op.code(), cthr = op.cthr();
-            const bool ok = (off & cthr) == cthr;
+            const auto controls = [&] { return (off & cthr) == cthr; };   // formed where an arm asks for it
             const int tgt = (int)((code >> 8) & 0xffu), creg = (int)((code >> 16) & 0xffu);
             R m[8];
             if constexpr (B) {
@@ -703,13 +715,14 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
             } else {
                 for (int i = 0; i < 4; ++i) m[i] = op.coef(i);
             }
-            double term = 0.;
-            R acc = R(0);
+            R acc = R(0);   // gradient term, in the registers' scale
             int arm = (int)(code & 0xffu);
             if (arm < 16) arm += m[1] != R(0) ? 4 : 0;   // rotations: the form comes with the coefficients
             const u64 zsrc = (tgt & 0x80) ? base : (u64)off;
+            const double scale = st.sc.hi;   // of the registers, before the op
 #define QG_ARM(C_)                                                                                  \
     case C_: {                                                                                      \
+        const bool ok = (C_) < 16 || controls();                                                   \
         const Cx<R> f = csel(ok, cx<R>(m[0], m[1]), one);                                          \
         if constexpr ((C_) / 4 == kFamAny) {   /* the second half of the matrix */                    \
             if constexpr (B) {                                                                     \
@@ -719,7 +732,6 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
             }                                                                                      \
         }                                                                                          \
         reg_arm<(C_), R, A, NS>(v, m, f, creg, ok, (int)((code >> 24) & 0xfu), tgt, zsrc, acc);          \
-        if constexpr (NS == 2) term = (double)acc * (st.sc.hi * st.sc.hi);                               \
         if constexpr ((C_) < 16) {                                                                    \
             st.sc.times(m[2], m[3]);                                                               \
             st.scaled = true;                                                                      \
@@ -733,31 +745,32 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
                 case kArmThread:
                 case kArmThreadCtrl: {
                     const bool b = ((off >> tgt) & 1u) != 0;
-                    Cx<R> f = csel(b, cx<R>(m[2], m[3]), cx<R>(m[0], m[1]));
-                    if (arm == kArmThreadCtrl) f = csel(ok, f, one);
+                    Cx<R> f = csel(b, cx<R>(m[0], m[1]), one);
+                    if constexpr (NS == 2) acc = b ? -u : u;
+                    if (arm == kArmThreadCtrl) {
+                        const bool ok = controls();
+                        f = csel(ok, f, one);
+                        acc = ok ? acc : R(0);
+                    }
                     st.tf = cmul(st.tf, f);
                     st.pending = true;
-                    if constexpr (NS == 2) {
-                        term = b ? -u : u;
-                        if (arm == kArmThreadCtrl) term = ok ? term : 0.;
-                    }
                     break;
                 }
                 case kArmOuter: {
-                    const bool b = ((base >> tgt) & 1u) != 0;
-                    const Cx<R> f = csel(ok, csel(b, cx<R>(m[2], m[3]), cx<R>(m[0], m[1])), one);
+                    const bool b = ((base >> tgt) & 1u) != 0, ok = controls();
+                    const Cx<R> f = csel(ok && b, cx<R>(m[0], m[1]), one);
                     st.tf = cmul(st.tf, f);
                     st.pending = true;
-                    if constexpr (NS == 2) term = ok ? (b ? -u : u) : 0.;
+                    if constexpr (NS == 2) acc = ok ? (b ? -u : u) : R(0);
                     break;
                 }
                 case kArmPhase:
-                    st.tf = cmul(st.tf, csel(ok, cx<R>(m[0], m[1]), one));
+                    st.tf = cmul(st.tf, csel(controls(), cx<R>(m[0], m[1]), one));
                     st.pending = true;
                     break;
                 case kArmSign:
-                    st.sign ^= ok ? 0x80000000u : 0u;
-                    st.pending = true;
+                    st.sign ^= controls() ? 0x80000000u : 0u;
+                    st.scaled = true;
                     break;
                 case kArmU:
                     if constexpr (NS == 2) {
@@ -766,7 +779,7 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
                             constexpr int j = decltype(jc)::value;
                             w = add_im_conj_mul(w, v[1][j], v[0][j]);
                         });
-                        u = (double)w * (st.sc.hi * st.sc.hi);
+                        u = w;
                     }
                     break;
                 case kArmFlush:
@@ -777,7 +790,7 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
 #undef QG_ARM
 #undef QG_ARMS
             if constexpr (NS == 2)
-                if (slot >= 0) sums.add(term, slot, lane);
+                if (slot >= 0) sums.add((double)acc, scale * scale, slot, lane);
         }
         op = next;
     }
@@ -1006,7 +1019,8 @@ void gate_coefs(const RegGate &g, R *c) {
     } else if (g.kind == kGateX) {
         rotation_coefs(c, g.m.m[0][0].real(), -g.m.m[0][1].imag());
     } else if (g.kind == kGateDiag) {
-        const std::complex<double> r = g.m.m[1][1] / g.m.m[0][0];
+        const std::complex<long double> r =
+            std::complex<long double>(g.m.m[1][1]) / std::complex<long double>(g.m.m[0][0]);
         c[0] = (R)g.m.m[0][0].real(); c[1] = (R)g.m.m[0][0].imag();
         c[2] = (R)g.m.m[1][1].real(); c[3] = (R)g.m.m[1][1].imag();
         c[4] = (R)r.real(); c[5] = (R)r.imag();
@@ -1026,12 +1040,15 @@ void append_flush(std::vector<RegOp<R>> &out, int group) {
     out.push_back(op);
 }
 
+// A phase of the whole state: diagonal gates on register bits leave one each.
+typedef std::complex<long double> GlobalPhase;
+
 // Appends the ops of gate g (index `row` in the coefficient table) in phase P. local: tile bit
 // of a state lane, -1 outside the tile. n_slots counts the gradient slots given out; have_u: the
-// sum of kArmU is that of the registers as they are.
+// sum of kArmU is that of the registers as they are; global takes the phases of the whole state.
 template <class R>
 void append_ops(std::vector<RegOp<R>> &out, const RegGate &g, int row, const PhasePlan &P, const int *local,
-                int &n_slots, bool &have_u) {
+                int &n_slots, bool &have_u, GlobalPhase &global) {
     if (g.pauli != 0 && n_slots > 0 && n_slots % 16 == 0) append_flush(out, n_slots / 16 - 1);
     const int rb = (int)P.regs.size();
     auto position = [&](int bit) { return (int)(std::find(P.regs.begin(), P.regs.end(), bit) - P.regs.begin()); };
@@ -1087,33 +1104,43 @@ void append_ops(std::vector<RegOp<R>> &out, const RegGate &g, int row, const Pha
             push(kArmFactorAny, 0, regs, coff, -1, o);
         }
     };
+    // diag(m00, m11) = m00 on the controls, then the ratio m11 / m00 on the controls and the target.
+    // With both entries as factors, each rounded, their moduli (equal, and off by the same rounding)
+    // would scale the whole state; of many rotations by one angle these errors add up.
     const bool one0 = d0 == 1. && g.pauli == 0;   // m00 == 1 whatever the parameter
-    if (tp < rb || creg != 0 || one0) {
-        RegOp<R> t = op;   // the controls and the target
-        int treg = creg;
-        if (lt < 0)
-            t.gctrl |= u64(1) << g.target;
-        else if (tp < rb)
-            treg |= 1 << tp;
+    if (!one0) {
+        const long double n = std::norm(GlobalPhase(d0));
+        if (g.ctrl.empty() && std::abs(n - 1.L) < 1e-14L)
+            global *= GlobalPhase(d0) / std::sqrt(n);
         else
-            t.cthr |= 1u << lt;
-        if (slot >= 0) {
-            if (creg == 0 && tp < rb)
-                push(4 * kFamZ + tp, 0, 0, 0, slot, op);
-            else   // target: register position, or RB + local bit, or 0x80 | RB + state bit
-                push(kArmZAny, tp < rb ? tp : lt >= 0 ? rb + lt : 0x80 | (rb + g.target), creg, 0, slot, op);
-        }
-        if (!one0) factor(op, creg, 0, d0);
-        factor(t, treg, one0 ? 2 : 4, one0 ? d1 : d1 / d0);
+            factor(op, creg, 0, d0);
+    }
+    const int coff = one0 ? 2 : 4;
+    if (slot >= 0 && creg == 0 && tp < rb) {   // term and factor in one op
+        push(4 * kFamZ + tp, 0, 1 << tp, coff, slot, op);
         return;
     }
-    if (slot >= 0 && !have_u) {
-        RegOp<R> u;
-        std::memset(&u, 0, sizeof(u));
-        push(kArmU, 0, 0, 0, -1, u);
-        have_u = true;
+    if (slot >= 0 && creg == 0) {
+        if (!have_u) {
+            RegOp<R> u;
+            std::memset(&u, 0, sizeof(u));
+            push(kArmU, 0, 0, 0, -1, u);
+            have_u = true;
+        }
+        push(lt < 0 ? kArmOuter : op.cthr != 0 ? kArmThreadCtrl : kArmThread, lt >= 0 ? lt : g.target, 0, coff, slot,
+             op);
+        return;
     }
-    push(lt < 0 ? kArmOuter : op.cthr != 0 ? kArmThreadCtrl : kArmThread, lt >= 0 ? lt : g.target, 0, 0, slot, op);
+    if (slot >= 0)   // target: register position, or RB + local bit, or 0x80 | RB + state bit
+        push(kArmZAny, tp < rb ? tp : lt >= 0 ? rb + lt : 0x80 | (rb + g.target), creg, 0, slot, op);
+    int treg = creg;
+    if (lt < 0)
+        op.gctrl |= u64(1) << g.target;
+    else if (tp < rb)
+        treg |= 1 << tp;
+    else
+        op.cthr |= 1u << lt;
+    factor(op, treg, coff, one0 ? d1 : d1 / d0);
 }
 
 // The register gates of the gate list of a sweep: rotations whole (their gradient terms are
@@ -1152,10 +1179,15 @@ struct BuiltPass {
 
 // Passes over a gate list: tiles of m of n lanes that hold the lowest `low`, rb register and wb
 // wave bits, at most max_gates gates, max_ops ops and max_phases phases a pass. Gates whose tile has no bit left
-// for them (tile bits == low bits) are refused by the caller's choice of m > low.
-template <class R>
-std::vector<BuiltPass<R>> build_passes(const std::vector<RegGate> &gates, int n, int m, int low, int rb, int wb,
-                                       int max_gates, int max_ops, int max_phases) {
+// for them (tile bits == low bits) are refused by the caller's choice of m > low. Phases of the whole
+// state are applied once per pass (the amplitudes are wanted) or left out (kNoGlobalPhase:
+// expectation values and gradients do not depend on them; batched rotations have theirs in no table).
+enum GlobalPhases { kGlobalPhase, kNoGlobalPhase };
+//
+// take(pass) is called with each pass as it is planned, so that the first ones can run meanwhile.
+template <class R, class Take>
+void for_each_pass(const std::vector<RegGate> &gates, int n, int m, int low, int rb, int wb, int max_gates,
+                   int max_ops, int max_phases, GlobalPhases keep, Take take) {
     QG_REQUIRE(low < m && m <= n, "register pass: %d tile bits, %d low, %d lanes", m, low, n);
     const int ng = (int)gates.size();
     std::vector<PlanGate> pg(ng);
@@ -1163,11 +1195,10 @@ std::vector<BuiltPass<R>> build_passes(const std::vector<RegGate> &gates, int n,
         pg[i] = PlanGate{gates[i].target, &gates[i].ctrl, gates[i].kind == kGateDiag,
                          gates[i].kind == kGateAny ? 2 : 1, gates[i].pauli != 0 ? 1 : 0};
     std::vector<char> done(ng, 0);
-    std::vector<BuiltPass<R>> out;
     for (int first = 0; first < ng;) {
-        // a diagonal gate on a register bit can take two ops (three with a gradient): a pass
-        // that comes out too long is planned again with fewer gates
-        for (int limit = std::min(max_gates, max_ops);; limit = limit * 3 / 4) {
+        // a diagonal gate on a register bit can take two ops: a pass that comes out too long is
+        // planned again with fewer gates
+        for (int limit = std::min(max_gates, max_ops);;) {
             std::vector<char> now(done);
             const PassBits pb = next_pass(pg, now, first, n, m, low, limit, kMaxSweepSlots);
             QG_REQUIRE(!pb.gates.empty(), "register pass takes no gate");
@@ -1179,14 +1210,25 @@ std::vector<BuiltPass<R>> build_passes(const std::vector<RegGate> &gates, int n,
             bp.low = pb.low;
             bp.gates = pb.gates;
             int slots = 0;
+            GlobalPhase global(1.L);
             for (const PhasePlan &P : plan_phases(pg, pb.gates, local, n, m, rb, wb)) {
                 const int begin = (int)bp.ops.size();
                 bool have_u = false;
                 for (int gi : P.order) {
-                    append_ops<R>(bp.ops, gates[gi], gi, P, local, slots, have_u);
+                    append_ops<R>(bp.ops, gates[gi], gi, P, local, slots, have_u, global);
                     if (gates[gi].pauli != 0) bp.slot_gate.push_back(gi);
                 }
                 bp.phases.push_back(phase_bits(P, begin, (int)bp.ops.size() - begin));
+            }
+            if (keep == kGlobalPhase && global != GlobalPhase(1.L)) {
+                RegOp<R> op;
+                std::memset(&op, 0, sizeof(op));
+                op.code = (unsigned)kArmPhase;
+                op.slot = -1;
+                op.c[0] = (R)global.real();
+                op.c[1] = (R)global.imag();
+                bp.ops.push_back(op);
+                bp.phases.back().n_ops += 1;
             }
             if (slots > 0) {   // the last slots
                 append_flush(bp.ops, (slots - 1) / 16);
@@ -1194,14 +1236,27 @@ std::vector<BuiltPass<R>> build_passes(const std::vector<RegGate> &gates, int n,
             }
             if ((int)bp.ops.size() > max_ops || (int)bp.phases.size() > max_phases) {
                 QG_REQUIRE(limit > 2, "register pass: a gate takes too many ops");
+                int weight = 0;
+                for (int gi : pb.gates) weight += pg[gi].weight;
+                limit = std::min(weight - 1, (int)bp.phases.size() > max_phases
+                                                 ? weight * 3 / 4
+                                                 : weight * max_ops / (int)bp.ops.size());
                 continue;
             }
             done.swap(now);
-            out.push_back(bp);
+            take(std::move(bp));
             break;
         }
         while (first < ng && done[first]) ++first;
     }
+}
+
+template <class R>
+std::vector<BuiltPass<R>> build_passes(const std::vector<RegGate> &gates, int n, int m, int low, int rb, int wb,
+                                       int max_gates, int max_ops, int max_phases, GlobalPhases keep) {
+    std::vector<BuiltPass<R>> out;
+    for_each_pass<R>(gates, n, m, low, rb, wb, max_gates, max_ops, max_phases, keep,
+                     [&](BuiltPass<R> &&bp) { out.push_back(std::move(bp)); });
     return out;
 }
 
