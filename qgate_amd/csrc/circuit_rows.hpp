@@ -54,14 +54,25 @@ __device__ __forceinline__ void row_coefs(const BRow<R> &row, const double *__re
 // row of each in the coefficient table. Rotations keep their form at every angle; fixed gates
 // are split as in the single-circuit passes. RegGate::source is the gate of the structure.
 template <class R>
-std::vector<RegGate> row_gates(const std::vector<CircuitOp> &ops, bool back, std::vector<BRow<R>> &rows) {
+std::vector<RegGate> row_gates(const std::vector<CircuitOp> &ops, int n_lanes, bool back,
+                               std::vector<BRow<R>> &rows) {
     std::vector<RegGate> out;
     const int n = (int)ops.size();
+    const std::vector<int> role = parity_roles(
+        n, n_lanes, [&](int i) -> const CircuitOp & { return ops[i]; },
+        [&](int i) { return ops[i].kind == 0 && ops[i].ctrl.size() == 1 && is_x(ops[i].mat); },
+        [&](int i) {
+            const CircuitOp &op = ops[i];
+            return op.ctrl.empty() && (op.kind == 1 ? op.pauli == 3 : diag2(op.mat) && has_ratio(op.mat));
+        });
     for (int k = 0; k < n; ++k) {
         const int i = back ? n - 1 - k : k;
         const CircuitOp &op = ops[i];
+        if (role[i] == kDropped) continue;
+        const size_t at = out.size();
         if (op.kind == 0) {
             append_fixed(out, back ? dagger(op.mat) : op.mat, op.ctrl, op.target, i);
+            if (role[i] != kKept && out.size() > at) out.back().parity = role[i];
             continue;
         }
         RegGate g;
@@ -71,6 +82,7 @@ std::vector<RegGate> row_gates(const std::vector<CircuitOp> &ops, bool back, std
         g.source = i;
         g.ctrl = op.ctrl;
         g.m = rotation(op.pauli, back ? -1. : 1.);   // its form; the angle is each item's own
+        if (role[i] != kKept) g.parity = role[i];
         out.push_back(g);
     }
     rows.clear();

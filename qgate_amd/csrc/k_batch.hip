@@ -717,7 +717,7 @@ void build_group(Group &g, const Tuning &t) {
     }
     std::vector<BRow<R>> frows, srows;
     if (fregs)
-        for (const BuiltPass<R> &bp : build_passes<R>(row_gates<R>(g.ops, false, frows), n, TC::MaxBits, lowf,
+        for (const BuiltPass<R> &bp : build_passes<R>(row_gates<R>(g.ops, n, false, frows), n, TC::MaxBits, lowf,
                                                       Log2<kFA>::v, kWB, TC::MaxOps, TC::MaxRegOps, kMaxPhases, kNoGlobalPhase))
             progs.push_back(reg_program(bp));
     // sweep passes: the gates in reverse order
@@ -766,7 +766,7 @@ void build_group(Group &g, const Tuning &t) {
         g.spasses.push_back(p);
     }
     if (sregs) {
-        const std::vector<RegGate> gates = row_gates<R>(g.ops, true, srows);
+        const std::vector<RegGate> gates = row_gates<R>(g.ops, n, true, srows);
         slot_out.clear();
         g.spass_slot_begin.clear();
         max_slots = 1;

@@ -457,7 +457,7 @@ void small_sweep(const Cx<R> *phi, const Cx<R> *lam, int n_lanes, const std::vec
     QG_REQUIRE((int)gates.size() <= small_max_gates(), "sweep in one workgroup: %d gates", (int)gates.size());
     for (size_t i = 0; i < gates.size(); ++i) out[i] = 0.;
     SmallTables<R> t;
-    plan_small(t, sweep_gates(gates), m, kNoGlobalPhase);
+    plan_small(t, sweep_gates(gates, n_lanes), m, kNoGlobalPhase);
     if (t.passes.empty()) return;
     t.ops.push_back(RegOp<R>());   // one more is read than there are
     TableLayout tab;
@@ -525,10 +525,10 @@ void SmallBatch::build(const std::vector<SmallGroupIn> &in) {
         std::vector<BRow<R>> fr, sr;
         g.f_op = (int)t.ops.size();
         g.f_phase = (int)t.phases.size();
-        plan_small_forward(t, row_gates<R>(*gi.ops, false, fr), m, kNoGlobalPhase);
+        plan_small_forward(t, row_gates<R>(*gi.ops, gi.n, false, fr), m, kNoGlobalPhase);
         g.f_phases = (int)t.phases.size() - g.f_phase;
         g.pass = (int)t.passes.size();
-        plan_small(t, row_gates<R>(*gi.ops, true, sr), m, kNoGlobalPhase);
+        plan_small(t, row_gates<R>(*gi.ops, gi.n, true, sr), m, kNoGlobalPhase);
         g.n_passes = (int)t.passes.size() - g.pass;
         g.n_ops = (int)t.ops.size() - g.f_op;
         passes_.push_back(g.n_passes);

@@ -661,7 +661,7 @@ static void sweep_in_registers(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::v
                                double *d_terms, int low) {
     typedef SweepCfg<R> C;
     constexpr int A = (1 << C::RegBits) / C::RegThreads;
-    const std::vector<RegGate> rg = sweep_gates(gates);
+    const std::vector<RegGate> rg = sweep_gates(gates, n_lanes);
     const std::vector<BuiltPass<R>> passes = build_passes<R>(
         rg, n_lanes, C::RegBits, low, Log2<A>::v, Log2<C::RegThreads / 64>::v, 1 << 30, 1 << 30,
         1 << 30, kNoGlobalPhase);
@@ -721,7 +721,7 @@ static void sweep_in_lds(Cx<R> *phi, Cx<R> *lam, int n_lanes, const std::vector<
     for (int i = 0; i < n_gates; ++i) {
         const SweepGate &g = gates[i];
         pg[i] = PlanGate{g.target, &g.ctrl, is_diagonal(g.udag) && (g.pauli == 0 || g.pauli == 3), 1,
-                         g.pauli != 0 ? 1 : 0};
+                         g.pauli != 0 ? 1 : 0, -1};
     }
     std::vector<char> done(n_gates, 0);
     std::vector<SweepOp<R>> ops;

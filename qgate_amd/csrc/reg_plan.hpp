@@ -1,4 +1,4 @@
-// Planning of register-resident tile passes (reg_engine.hpp), on the host: how a gate list
+// Planning of register-resident tile passes (tile_reg.hpp), on the host: how a gate list
 // becomes the ops, phases and passes that the kernels run. Shared by the single-circuit passes
 // (k_tile.hip) and the batched ones (k_batch.hip).
 #pragma once
@@ -32,6 +32,7 @@ struct RegGate {
     int target = 0;
     int pauli = 0;      // gradient generator (1 X, 2 Y, 3 Z) of a sweep's rotation, 0: none
     int source = 0;     // the gate of the caller's list that it came from
+    int parity = -1;    // diagonal gates: it acts by target ^ this lane (no controls), -1: by the target
     std::vector<int> ctrl;
     GateMatrix m;
 };
@@ -108,6 +109,35 @@ inline bool has_ratio(const GateMatrix &g) {
 
 inline bool trivial_diag(std::complex<double> d0, std::complex<double> d1) { return d0 == 1. && d1 == 1.; }
 
+// CX . D . CX with D diagonal on the target (an exp(-i a Z Z / 2), for instance) is D by the parity of
+// control and target: one diagonal gate and no register moves. role[i] is then kDropped for the CX
+// gates and the control's lane for D, kKept for all other gates. A triple is taken if no other gate on
+// its two lanes lies between. gate(i): ctrl, target; is_cx(i): X with one control; is_diag(i): a
+// diagonal gate without controls (for every parameter). (13 qubits, 6 layers of ZZ and X rotations: 307 gates become 163.)
+constexpr int kKept = -1, kDropped = -2;
+template <class GateAt, class IsCx, class IsDiag>
+std::vector<int> parity_roles(int n_gates, int n_lanes, GateAt gate, IsCx is_cx, IsDiag is_diag) {
+    std::vector<int> role(n_gates, kKept), last(n_lanes, -1), before(n_gates, -1);   // before: on the target
+    for (int i = 0; i < n_gates; ++i) {
+        const int t = gate(i).target;
+        const std::vector<int> &ctrl = gate(i).ctrl;
+        if (is_cx(i)) {
+            const int c = ctrl[0], d = last[t], x = d >= 0 ? before[d] : -1;
+            if (x >= 0 && role[d] == kKept && role[x] == kKept && is_diag(d) && is_cx(x) && last[c] == x &&
+                gate(x).target == t && gate(x).ctrl[0] == c) {
+                role[x] = role[i] = kDropped;
+                role[d] = c;
+                last[c] = d;
+                continue;
+            }
+        }
+        before[i] = last[t];
+        last[t] = i;
+        for (int c : ctrl) last[c] = i;
+    }
+    return role;
+}
+
 // Appends the register gates of one fixed gate (no parameter), in the order they apply.
 inline void append_fixed(std::vector<RegGate> &out, const GateMatrix &m, const std::vector<int> &ctrl, int target,
                          int source) {
@@ -157,6 +187,9 @@ std::vector<RegGate> merged_gates(int n_gates, int n_lanes, GateAt gate) {
     out.reserve((size_t)n_gates * 2);
     std::vector<GateMatrix> run(n_lanes);
     std::vector<int> last(n_lanes, -1);   // source of the lane's run, -1: none
+    const std::vector<int> role = parity_roles(
+        n_gates, n_lanes, gate, [&](int i) { return gate(i).ctrl.size() == 1 && is_x(gate(i).m); },
+        [&](int i) { return gate(i).ctrl.empty() && diag2(gate(i).m) && has_ratio(gate(i).m); });
     auto emit = [&](int lane, bool keep_diagonal) {
         if (last[lane] < 0) return;
         GateMatrix &m = run[lane];
@@ -174,6 +207,15 @@ std::vector<RegGate> merged_gates(int n_gates, int n_lanes, GateAt gate) {
     };
     for (int i = 0; i < n_gates; ++i) {
         const auto &g = gate(i);
+        if (role[i] == kDropped) continue;
+        if (role[i] != kKept) {
+            emit(role[i], true);
+            emit(g.target, true);
+            const size_t at = out.size();
+            append_fixed(out, g.m, {}, g.target, i);
+            if (out.size() > at) out.back().parity = role[i];
+            continue;
+        }
         if (g.ctrl.empty()) {
             GateMatrix &m = run[g.target];
             if (last[g.target] < 0) {
@@ -216,6 +258,7 @@ struct PlanGate {
     bool diag;
     int weight;    // ops it may take
     int slots;     // gradient slots
+    int parity;    // second lane of a parity gate, -1: none
 };
 
 // Lanes held by the gates left out of a scan: two gates commute when on every lane they share
@@ -227,11 +270,12 @@ class HeldLanes {
         if (g.diag ? held_[g.target] == 2 : held_[g.target] != 0) return true;
         for (int c : *g.ctrl)
             if (held_[c] == 2) return true;
-        return false;
+        return g.parity >= 0 && held_[g.parity] == 2;
     }
     void hold(const PlanGate &g) {
         put(g.target, g.diag ? 1 : 2);
         for (int c : *g.ctrl) put(c, 1);
+        if (g.parity >= 0) put(g.parity, 1);
     }
     bool all() const { return full_ == (int)held_.size(); }
 
@@ -288,7 +332,8 @@ constexpr int kMaxScaled = 16;
 // whose non-diagonal target is one of its rb register bits or can become one; then each diagonal
 // gate moves, between the pair gates on its lanes before and after it, to a phase where none of
 // its lanes is a register bit (there it is one factor per thread instead of an update of the
-// registers), if possible one that already has such factors.
+// registers), if possible one that already has such factors. A parity gate stays in a phase where
+// neither of its lanes becomes a register bit, so that it is always such a factor.
 inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const std::vector<int> &gates,
                                           const int *local, int n, int m, int rb, int wb) {
     std::vector<PhasePlan> out;
@@ -297,15 +342,21 @@ inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const 
     size_t first = 0;
     while (first < gates.size()) {
         PhasePlan P;
-        unsigned in = 0;
+        unsigned in = 0, out_of = 0;   // register bits, and bits that may not become ones
         HeldLanes held(n);
         int pairs = 0, free_regs = rb;
         for (size_t k = first; k < gates.size(); ++k) {
             if (done[k]) continue;
             const PlanGate &q = g[gates[k]];
             const unsigned bit = q.diag ? 0u : 1u << local[q.target];
-            const bool fits = q.diag || (pairs < kMaxScaled && ((in & bit) || free_regs > 0));
+            bool fits = q.diag || (pairs < kMaxScaled && ((in & bit) || (free_regs > 0 && !(out_of & bit))));
+            unsigned lanes = 0;
+            if (q.parity >= 0) {
+                for (int l : {q.target, q.parity}) lanes |= local[l] >= 0 ? 1u << local[l] : 0u;
+                fits = !(in & lanes) && m - __builtin_popcount(in | out_of | lanes) >= free_regs;
+            }
             if (fits && !held.conflicts(q)) {
+                out_of |= lanes;
                 if (!q.diag) {
                     if (!(in & bit)) --free_regs;
                     in |= bit;
@@ -321,7 +372,7 @@ inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const 
         while (first < gates.size() && done[first]) ++first;
         // pad with the highest free bits, so that the lane bits are the lowest ones
         for (int b = m - 1; free_regs > 0 && b >= 0; --b)
-            if (!((in >> b) & 1)) in |= 1u << b, --free_regs;
+            if (!(((in | out_of) >> b) & 1)) in |= 1u << b, --free_regs;
         for (int b = 0; b < m; ++b)
             ((in >> b) & 1 ? P.regs : (int)P.lanes.size() < 6 ? P.lanes : P.waves).push_back(b);
         if ((int)P.waves.size() != wb) raise_error("tile layout does not match the workgroup");
@@ -341,7 +392,7 @@ inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const 
             if (g[gi].diag) {
                 int lo = seen[g[gi].target];
                 for (int c : *g[gi].ctrl) lo = std::max(lo, seen[c]);
-                diags.push_back(Diag{gi, lo, (int)pairs.size(), 0, 0});
+                diags.push_back(Diag{gi, lo, (int)pairs.size(), 0, (int)ph});
             } else {
                 pairs.push_back(gi);
                 phase_of.push_back((int)ph);
@@ -354,6 +405,10 @@ inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const 
     for (int d = (int)diags.size() - 1, k = np; d >= 0; --d) {
         Diag &q = diags[d];
         for (; k > q.hi; --k) seen[g[pairs[k - 1]].target] = k - 1;
+        if (g[q.gate].parity >= 0) {   // stays where it is
+            q.at = q.hi;
+            continue;
+        }
         q.hi = seen[g[q.gate].target];
         for (int c : *g[q.gate].ctrl) q.hi = std::min(q.hi, seen[c]);
     }
@@ -361,6 +416,11 @@ inline std::vector<PhasePlan> plan_phases(const std::vector<PlanGate> &g, const 
     std::vector<int> count(np + 2, 0);
     for (Diag &d : diags) {
         const PlanGate &q = g[d.gate];
+        if (q.parity >= 0) {
+            has_factor[d.phase] = 1;
+            ++count[d.at + 1];
+            continue;
+        }
         const auto bit = [&](int lane) { return local[lane] >= 0 ? 1u << local[lane] : 0u; };
         unsigned mask = bit(q.target);
         for (int c : *q.ctrl) mask |= bit(c);

@@ -9,11 +9,6 @@ namespace qg {
 // diagonal on a tile bit, or as a diagonal whose target lies outside the tile (one factor for
 // the whole tile).
 enum : int { kOpPair = 0, kOpDiagLocal = 1, kOpDiagOuter = 2 };
-// Cheaper forms of the same updates (register-resident passes): a pair gate that only swaps
-// (X, CX, CCX targets), a pair gate with a real matrix (H, RY), and a diagonal on a tile bit
-// with m00 == 1 (Z, S, T, U1, CZ, cu1: only the |1> half changes).
-enum : int { kOpPairSwap = 3, kOpPairReal = 4, kOpDiagPhase = 5 };
-
 // Tile layouts hold at most kTilePosMax tile bits; pos[] arrays have that many entries.
 constexpr int kTilePosMax = 16;
 

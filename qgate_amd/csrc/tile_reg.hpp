@@ -102,7 +102,8 @@ enum : int {
     kArmSign = 54,         // a sign where they are
     kArmU = 55,            // the thread's sum that the Z terms on bits that are no register bits share
     kArmFlush = 56,        // 16 gradient slots are complete
-    kArmNone = 57          // the second half of a general 2x2
+    kArmNone = 57,         // the second half of a general 2x2
+    kArmParity = 58        // a factor where two bits differ, with the gradient term of their ZZ
 };
 
 // One op of a register pass. code: arm | target << 8 | creg << 16 | generator << 24 | first
@@ -764,6 +765,16 @@ __device__ __forceinline__ void run_phase(Cx<R> (&v)[NS][A], const RegOp<R> *ops
                     if constexpr (NS == 2) acc = ok ? (b ? -u : u) : R(0);
                     break;
                 }
+                case kArmParity: {   // bits: of the tile, or 0x80 | of the state
+                    const auto bit = [&](int x) {
+                        return (x & 0x80) ? (unsigned)(base >> (x & 0x7f)) & 1u : (off >> x) & 1u;
+                    };
+                    const bool b = (bit(tgt) ^ bit(creg)) != 0;
+                    if constexpr (NS == 2) acc = b ? -u : u;
+                    st.tf = cmul(st.tf, csel(b, cx<R>(m[0], m[1]), one));
+                    st.pending = true;
+                    break;
+                }
                 case kArmPhase:
                     st.tf = cmul(st.tf, csel(controls(), cx<R>(m[0], m[1]), one));
                     st.pending = true;
@@ -1116,6 +1127,19 @@ void append_ops(std::vector<RegOp<R>> &out, const RegGate &g, int row, const Pha
             factor(op, creg, 0, d0);
     }
     const int coff = one0 ? 2 : 4;
+    if (g.parity >= 0) {
+        auto where = [&](int lane) { return local[lane] >= 0 ? local[lane] : 0x80 | lane; };
+        for (int lane : {g.target, g.parity})
+            QG_REQUIRE(local[lane] < 0 || position(local[lane]) >= rb, "register phase: parity on a register bit");
+        if (slot >= 0 && !have_u) {
+            RegOp<R> u;
+            std::memset(&u, 0, sizeof(u));
+            push(kArmU, 0, 0, 0, -1, u);
+            have_u = true;
+        }
+        push(kArmParity, where(g.target), where(g.parity), coff, slot, op);
+        return;
+    }
     if (slot >= 0 && creg == 0 && tp < rb) {   // term and factor in one op
         push(4 * kFamZ + tp, 0, 1 << tp, coff, slot, op);
         return;
@@ -1145,23 +1169,33 @@ void append_ops(std::vector<RegOp<R>> &out, const RegGate &g, int row, const Pha
 
 // The register gates of the gate list of a sweep: rotations whole (their gradient terms are
 // taken right before them), fixed gates split as in the forward pass.
-inline std::vector<RegGate> sweep_gates(const std::vector<SweepGate> &gates) {
+inline std::vector<RegGate> sweep_gates(const std::vector<SweepGate> &gates, int n_lanes) {
     std::vector<RegGate> out;
     out.reserve(gates.size() + gates.size() / 4);
+    const std::vector<int> role = parity_roles(
+        (int)gates.size(), n_lanes, [&](int i) -> const SweepGate & { return gates[i]; },
+        [&](int i) { return gates[i].pauli == 0 && gates[i].ctrl.size() == 1 && is_x(gates[i].udag); },
+        [&](int i) {
+            const SweepGate &g = gates[i];
+            return g.ctrl.empty() && (g.pauli == 3 || (g.pauli == 0 && diag2(g.udag) && has_ratio(g.udag)));
+        });
     for (int i = 0; i < (int)gates.size(); ++i) {
         const SweepGate &g = gates[i];
+        if (role[i] == kDropped) continue;
+        const size_t at = out.size();
         if (g.pauli == 0) {
             append_fixed(out, g.udag, g.ctrl, g.target, i);
-            continue;
+        } else {
+            RegGate r;
+            r.kind = g.pauli == 3 ? kGateDiag : !g.ctrl.empty() ? kGateAny : g.pauli == 1 ? kGateX : kGateY;
+            r.target = g.target;
+            r.pauli = g.pauli;
+            r.source = i;
+            r.ctrl = g.ctrl;
+            r.m = g.udag;
+            out.push_back(r);
         }
-        RegGate r;
-        r.kind = g.pauli == 3 ? kGateDiag : !g.ctrl.empty() ? kGateAny : g.pauli == 1 ? kGateX : kGateY;
-        r.target = g.target;
-        r.pauli = g.pauli;
-        r.source = i;
-        r.ctrl = g.ctrl;
-        r.m = g.udag;
-        out.push_back(r);
+        if (role[i] != kKept && out.size() > at) out.back().parity = role[i];
     }
     return out;
 }
@@ -1193,7 +1227,7 @@ void for_each_pass(const std::vector<RegGate> &gates, int n, int m, int low, int
     std::vector<PlanGate> pg(ng);
     for (int i = 0; i < ng; ++i)
         pg[i] = PlanGate{gates[i].target, &gates[i].ctrl, gates[i].kind == kGateDiag,
-                         gates[i].kind == kGateAny ? 2 : 1, gates[i].pauli != 0 ? 1 : 0};
+                         gates[i].kind == kGateAny ? 2 : 1, gates[i].pauli != 0 ? 1 : 0, gates[i].parity};
     std::vector<char> done(ng, 0);
     for (int first = 0; first < ng;) {
         // a diagonal gate on a register bit can take two ops: a pass that comes out too long is
