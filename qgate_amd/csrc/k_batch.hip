@@ -8,15 +8,18 @@
 // the per-circuit gate matrices (computed on the device from each circuit's parameters) and
 // observable coefficients are picked by the tile's item index. Groups whose circuits fit one
 // workgroup run there whole (k_small.hip). Any other group runs as:
-//   k_batch_mats     U and U^dagger of every (item, gate), from the parameters (FP64 sincos)
+//   k_row_coefs      the coefficients of every (item, gate), from the parameters (FP64 sincos)
+//                    (k_batch_mats: U and U^dagger instead, for LDS passes)
 //   k_batch_zero     |0...0> in every item
-//   k_batch_pass     forward tile passes (gates applied in LDS, many per pass)
-//   k_batch_pauli    lambda = H psi in tile passes, the last one with Re<psi|lambda> partials
-//   k_batch_sweep    backward sweep passes over psi and lambda with gradient partials
+//   k_tile_reg       forward tile passes (k_batch_pass: in LDS)
+//   k_batch_pauli_full   lambda = H psi in tile passes, the last one with Re<psi|lambda> partials
+//                    (k_batch_pauli: tiles that are not full-size)
+//   k_tile_sweep_reg     backward sweep passes over psi and lambda with gradient partials
+//                    (k_batch_sweep: in LDS)
 //   k_rows_sum       partials -> values and per-gate gradient terms (fixed order)
 //   k_batch_grads    per-gate terms -> per-parameter gradients (fixed order)
-// The pass kernels are persistent: a fixed grid of workgroups strides over the tiles. Tile
-// size, workgroup size and grid size per group are picked by timing candidates on the first
+// The LDS pass kernels are persistent: a fixed grid of workgroups strides over the tiles. Register
+// or LDS passes, tile size, workgroup size and grid size per group are picked by timing candidates on the first
 // run (the autotuner below); the whole sequence for all groups is then captured once into a
 // HIP graph and replayed by later runs with new parameters.
 #include <algorithm>
@@ -389,8 +392,7 @@ struct BCfg<double> {
     static constexpr int Low = 3;
 };
 // Register-resident passes (tile_reg.hpp): 256 threads, 2^12 / 2^11 amplitudes per forward tile
-// (16 / 8 per thread) and 2^11 / 2^10 per sweep tile (8 / 4 per thread and state), as in the
-// single-circuit passes.
+// (16 / 8 per thread) and 2^11 / 2^10 per sweep tile (8 / 4 per thread and state).
 constexpr int kBatchRegThreads = 256;
 static_assert(BCfg<float>::MaxBits == TileCfg<float>::MaxBits && BCfg<double>::MaxBits == TileCfg<double>::MaxBits,
               "forward tiles");

@@ -6,11 +6,11 @@
 // amplitudes (M >= n; amplitudes above 2^n are zero and stay zero) in 2^(M - 3) threads, 8 each,
 // worked on by the register engine of the tile passes (tile_reg.hpp), with LDS for its layout
 // changes. No op has a bit outside the tile.
-// What is left is latency too: at 13 qubits each op waits about 0.4 us for its decoding, its LDS
-// hand-over or a table line, with 4 waves on each SIMD of one compute unit (a 13-qubit sweep of
-// 307 gates 233 us, its forward part 165 us).
-// <H> and gradient, whole calls, before and after: 6 qubits complex128 336 -> 229 us; 13 qubits
-// complex64, 307 gates, 808 -> 671 us; a batch of 96 circuits of 6 to 11 qubits 1580 -> 521 us.
+// What is left is latency too: at 13 qubits an op takes 0.4 to 0.6 us, of decoding, LDS hand-overs and
+// table lines, with 4 waves on each SIMD of one compute unit (307 gates, 176 ops forward: 99 us, the
+// sweep 137 us).
+// <H> and gradient, whole calls, before the circuits ran here and now: 6 qubits complex128 336 ->
+// 229 us; 13 qubits complex64, 307 gates, 808 -> 547 us; 96 circuits of 6 to 11 qubits 1580 -> 503 us.
 //   one circuit      k_small_expect and k_small_sweep, one launch for each of the two calls
 //   a batch          k_small_rows (coefficients of every item, from its parameters), then one
 //                    workgroup an item, k_small_batch, from |0...0> to the item's gradient
