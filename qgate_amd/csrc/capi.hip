@@ -150,16 +150,21 @@ constexpr int kDenseWidth = 6;   // default block width of QGHIP_FUSION_DENSE
 
 bool queued(const qghip_qubit_states *qs) { return !qs->pending.empty() || qs->dec_lane >= 0; }
 
-// qs is about to be written or freed: bounded pools drawing from it can no longer draw, and
-// nothing is known of its lanes.
-void touch(qghip_qubit_states *qs) {
-    if (qs == nullptr) return;
-    qs->known = KnownLanes();
+// qs changes: bounded pools drawing from it can no longer draw.
+void stale_pools(qghip_qubit_states *qs) {
     for (qghip_sampling_pool *pl : qs->readers) {
         pl->stale = true;
         pl->src = nullptr;
     }
     qs->readers.clear();
+}
+
+// qs is about to be written or freed: nothing is known of its lanes any more. A recorded collapse
+// that is launched in between makes its lane known, so a caller that applies one flushes first.
+void touch(qghip_qubit_states *qs) {
+    if (qs == nullptr) return;
+    qs->known = KnownLanes();
+    stale_pools(qs);
 }
 
 // The collapse recorded on qs: run(known, norm) launches it with the norm in the state
@@ -262,12 +267,12 @@ void apply_matrix(const qghip_qubit_processor *p, Prec prec, qghip_qubit_states 
     std::sort(sorted.begin(), sorted.end());
     if (std::adjacent_find(sorted.begin(), sorted.end()) != sorted.end())
         value_error("duplicate control lanes");
-    touch(qs);
     if (p != nullptr && (p->fusion == QGHIP_FUSION_TILE || p->fusion == QGHIP_FUSION_DENSE)) {
         // gates queued under other settings are applied under those first
         if (!qs->pending.empty() &&
             (qs->fuse_mode != p->fusion || qs->tile_bits != p->tile_bits || qs->low_bits != p->low_bits))
             flush(qs);
+        stale_pools(qs);   // known lanes: of the amplitudes as they are until the queue is applied
         if (!queued(qs)) pending_states().push_back(qs);
         qs->fuse_mode = p->fusion;
         qs->tile_bits = p->tile_bits;
@@ -277,6 +282,7 @@ void apply_matrix(const qghip_qubit_processor *p, Prec prec, qghip_qubit_states 
         return;
     }
     flush(qs);
+    touch(qs);
     by_prec(prec, [&](auto r) {
         typedef decltype(r) R;
         launch_gate<R>(amps<R>(qs), qs->n_lanes, m, controls, target);

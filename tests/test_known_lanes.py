@@ -85,3 +85,42 @@ def test_collapse_onto_the_value_a_lane_does_not_have(hip_module, dtype, lane):
         assert np.all(out[~kept] == 0.)
         assert np.all(out[kept] == 0.) if want == 'zero' else np.all(np.isnan(out[kept].real))
         qs.delete()
+
+
+def _use_lane_again(proc, qs, n, lane, gate, probs):
+    """Measures `lane`, applies `gate` to it, and reads every lane; then collapses `lane` again."""
+    other = (lane + 2) % n
+    for q, want in ((other, 0), (lane, 1), (lane, 0)):   # both outcomes, after an earlier collapse
+        p = proc.calc_probability(qs, q)
+        probs.append(p)
+        proc.decohere(want, p, qs, q)
+        if gate == 'controlled':
+            proc.apply_controlled_gate(gtype.U(0.9, 0.4, 1.3), False, qs, [other], lane)
+            proc.apply_controlled_gate(gtype.U(1.1, 0.2, 0.7), False, qs, [lane], other)
+        proc.apply_gate(gtype.X() if gate == 'X' else gtype.U(1.2, 0.5, 2.1), False, qs, q)
+        probs += [proc.calc_probability(qs, k) for k in range(n)]
+    p = proc.calc_probability(qs, lane)
+    if min(p, 1. - p) > 0.1:
+        proc.decohere(1, p, qs, lane)
+    probs += [proc.calc_probability(qs, k) for k in range(n)]
+
+
+@pytest.mark.parametrize('dtype', [np.float64, np.float32])
+@pytest.mark.parametrize('fusion', ['off', 'tile', 'dense'])
+@pytest.mark.parametrize('gate', ['U', 'X', 'controlled'])
+@pytest.mark.parametrize('lane', [2, 3, 4, 5, 8, 12])
+def test_gate_on_the_lane_just_collapsed(hip_module, port_module, lane, gate, fusion, dtype):
+    """A gate ends what a collapse that is launched together with it made known of its lane."""
+    n, results = 13, []
+    for module, real, read in ((hip_module, dtype, lambda qs: _read(hip_module, qs, n, dtype)),
+                               (port_module, np.float64, lambda qs: qs.local_states())):
+        qs = _prepared(module, n, real, 21)
+        if module is hip_module:
+            qs.processor.set_fusion(fusion)
+        probs = []
+        _use_lane_again(qs.processor, qs, n, lane, gate, probs)
+        results.append((np.array(probs), read(qs)))
+        qs.delete()
+    (gp, g), (wp, w) = results
+    assert np.max(np.abs(gp - wp)) < tol(dtype), (gp, wp)
+    assert np.max(np.abs(g - w)) < tol(dtype)
