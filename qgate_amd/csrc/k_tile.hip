@@ -507,20 +507,18 @@ static void run_register_passes(Cx<R> *a, int n_lanes, const std::vector<QueuedG
     const u64 n_tiles = u64(1) << (n_lanes - M);
     const u64 piece = launch_piece_items() / T;   // keeps every grid within launch_piece_items() threads
     const auto run = [&](const BuiltPass<R> &bp) {
-        // a pass that comes to one gate streams faster than through a tile
+        // a pass that comes to one gate streams faster than through a tile (a parity gate is none of
+        // those that the streaming kernels take: its second lane is no control)
         const RegGate &g0 = gates[bp.gates[0]];
-        bool lone = bp.gates.size() == 1;
+        bool lone = g0.parity < 0 && (g0.ctrl.empty() || bp.gates.size() == 1);
         GateMatrix m = g0.m;
-        if (g0.ctrl.empty() && !lone) {
-            lone = true;
-            for (size_t k = 1; k < bp.gates.size() && lone; ++k) {
-                const RegGate &g = gates[bp.gates[k]];
-                lone = g.ctrl.empty() && g.target == g0.target;
-                GateMatrix p;
-                for (int r = 0; r < 2; ++r)
-                    for (int c = 0; c < 2; ++c) p.m[r][c] = g.m.m[r][0] * m.m[0][c] + g.m.m[r][1] * m.m[1][c];
-                m = p;
-            }
+        for (size_t k = 1; k < bp.gates.size() && lone; ++k) {
+            const RegGate &g = gates[bp.gates[k]];
+            lone = g.parity < 0 && g.ctrl.empty() && g.target == g0.target;
+            GateMatrix p;
+            for (int r = 0; r < 2; ++r)
+                for (int c = 0; c < 2; ++c) p.m[r][c] = g.m.m[r][0] * m.m[0][c] + g.m.m[r][1] * m.m[1][c];
+            m = p;
         }
         if (lone) {
             launch_gate<R>(a, n_lanes, m, g0.ctrl, g0.target);
