@@ -166,9 +166,11 @@ def test_parity_gates_left_to_the_forward_pass(hip_module, dtype, n):
     for controls in ([0], [0, 4, last - 1]):
         results = []
         for mode, real in (('off', np.float64), ('tile', dtype)):
-            c, gates = ParametricCircuit(n, real), last + 1
+            c, gates = ParametricCircuit(n, real), 2 * last
             for q in range(last + 1):
                 c.rx(q, q)
+            for q in range(last - 1):
+                c.gate(np.diag([1, -1]), q + 1, controls=[q])
             for k, a in enumerate(controls):
                 c.gate(X, last, controls=[a])
                 c.rz(last, last + 1 + k)
