@@ -401,7 +401,7 @@ double small_expectation(Cx<R> *psi, Cx<R> *lam, int n_lanes, const std::vector<
     const int m = small_bits<R>(n_lanes);
     SmallTables<R> t;
     plan_small_forward(
-        t, merged_gates((int)gates.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates[i]; }), m,
+        t, merged_gates<R>((int)gates.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates[i]; }), m,
         kGlobalPhase);
     t.ops.push_back(RegOp<R>());   // one more is read than there are
     std::vector<u64> xmask, zmask;

@@ -502,7 +502,7 @@ template <class R, int M, int T>
 static void run_register_passes(Cx<R> *a, int n_lanes, const std::vector<QueuedGate> &gates_in, int low) {
     constexpr int A = (1 << M) / T;
     const std::vector<RegGate> gates =
-        merged_gates((int)gates_in.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates_in[i]; });
+        merged_gates<R>((int)gates_in.size(), n_lanes, [&](int i) -> const QueuedGate & { return gates_in[i]; });
     hipStream_t s = stream();
     const u64 n_tiles = u64(1) << (n_lanes - M);
     const u64 piece = launch_piece_items() / T;   // keeps every grid within launch_piece_items() threads

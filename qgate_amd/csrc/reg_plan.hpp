@@ -7,6 +7,8 @@
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "gate_matrix.hpp"
@@ -57,11 +59,69 @@ inline bool is_x_rotation(const GateMatrix &g) {
            g.m[0][0] == g.m[1][1] && g.m[0][1] == g.m[1][0] && (g.m[0][0] != 0. || g.m[0][1] != 0.);
 }
 
+// A product of gates, rounded to FP64 where a register gate is made of it: T is long double for
+// complex128 states (rounded at every product, a run of 4000 gates was off by 13 2^-53, now 0.4), double
+// for complex64 ones.
+template <class T>
+struct Product {
+    std::complex<T> m[2][2];
+};
+template <class R>
+using ProductOf = typename std::conditional<sizeof(R) == 8, long double, double>::type;
+
+template <class A, class T>
+std::complex<T> times(const std::complex<A> &a, const std::complex<T> &b) {   // (no check for infinities)
+    return std::complex<T>(a.real() * b.real() - a.imag() * b.imag(), a.real() * b.imag() + a.imag() * b.real());
+}
+template <class T>
+std::complex<double> rounded(const std::complex<T> &v) {
+    return std::complex<double>((double)v.real(), (double)v.imag());
+}
+template <class T>
+GateMatrix rounded(const Product<T> &w) {
+    GateMatrix g;
+    for (int r = 0; r < 2; ++r)
+        for (int c = 0; c < 2; ++c) g.m[r][c] = rounded(w.m[r][c]);
+    return g;
+}
+template <class T>
+void widen(const GateMatrix &g, Product<T> &w) {
+    for (int r = 0; r < 2; ++r)
+        for (int c = 0; c < 2; ++c) w.m[r][c] = std::complex<T>(g.m[r][c]);
+}
+template <class T>
+bool diag2(const Product<T> &w) {
+    return w.m[0][1] == T(0) && w.m[1][0] == T(0);
+}
+// a <- b a, in place: copies of extended values cost more than their products
+template <class T>
+void multiply(const GateMatrix &b, Product<T> &a) {
+    typedef std::complex<T> C;
+    if (diag2(a)) {   // what a split has left
+        const C d0 = a.m[0][0], d1 = a.m[1][1];
+        for (int r = 0; r < 2; ++r) {
+            a.m[r][0] = times(b.m[r][0], d0);
+            a.m[r][1] = times(b.m[r][1], d1);
+        }
+        return;
+    }
+    const bool db = diag2(b);
+    for (int c = 0; c < 2; ++c) {
+        const C x = a.m[0][c], y = a.m[1][c];
+        a.m[0][c] = times(b.m[0][0], x);
+        a.m[1][c] = times(b.m[1][1], y);
+        if (db) continue;
+        a.m[0][c] += times(b.m[0][1], y);
+        a.m[1][c] += times(b.m[1][0], x);
+    }
+}
+
 // U = diag(a0, a1) RY diag(1, b) for a unitary U (to FP64 rounding); false for any other. In
 // extended precision and rounded once, so that the factors' moduli are as close to 1 as those of
 // rounded sines and cosines.
-inline bool split_unitary(const GateMatrix &u, std::complex<double> &a0, std::complex<double> &a1,
-                          std::complex<double> &b, GateMatrix &ry) {
+template <class T>
+bool split_unitary(const Product<T> &u, std::complex<T> &a0, std::complex<T> &a1, std::complex<T> &b,
+                   GateMatrix &ry) {
     typedef std::complex<long double> cl;
     const cl m00 = cl(u.m[0][0]), m01 = cl(u.m[0][1]), m10 = cl(u.m[1][0]), m11 = cl(u.m[1][1]);
     const long double tol = 4e-15L;
@@ -78,27 +138,15 @@ inline bool split_unitary(const GateMatrix &u, std::complex<double> &a0, std::co
     };
     const cl p0 = phase(m00), p1 = phase(m10);
     const cl pb = r0 >= r1 ? phase(m11) * std::conj(p1) : -phase(m01) * std::conj(p0);
-    auto rounded = [](const cl &v) { return std::complex<double>((double)v.real(), (double)v.imag()); };
-    a0 = rounded(p0);
-    a1 = rounded(p1);
-    b = rounded(pb);
+    a0 = std::complex<T>((T)p0.real(), (T)p0.imag());
+    a1 = std::complex<T>((T)p1.real(), (T)p1.imag());
+    b = std::complex<T>((T)pb.real(), (T)pb.imag());
     const double c = (double)(r0 / r), s = (double)(r1 / r);
     ry.m[0][0] = c;
     ry.m[0][1] = -s;
     ry.m[1][0] = s;
     ry.m[1][1] = c;
     return true;
-}
-
-inline RegGate diag_gate(std::complex<double> d0, std::complex<double> d1, int target, int source) {
-    RegGate g;
-    g.kind = kGateDiag;
-    g.target = target;
-    g.source = source;
-    g.m.m[0][0] = d0;
-    g.m.m[0][1] = g.m.m[1][0] = 0.;
-    g.m.m[1][1] = d1;
-    return g;
 }
 
 // A diagonal gate with m00 == 0 (or nearly) has no ratio m11 / m00 for the register passes.
@@ -108,6 +156,19 @@ inline bool has_ratio(const GateMatrix &g) {
 }
 
 inline bool trivial_diag(std::complex<double> d0, std::complex<double> d1) { return d0 == 1. && d1 == 1.; }
+
+inline void append_diag(std::vector<RegGate> &out, std::complex<double> d0, std::complex<double> d1, int target,
+                        int source) {
+    if (trivial_diag(d0, d1)) return;
+    RegGate g;
+    g.kind = kGateDiag;
+    g.target = target;
+    g.source = source;
+    g.m.m[0][0] = d0;
+    g.m.m[0][1] = g.m.m[1][0] = 0.;
+    g.m.m[1][1] = d1;
+    out.push_back(std::move(g));
+}
 
 // CX . D . CX with D diagonal on the target (an exp(-i a Z Z / 2), for instance) is D by the parity of
 // control and target: one diagonal gate and no register moves. role[i] is then kDropped for the CX
@@ -138,9 +199,11 @@ std::vector<int> parity_roles(int n_gates, int n_lanes, GateAt gate, IsCx is_cx,
     return role;
 }
 
-// Appends the register gates of one fixed gate (no parameter), in the order they apply.
-inline void append_fixed(std::vector<RegGate> &out, const GateMatrix &m, const std::vector<int> &ctrl, int target,
-                         int source) {
+// Appends the register gates of one fixed gate (no parameter), in the order they apply. exact: m before
+// it was rounded, if it is a product.
+template <class T = double>
+void append_fixed(std::vector<RegGate> &out, const GateMatrix &m, const std::vector<int> &ctrl, int target,
+                  int source, const Product<T> *exact = nullptr) {
     RegGate g;
     g.target = target;
     g.source = source;
@@ -148,12 +211,12 @@ inline void append_fixed(std::vector<RegGate> &out, const GateMatrix &m, const s
     g.m = m;
     if (diag2(m) && has_ratio(m)) {
         g.kind = kGateDiag;
-        if (!trivial_diag(m.m[0][0], m.m[1][1])) out.push_back(g);
+        if (!trivial_diag(m.m[0][0], m.m[1][1])) out.push_back(std::move(g));
         return;
     }
     if (is_x(m)) {
         g.kind = kGateSwap;
-        out.push_back(g);
+        out.push_back(std::move(g));
         return;
     }
     if (ctrl.empty()) {
@@ -162,47 +225,54 @@ inline void append_fixed(std::vector<RegGate> &out, const GateMatrix &m, const s
             out.push_back(g);
             return;
         }
-        std::complex<double> a0, a1, b;
-        GateMatrix ry;
-        if (split_unitary(m, a0, a1, b, ry)) {
-            if (!trivial_diag(1., b)) out.push_back(diag_gate(1., b, target, source));
+        Product<T> u;
+        if (exact == nullptr) {
+            widen(m, u);
+            exact = &u;
+        }
+        std::complex<T> a0, a1, b;
+        if (split_unitary(*exact, a0, a1, b, g.m)) {
+            append_diag(out, 1., rounded(b), target, source);
             g.kind = kGateY;
-            g.m = ry;
             out.push_back(g);
-            if (!trivial_diag(a0, a1)) out.push_back(diag_gate(a0, a1, target, source));
+            append_diag(out, rounded(a0), rounded(a1), target, source);
             return;
         }
     }
     g.kind = kGateAny;
-    out.push_back(g);
+    out.push_back(std::move(g));
 }
 
 // The register gates of a gate list whose matrices are all known. The uncontrolled gates of a lane
-// between controlled ones multiply into one (in FP64); of its split diag . RY . diag the last
-// diagonal waits for the lane's next gate where what comes between acts diagonally on the lane.
-// gate(i) has m, ctrl and target.
-template <class GateAt>
+// between controlled ones multiply into one; of its split diag . RY . diag the last diagonal waits for
+// the lane's next gate where what comes between acts diagonally on the lane.
+// gate(i) has m, ctrl and target; R: the precision of the state.
+template <class R, class GateAt>
 std::vector<RegGate> merged_gates(int n_gates, int n_lanes, GateAt gate) {
     std::vector<RegGate> out;
     out.reserve((size_t)n_gates * 2);
-    std::vector<GateMatrix> run(n_lanes);
+    typedef ProductOf<R> T;
+    std::vector<Product<T>> run(n_lanes);
     std::vector<int> last(n_lanes, -1);   // source of the lane's run, -1: none
     const std::vector<int> role = parity_roles(
         n_gates, n_lanes, gate, [&](int i) { return gate(i).ctrl.size() == 1 && is_x(gate(i).m); },
         [&](int i) { return gate(i).ctrl.empty() && diag2(gate(i).m) && has_ratio(gate(i).m); });
     auto emit = [&](int lane, bool keep_diagonal) {
         if (last[lane] < 0) return;
-        GateMatrix &m = run[lane];
-        if (keep_diagonal && diag2(m)) return;
-        std::complex<double> a0, a1, b;
+        Product<T> &w = run[lane];
+        if (keep_diagonal && diag2(w)) return;
+        const GateMatrix m = rounded(w);
+        std::complex<T> a0, a1, b;
         GateMatrix ry;
-        if (keep_diagonal && !is_x(m) && !is_y_rotation(m) && !is_x_rotation(m) && split_unitary(m, a0, a1, b, ry)) {
-            append_fixed(out, diag_gate(1., b, lane, last[lane]).m, {}, lane, last[lane]);
+        if (keep_diagonal && !is_x(m) && !is_y_rotation(m) && !is_x_rotation(m) && split_unitary(w, a0, a1, b, ry)) {
+            append_diag(out, 1., rounded(b), lane, last[lane]);
             append_fixed(out, ry, {}, lane, last[lane]);
-            m = diag_gate(a0, a1, lane, last[lane]).m;
+            w.m[0][0] = a0;
+            w.m[0][1] = w.m[1][0] = T(0);
+            w.m[1][1] = a1;
             return;
         }
-        append_fixed(out, m, {}, lane, last[lane]);
+        append_fixed(out, m, {}, lane, last[lane], &w);
         last[lane] = -1;
     };
     for (int i = 0; i < n_gates; ++i) {
@@ -217,15 +287,10 @@ std::vector<RegGate> merged_gates(int n_gates, int n_lanes, GateAt gate) {
             continue;
         }
         if (g.ctrl.empty()) {
-            GateMatrix &m = run[g.target];
-            if (last[g.target] < 0) {
-                m = g.m;
-            } else {
-                GateMatrix p;
-                for (int r = 0; r < 2; ++r)
-                    for (int c = 0; c < 2; ++c) p.m[r][c] = g.m.m[r][0] * m.m[0][c] + g.m.m[r][1] * m.m[1][c];
-                m = p;
-            }
+            if (last[g.target] < 0)
+                widen(g.m, run[g.target]);
+            else
+                multiply(g.m, run[g.target]);
             last[g.target] = i;
             continue;
         }

@@ -70,3 +70,36 @@ def test_ops_on_every_kind_of_bit(hip_module, dtype, n, unitary):
     if unitary:   # the sweep un-computes with U^dagger
         terms = 4 * 2 * n / len(ANGLES)
         assert np.max(np.abs(g1 - g0)) < tol * terms * np.sum(np.abs(h.coefs))
+
+
+@pytest.mark.parametrize('diagonals', [False, True])
+def test_a_run_on_one_lane_rounds_once(hip_module, diagonals):
+    """4000 gates on one lane, in complex128, become one gate whose product is formed in extended
+    precision: its amplitudes are off by the roundings of that gate's parts (a diagonal, a rotation, a
+    diagonal, their product and its application, at most 2^-53 each and two components: 12 of them),
+    not by those of 4000 products (13 and 14 2^-53 when each was rounded). Up to norm and phase, which the split drops from
+    matrices that are rounded themselves."""
+    from tests.test_dense_fusion import _read
+    rs = np.random.RandomState(3)
+    n, lane = 14, 9
+    qs = hip_module.create_qubit_states(np.float64)
+    proc = qs.processor
+    proc.set_fusion('tile')
+    proc.initialize_qubit_states(qs, n)
+    proc.reset_qubit_states(qs)
+    want = np.array([1, 0], np.clongdouble)
+    for k in range(4000):
+        t = rs.uniform(-3, 3)
+        m = np.array([[math.cos(t), -math.sin(t)], [math.sin(t), math.cos(t)]], complex)
+        if diagonals and k % 2:
+            m = np.diag([_e(-t), _e(t)])
+        proc.apply_matrix(m, qs, [], lane)
+        want = m.astype(np.clongdouble) @ want
+    out = _read(hip_module, qs, n, np.float64)
+    qs.delete()
+    got = out[[0, 1 << lane]].astype(np.clongdouble)
+    got, want = (v / np.sqrt(np.sum(np.abs(v) ** 2)) for v in (got, want))
+    phase = np.sum(np.conj(want) * got)
+    error = float(np.sqrt(np.sum(np.abs(got - want * phase / np.abs(phase)) ** 2))) * 2. ** 53
+    print('error', error)
+    assert error < 12
