@@ -45,18 +45,24 @@ inline bool is_x(const GateMatrix &g) {
 
 inline bool diag2(const GateMatrix &g) { return g.m[0][1] == 0. && g.m[1][0] == 0.; }
 
+// Far from a unitary matrix's entries, quotients of entries and squares of them can leave the range of a
+// state's numbers where the entries themselves are within it: such gates take the general update.
+inline bool moderate(double a) { return a > 1e-6 && a < 1e6; }
+
 // [[c, -s], [s, c]] with real entries, exactly
 inline bool is_y_rotation(const GateMatrix &g) {
     for (int r = 0; r < 2; ++r)
         for (int c = 0; c < 2; ++c)
             if (g.m[r][c].imag() != 0.) return false;
-    return g.m[0][0] == g.m[1][1] && g.m[0][1] == -g.m[1][0] && (g.m[0][0] != 0. || g.m[0][1] != 0.);
+    return g.m[0][0] == g.m[1][1] && g.m[0][1] == -g.m[1][0] &&
+           moderate(std::max(std::abs(g.m[0][0].real()), std::abs(g.m[0][1].real())));
 }
 
 // [[c, -i s], [-i s, c]], exactly
 inline bool is_x_rotation(const GateMatrix &g) {
     return g.m[0][0].imag() == 0. && g.m[1][1].imag() == 0. && g.m[0][1].real() == 0. && g.m[1][0].real() == 0. &&
-           g.m[0][0] == g.m[1][1] && g.m[0][1] == g.m[1][0] && (g.m[0][0] != 0. || g.m[0][1] != 0.);
+           g.m[0][0] == g.m[1][1] && g.m[0][1] == g.m[1][0] &&
+           moderate(std::max(std::abs(g.m[0][0].real()), std::abs(g.m[0][1].imag())));
 }
 
 // A product of gates, rounded to FP64 where a register gate is made of it: T is long double for
@@ -149,10 +155,10 @@ bool split_unitary(const Product<T> &u, std::complex<T> &a0, std::complex<T> &a1
     return true;
 }
 
-// A diagonal gate with m00 == 0 (or nearly) has no ratio m11 / m00 for the register passes.
+// Whether a diagonal gate can be applied as m00 and the ratio m11 / m00.
 inline bool has_ratio(const GateMatrix &g) {
-    const double a = std::abs(g.m[0][0]);
-    return a > 1e-30 && a < 1e30;
+    const double b = std::abs(g.m[1][1]);
+    return moderate(std::abs(g.m[0][0])) && (b == 0. || moderate(b));
 }
 
 inline bool trivial_diag(std::complex<double> d0, std::complex<double> d1) { return d0 == 1. && d1 == 1.; }

@@ -103,3 +103,37 @@ def test_a_run_on_one_lane_rounds_once(hip_module, diagonals):
     error = float(np.sqrt(np.sum(np.abs(got - want * phase / np.abs(phase)) ** 2))) * 2. ** 53
     print('error', error)
     assert error < 12
+
+
+FAR = {
+    'ratio': np.diag([2e-30, 1e9]), 'small': np.diag([1e-25, 1e25j]), 'large': np.diag([1e20j, 1e-15]),
+    'ry': 1e-25 * np.array([[0.8, -0.6], [0.6, 0.8]]), 'rx': 1e18 * np.array([[0.6, -0.8j], [-0.8j, 0.6]]),
+}
+FAR_DOUBLE = {   # squares and quotients beyond the range of FP64 itself
+    'ratio64': np.diag([1e-25, 1e290]), 'ry64': 1e-200 * np.array([[0.8, -0.6], [0.6, 0.8]]),
+    'rx64': 1e200 * np.array([[0.6, -0.8j], [-0.8j, 0.6]]),
+}
+
+
+@pytest.mark.parametrize('dtype,name', [(np.float32, m) for m in sorted(FAR)] +
+                         [(np.float64, m) for m in sorted({**FAR, **FAR_DOUBLE})])
+@pytest.mark.parametrize('controls', [0, 1])
+def test_matrices_far_from_unitary(hip_module, dtype, name, controls):
+    """Entries that the state's precision holds give the amplitudes that the gate-by-gate path gives,
+    each within 32 eps, though their quotient or their squares leave its range."""
+    from tests.test_dense_fusion import _prepared, _read
+    n, m = 14, {**FAR, **FAR_DOUBLE}[name]
+    h = FIXED['h']
+    for target in (0, 5, 9, 13):
+        out = []
+        for mode in ('off', 'tile'):
+            qs = _prepared(hip_module, n, dtype, 4)
+            qs.processor.set_fusion(mode)
+            for mat, ctrl, q in ((h, [], 3), (m, [7] * controls, target), (h, [], 4)):
+                qs.processor.apply_matrix(mat, qs, ctrl, q)
+            out.append(_read(hip_module, qs, n, dtype))
+            qs.delete()
+        off, tile = out
+        assert np.all(np.isfinite(off.view(np.float64)))
+        scale = np.max(np.abs(off).reshape(-1, 4, 8), 1)   # of the amplitudes that the H gates mix
+        assert np.max(np.abs(tile - off).reshape(-1, 4, 8) / scale[:, None]) < 32 * np.finfo(dtype).eps
