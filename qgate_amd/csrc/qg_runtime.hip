@@ -38,10 +38,12 @@ namespace {
 constexpr size_t kCacheMaxBlock = size_t(1) << 30;   // power-of-two classes up to 1 GiB
 constexpr size_t kCacheMaxTotal = size_t(8) << 30;   // keep at most 8 GiB of those cached
 // Larger blocks (state vectors and pools of 27 and more qubits) are kept in sizes of whole
-// 2 MiB, at most 8 GiB of them, the oldest given up first. While they went back to the driver
-// at each free, a 28-qubit pool (2 GiB) built again and again, with draws and a marginal, took
-// 67.8 ms a time, 66 of them in the driver's allocation and free; kept, 1.64 ms.
-constexpr size_t kLargeMaxTotal = size_t(8) << 30;
+// 2 MiB, the oldest given up first, as far as all kept blocks stay within the same 8 GiB (another
+// allocator of the process, torch's, cannot ask for them back) and 256 MiB, for the tables and
+// partial sums beside an 8 GiB state. While they went back to the driver at each free, a
+// 28-qubit pool (2 GiB) built again and again, with draws and a marginal, took 67.8 ms a time, 66
+// of them in the driver's allocation and free; kept, 1.64 ms.
+constexpr size_t kKeptMax = kCacheMaxTotal + (size_t(256) << 20);
 constexpr size_t kLargeGrain = size_t(2) << 20;
 
 std::map<size_t, std::vector<void *>> &free_lists() {
@@ -65,6 +67,18 @@ size_t size_class(size_t bytes) {
     size_t c = 256;
     while (c < bytes) c <<= 1;
     return c;
+}
+
+// Gives the oldest large blocks back until all kept blocks are within kKeptMax.
+void trim_large() {
+    if (g_cached + g_large_cached <= kKeptMax) return;
+    QG_HIP(hipStreamSynchronize(runtime().stream));   // queued kernels may still read them
+    while (g_cached + g_large_cached > kKeptMax && !large_blocks().empty()) {
+        const LargeBlock old = large_blocks().front();
+        large_blocks().erase(large_blocks().begin());
+        g_large_cached -= old.bytes;
+        QG_HIP(hipFree(old.ptr));
+    }
 }
 
 void release_cache() {
@@ -329,22 +343,16 @@ void dev_free(void *ptr, size_t bytes) {
     if (bytes <= kCacheMaxBlock && g_cached + bytes <= kCacheMaxTotal) {
         free_lists()[bytes].push_back(ptr);
         g_cached += bytes;
+        trim_large();
         return;
     }
-    // a block that goes back to the driver may still be read by queued kernels
-    if (bytes > kCacheMaxBlock && bytes <= kLargeMaxTotal) {
-        std::vector<LargeBlock> &large = large_blocks();
-        if (g_large_cached + bytes > kLargeMaxTotal) QG_HIP(hipStreamSynchronize(rt.stream));
-        while (g_large_cached + bytes > kLargeMaxTotal) {
-            const LargeBlock old = large.front();
-            large.erase(large.begin());
-            g_large_cached -= old.bytes;
-            QG_HIP(hipFree(old.ptr));
-        }
-        large.push_back(LargeBlock{ptr, bytes});
+    if (bytes > kCacheMaxBlock && g_cached + bytes <= kKeptMax) {
+        large_blocks().push_back(LargeBlock{ptr, bytes});
         g_large_cached += bytes;
+        trim_large();
         return;
     }
+    // the block may still be read by queued kernels: drain the stream first
     QG_HIP(hipStreamSynchronize(rt.stream));
     QG_HIP(hipFree(ptr));
 }

@@ -34,7 +34,7 @@ hipStream_t stream();
 void sync();
 
 // Device allocations: power-of-two size classes up to 1 GiB (at most 8 GiB of them), and larger
-// blocks by their size in 2 MiB steps (at most 8 GiB of those), are cached after free and
+// blocks by their size in 2 MiB steps (as far as these 8 GiB last), are cached after free and
 // reused without a device synchronisation (all users share the one stream, so reuse is
 // stream-ordered). An allocation that fails gives the whole cache back and tries again.
 void *dev_alloc(size_t bytes);

@@ -1,6 +1,7 @@
 """Device blocks above 1 GiB are kept after free, reused by size, and bounded at 8 GiB."""
 import ctypes
 import gc
+import time
 
 import numpy as np
 import pytest
@@ -48,3 +49,25 @@ def test_large_blocks_are_reused_and_bounded(hip_module, sizes):
     assert given_back - free_before <= 2 * LARGE_MAX + GIB
     fits = [16 << n for n in sizes if (16 << n) <= LARGE_MAX]
     assert given_back - free_before >= min(max(fits), LARGE_MAX) - GIB // 2
+
+
+@pytest.mark.parametrize('order', ['small first', 'large first'])
+def test_one_bound_for_blocks_of_all_sizes(hip_module, order):
+    """After 7 GiB of complex128 states of 26 qubits (1 GiB, a power-of-two class) and 6 GiB of 27 and 28
+    (large blocks) are freed, all that stays is 8 GiB and 256 MiB; what another allocator may take."""
+    gc.collect()
+    hip_module.module_finalize()
+    hip_module.module_init()
+    keep = _state(hip_module, 4)
+    before = _free_bytes(hip_module)
+    small, large = [_state(hip_module, 26) for _ in range(7)], [_state(hip_module, n) for n in (27, 28)]
+    for qs in small + large if order == 'small first' else large + small:
+        qs.delete()
+    for _ in range(50):                      # the driver takes freed memory back with a delay
+        kept = before - _free_bytes(hip_module)
+        print(order, kept / GIB)
+        if kept <= LARGE_MAX + GIB // 2:
+            break
+        time.sleep(0.1)
+    assert kept <= LARGE_MAX + GIB // 2 and kept >= 7 * GIB - GIB // 2
+    keep.delete()
