@@ -493,6 +493,8 @@ template void small_sweep<double>(const Cx<double> *, const Cx<double> *, int, c
 
 // ---- batch ---------------------------------------------------------------------------------
 
+SmallBatch::~SmallBatch() { dev_free_quiet(block_, bytes_); }
+
 void SmallBatch::clear() {
     if (block_ != nullptr) dev_free(block_, bytes_);
     block_ = nullptr;

@@ -628,7 +628,7 @@ class SweepRows {
         bytes_ = o_part_ + std::max<size_t>(8, row_bytes * (size_t)cap_);
         buf_ = static_cast<char *>(dev_alloc(bytes_));
     }
-    ~SweepRows() { dev_free(buf_, bytes_); }
+    ~SweepRows() { dev_free_quiet(buf_, bytes_); }
     char *tables() const { return buf_; }
     // rows of the next pass; sums the pending ones first if it would not fit
     double *rows(int n_slots, const int *d_slot_gate, double *d_terms) {

@@ -357,6 +357,13 @@ void dev_free(void *ptr, size_t bytes) {
     QG_HIP(hipFree(ptr));
 }
 
+void dev_free_quiet(void *ptr, size_t bytes) noexcept {
+    try {
+        dev_free(ptr, bytes);
+    } catch (...) {
+    }
+}
+
 size_t dev_cached_bytes() { return g_cached + g_large_cached; }
 
 }  // namespace qg

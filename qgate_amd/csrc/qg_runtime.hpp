@@ -39,6 +39,9 @@ void sync();
 // stream-ordered). An allocation that fails gives the whole cache back and tries again.
 void *dev_alloc(size_t bytes);
 void dev_free(void *ptr, size_t bytes);
+// dev_free for destructors: an error of the device (the next call reports it too) is not thrown,
+// which would end the process where one is already on its way.
+void dev_free_quiet(void *ptr, size_t bytes) noexcept;
 size_t dev_cached_bytes();
 
 // Grid size that fills the device for grid-stride reductions.

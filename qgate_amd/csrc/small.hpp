@@ -40,7 +40,7 @@ class SmallBatch {
     SmallBatch() = default;
     SmallBatch(const SmallBatch &) = delete;
     SmallBatch &operator=(const SmallBatch &) = delete;
-    ~SmallBatch() { clear(); }
+    ~SmallBatch();
     void clear();
     template <class R>
     void build(const std::vector<SmallGroupIn> &groups);
