@@ -52,7 +52,7 @@ class SmallBatch {
     void download();
     const double *values(int k) const { return host_.data() + value_at_[k]; }
     const double *grads(int k) const { return host_.data() + grad_at_[k]; }
-    int sweep_passes(int k) const { return passes_[k]; }
+    int sweep_passes(int k) const { return k < (int)passes_.size() ? passes_[k] : 0; }   // 0: not built
 
   private:
     struct Launch {          // one width of workgroup
