@@ -1081,8 +1081,9 @@ double time_group(Group &g, int reps) {
 // two stages. First the tile shape: register-resident passes (full-size tiles; groups of at
 // least the sweep tile's qubit count) and LDS passes of up to three tile sizes, at 256
 // threads and 4 workgroups per compute unit. Then, for the fastest shape, the workgroup size
-// and persistent grid of the LDS passes (every group has Pauli passes in LDS). Knobs fixed
-// by qghip_batch_set_tuning are not searched.
+// and persistent grid of its LDS passes, if it has any: forward and sweep in registers with Pauli
+// sums on full-size tiles have none, and the candidates would all be the same. Knobs fixed by
+// qghip_batch_set_tuning are not searched.
 template <class R>
 void tune_group(qghip_batch *b, Group &g) {
     typedef BCfg<R> C;
@@ -1124,6 +1125,7 @@ void tune_group(qghip_batch *b, Group &g) {
     sample.coefs.assign(g.coefs.begin(), g.coefs.begin() + keep * g.zmask.size() * 2);
     Tuning best;
     best.ms = -1.;
+    bool best_lds = true;
     auto try_tuning = [&](int tb, int rg, int th, int gr) {
         Tuning t;
         t.tile_bits = tb;
@@ -1132,14 +1134,18 @@ void tune_group(qghip_batch *b, Group &g) {
         t.grid_per_cu = gr;
         build_group<R>(sample, t);
         t.ms = time_group<R>(sample, 2);
-        if (best.ms < 0. || t.ms < best.ms) best = t;
+        if (best.ms < 0. || t.ms < best.ms) {
+            best = t;
+            best_lds = !(sample.fregs && sample.sregs && sample.pauli_full);
+        }
     };
     try {
         for (const auto &sh : shapes) try_tuning(sh.first, sh.second, threads[0], grids[0]);
         const Tuning shape = best;
-        for (int th : threads)
-            for (int gr : grids)
-                if (th != threads[0] || gr != grids[0]) try_tuning(shape.tile_bits, shape.registers, th, gr);
+        if (best_lds)
+            for (int th : threads)
+                for (int gr : grids)
+                    if (th != threads[0] || gr != grids[0]) try_tuning(shape.tile_bits, shape.registers, th, gr);
     } catch (...) {
         free_group(sample);
         throw;

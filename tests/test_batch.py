@@ -210,3 +210,15 @@ def test_batch_argument_errors(hip_module):
         batch.set_tuning(13, 0, 0)
     with pytest.raises(ValueError):
         batch.set_tuning(registers=2)
+
+
+@pytest.mark.parametrize('dtype', DTYPES)
+def test_groups_without_lds_passes_have_nothing_to_tune(hip_module, dtype):
+    """Register passes on full-size tiles use neither knob of the LDS passes: they stay at the first
+    candidates, and no timing noise picks others."""
+    batch, circuits, items = _hea_batch(dtype, [14, 14, 15, 16, 17], 1, seed=9)
+    batch.set_tuning(registers=1)
+    _check(batch.run(), circuits, items, dtype)
+    for g in batch.tuning:
+        assert (g['forward_in_registers'], g['sweep_in_registers']) == (1, 1)
+        assert (g['threads'], g['grid_per_cu']) == (256, 4)
