@@ -877,7 +877,7 @@ void build_group(Group &g, const Tuning &t) {
     const size_t o_terms = carve(sizeof(double) * ni * std::max(1, n_gates));
     const size_t o_values = carve(sizeof(double) * ni);
     const size_t o_grads = carve(sizeof(double) * ni * std::max(1, g.n_params));
-    const size_t o_mats = carve(sizeof(BMats<R>) * ni * std::max(1, n_gates));
+    const size_t o_mats = carve(fregs && sregs ? 0 : sizeof(BMats<R>) * ni * std::max(1, n_gates));   // LDS passes
     const size_t o_gates = carve(sizeof(BGate) * gates.size());
     const size_t o_fops = carve(sizeof(BOp) * fops.size());
     const size_t o_sops = carve(sizeof(BOp) * sops.size());
