@@ -71,7 +71,7 @@ constexpr int kMaxPhases = 24;
 // Bit layout of one register phase, packed in dwords so that a phase read at a runtime
 // index takes scalar loads (a byte array read at a runtime index would be a vector load,
 // whose wait also waits for HBM traffic in flight). Byte k of `bits` is the local bit of
-// register bit k (k < 5), of lane bit k - 5 (5 <= k < 11) or of wave bit k - 11 (k < 14).
+// register bit k (k < 5), of lane bit k - 5 (5 <= k < 11) or of wave bit k - 11 (k < 16).
 struct PhaseBits {
     unsigned bits[4];
     int op_begin, n_ops;   // ops of the pass
@@ -1011,6 +1011,7 @@ __global__ __launch_bounds__(T) void k_tile_sweep_reg(Cx<R> *__restrict__ phi, C
 
 // Packed form of a phase layout (ops [begin, begin + n) of its pass).
 inline PhaseBits phase_bits(const PhasePlan &P, int begin, int n) {
+    QG_REQUIRE(P.regs.size() <= 5 && P.lanes.size() <= 6 && P.waves.size() <= 5, "register phase: too many bits");
     PhaseBits h;
     std::memset(&h, 0, sizeof(h));
     for (int b = 0; b < (int)P.regs.size(); ++b) h.set(b, P.regs[b]);
