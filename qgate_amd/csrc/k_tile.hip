@@ -112,14 +112,14 @@ void set_pauli(GateMatrix &g, int pauli) {
     }
 }
 
-// Register tiles of the single-circuit passes on states of kWideLanes lanes or more: one bit
-// wider than the LDS-pass tiles (64 KiB), 512-thread workgroups with 16 (complex64) / 8
-// (complex128) amplitudes a thread, so the registers per thread are those of the 32 KiB tiles
-// (two workgroups share a compute unit's LDS). A pass then carries the gates of one more
-// target bit: the 2000-gate 30-qubit random circuit takes 123 passes instead of 144, and its
-// step 499 ms instead of 507 (complex64), 991 ms instead of 1034 (complex128). On a
-// 24-qubit state the narrower tiles are faster (an 864-gate circuit 3.74 ms against 4.07).
-constexpr int kWideLanes = 28;
+// Register tiles one bit wider than the default ones (64 KiB), for callers that ask for them by
+// width: 512-thread workgroups with 16 (complex64) / 8 (complex128) amplitudes a thread, so the
+// registers per thread are those of the 32 KiB tiles (two workgroups share a compute unit's LDS). A
+// pass then carries the gates of one more target bit, and costs more than it saves: passes are bound
+// by instruction issue, and 256-thread workgroups wait less at the hand-overs. Wide against
+// default tiles, random circuits: 30 qubits, 2000 gates complex64 327 ms in 59 passes of 5.45 ms
+// against 316 in 69 of 4.45, complex128 657 against 624; 500 gates 86.4 against 82.5; 32 qubits, 500
+// gates 354 against 326; 28 qubits 38.9 against 37.1, 24 qubits 5.3 against 5.2.
 template <class R>
 struct WideCfg;
 template <>
@@ -540,8 +540,7 @@ template <class R>
 void apply_gate_sequence(Cx<R> *a, int n_lanes, const std::vector<QueuedGate> &gates_in, int max_bits,
                          int low_bits) {
     typedef TileCfg<R> C;
-    // wide tiles by default from kWideLanes lanes up, on any state when asked for by width
-    const bool wide = use_register_tiles() && (n_lanes >= kWideLanes || max_bits > C::MaxBits);
+    const bool wide = use_register_tiles() && max_bits > C::MaxBits;
     const int cap = wide ? WideCfg<R>::Bits : C::MaxBits;
     const int mb = std::min(max_bits > 0 ? std::min(max_bits, cap) : cap, n_lanes);
     const int low = std::min(low_bits >= 0 ? low_bits : C::Low, mb);
