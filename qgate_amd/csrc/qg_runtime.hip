@@ -35,60 +35,56 @@ std::string &last_error() {
 
 namespace {
 
-constexpr size_t kCacheMaxBlock = size_t(1) << 30;   // power-of-two classes up to 1 GiB
-constexpr size_t kCacheMaxTotal = size_t(8) << 30;   // keep at most 8 GiB of those cached
-// Larger blocks (state vectors and pools of 27 and more qubits) are kept in sizes of whole
-// 2 MiB, the oldest given up first, as far as all kept blocks stay within the same 8 GiB (another
+// Blocks are kept after free, by size: power-of-two classes up to 1 GiB, larger ones (state vectors
+// and pools of 27 and more qubits) in whole 2 MiB. All of them together stay within 8 GiB (another
 // allocator of the process, torch's, cannot ask for them back) and 256 MiB, for the tables and
-// partial sums beside an 8 GiB state. While they went back to the driver at each free, a
-// 28-qubit pool (2 GiB) built again and again, with draws and a marginal, took 67.8 ms a time, 66
-// of them in the driver's allocation and free; kept, 1.64 ms.
-constexpr size_t kKeptMax = kCacheMaxTotal + (size_t(256) << 20);
+// partial sums beside an 8 GiB state; the block that has been free for longest goes first, so that
+// neither size crowds out the other. While large blocks went back to the driver at each free, a
+// 28-qubit pool (2 GiB) built again and again, with draws and a marginal, took 67.8 ms a time, 66 of
+// them in the driver's allocation and free; kept, 1.64 ms.
+constexpr size_t kClassMax = size_t(1) << 30;
 constexpr size_t kLargeGrain = size_t(2) << 20;
+constexpr size_t kKeptMax = (size_t(8) << 30) + (size_t(256) << 20);
 
-std::map<size_t, std::vector<void *>> &free_lists() {
-    static std::map<size_t, std::vector<void *>> lists;
+struct Kept {
+    void *ptr;
+    u64 freed;   // counts up
+};
+std::map<size_t, std::vector<Kept>> &free_lists() {   // each list oldest first
+    static std::map<size_t, std::vector<Kept>> lists;
     return lists;
 }
 size_t g_cached = 0;
-
-struct LargeBlock {
-    void *ptr;
-    size_t bytes;
-};
-std::vector<LargeBlock> &large_blocks() {   // oldest first
-    static std::vector<LargeBlock> blocks;
-    return blocks;
-}
-size_t g_large_cached = 0;
+u64 g_frees = 0;
 
 size_t size_class(size_t bytes) {
-    if (bytes > kCacheMaxBlock) return (bytes + kLargeGrain - 1) / kLargeGrain * kLargeGrain;
+    if (bytes > kClassMax) return (bytes + kLargeGrain - 1) / kLargeGrain * kLargeGrain;
     size_t c = 256;
     while (c < bytes) c <<= 1;
     return c;
 }
 
-// Gives the oldest large blocks back until all kept blocks are within kKeptMax.
-void trim_large() {
-    if (g_cached + g_large_cached <= kKeptMax) return;
+// Gives the oldest blocks back until all kept ones are within kKeptMax.
+void trim_cache() {
+    if (g_cached <= kKeptMax) return;
     QG_HIP(hipStreamSynchronize(runtime().stream));   // queued kernels may still read them
-    while (g_cached + g_large_cached > kKeptMax && !large_blocks().empty()) {
-        const LargeBlock old = large_blocks().front();
-        large_blocks().erase(large_blocks().begin());
-        g_large_cached -= old.bytes;
-        QG_HIP(hipFree(old.ptr));
+    while (g_cached > kKeptMax) {
+        auto oldest = free_lists().end();
+        for (auto it = free_lists().begin(); it != free_lists().end(); ++it)
+            if (oldest == free_lists().end() || it->second.front().freed < oldest->second.front().freed) oldest = it;
+        void *p = oldest->second.front().ptr;
+        g_cached -= oldest->first;
+        oldest->second.erase(oldest->second.begin());
+        if (oldest->second.empty()) free_lists().erase(oldest);
+        QG_HIP(hipFree(p));
     }
 }
 
 void release_cache() {
     for (auto &kv : free_lists())
-        for (void *p : kv.second) hipFree(p);
+        for (const Kept &k : kv.second) hipFree(k.ptr);
     free_lists().clear();
     g_cached = 0;
-    for (const LargeBlock &b : large_blocks()) hipFree(b.ptr);
-    large_blocks().clear();
-    g_large_cached = 0;
 }
 
 }  // namespace
@@ -300,23 +296,13 @@ void *dev_alloc(size_t bytes) {
     Runtime &rt = runtime();
     std::lock_guard<std::recursive_mutex> lk(rt.mtx);
     bytes = size_class(bytes);
-    if (bytes <= kCacheMaxBlock) {
-        auto it = free_lists().find(bytes);
-        if (it != free_lists().end() && !it->second.empty()) {
-            void *p = it->second.back();
-            it->second.pop_back();
-            g_cached -= bytes;
-            return p;
-        }
-    } else {
-        std::vector<LargeBlock> &large = large_blocks();
-        for (size_t i = large.size(); i-- > 0;) {
-            if (large[i].bytes != bytes) continue;
-            void *p = large[i].ptr;
-            large.erase(large.begin() + i);
-            g_large_cached -= bytes;
-            return p;
-        }
+    auto it = free_lists().find(bytes);
+    if (it != free_lists().end()) {
+        void *p = it->second.back().ptr;
+        it->second.pop_back();
+        if (it->second.empty()) free_lists().erase(it);
+        g_cached -= bytes;
+        return p;
     }
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
@@ -340,16 +326,10 @@ void dev_free(void *ptr, size_t bytes) {
     std::lock_guard<std::recursive_mutex> lk(rt.mtx);
     if (bytes == 0) bytes = 1;
     bytes = size_class(bytes);
-    if (bytes <= kCacheMaxBlock && g_cached + bytes <= kCacheMaxTotal) {
-        free_lists()[bytes].push_back(ptr);
+    if (bytes <= kKeptMax) {
+        free_lists()[bytes].push_back(Kept{ptr, ++g_frees});
         g_cached += bytes;
-        trim_large();
-        return;
-    }
-    if (bytes > kCacheMaxBlock && g_cached + bytes <= kKeptMax) {
-        large_blocks().push_back(LargeBlock{ptr, bytes});
-        g_large_cached += bytes;
-        trim_large();
+        trim_cache();
         return;
     }
     // the block may still be read by queued kernels: drain the stream first
@@ -364,6 +344,6 @@ void dev_free_quiet(void *ptr, size_t bytes) noexcept {
     }
 }
 
-size_t dev_cached_bytes() { return g_cached + g_large_cached; }
+size_t dev_cached_bytes() { return g_cached; }
 
 }  // namespace qg

@@ -33,10 +33,10 @@ void runtime_clear();
 hipStream_t stream();
 void sync();
 
-// Device allocations: power-of-two size classes up to 1 GiB (at most 8 GiB of them), and larger
-// blocks by their size in 2 MiB steps (as far as these 8 GiB last), are cached after free and
-// reused without a device synchronisation (all users share the one stream, so reuse is
-// stream-ordered). An allocation that fails gives the whole cache back and tries again.
+// Device allocations: blocks are cached after free by size (power-of-two classes up to 1 GiB, whole
+// 2 MiB above), at most 8.25 GiB of them, and reused without a device synchronisation (all users
+// share the one stream, so reuse is stream-ordered). An allocation that fails gives the whole cache
+// back and tries again.
 void *dev_alloc(size_t bytes);
 void dev_free(void *ptr, size_t bytes);
 // dev_free for destructors: an error of the device (the next call reports it too) is not thrown,

@@ -54,7 +54,8 @@ def test_large_blocks_are_reused_and_bounded(hip_module, sizes):
 @pytest.mark.parametrize('order', ['small first', 'large first'])
 def test_one_bound_for_blocks_of_all_sizes(hip_module, order):
     """After 7 GiB of complex128 states of 26 qubits (1 GiB, a power-of-two class) and 6 GiB of 27 and 28
-    (large blocks) are freed, all that stays is 8 GiB and 256 MiB; what another allocator may take."""
+    (large blocks) are freed, all that stays is 8 GiB and 256 MiB; what another allocator may take.
+    What was freed last is there again: neither size crowds out the other."""
     gc.collect()
     hip_module.module_finalize()
     hip_module.module_init()
@@ -70,4 +71,7 @@ def test_one_bound_for_blocks_of_all_sizes(hip_module, order):
             break
         time.sleep(0.1)
     assert kept <= LARGE_MAX + GIB // 2 and kept >= 7 * GIB - GIB // 2
-    keep.delete()
+    again = [_state(hip_module, 28)] if order == 'small first' else [_state(hip_module, 26) for _ in range(4)]
+    assert before - _free_bytes(hip_module) <= kept + GIB // 2
+    for qs in again + [keep]:
+        qs.delete()
