@@ -9,8 +9,9 @@
 // What is left is latency too: at 13 qubits an op takes 0.4 to 0.6 us, of decoding, LDS hand-overs and
 // table lines, with 4 waves on each SIMD of one compute unit (307 gates, 176 ops forward: 99 us, the
 // sweep 137 us).
-// <H> and gradient, whole calls, before the circuits ran here and now: 6 qubits complex128 336 ->
-// 229 us; 13 qubits complex64, 307 gates, 808 -> 547 us; 96 circuits of 6 to 11 qubits 1580 -> 503 us.
+// <H> and gradient, whole calls, on the tile passes and here: 6 qubits complex128 337 -> 257 us (their
+// host part differs by 60 us from process to process); 13 qubits complex64, 307 gates, 808 -> 671 us
+// (540 since its ZZ rotations are parity gates); 96 circuits of 6 to 11 qubits 1580 -> 507 us.
 //   one circuit      k_small_expect and k_small_sweep, one launch for each of the two calls
 //   a batch          k_small_rows (coefficients of every item, from its parameters), then one
 //                    workgroup an item, k_small_batch, from |0...0> to the item's gradient

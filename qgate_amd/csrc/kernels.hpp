@@ -80,12 +80,12 @@ double pauli_expectation(const Cx<R> *psi, Cx<R> *lam, int n_lanes, const std::v
 template <class R> void launch_set_zero_state(Cx<R> *a, int n_lanes);
 // dst = src (bytes a multiple of 16): the non-temporal streaming copy used as the HBM ceiling.
 void launch_stream_copy(void *dst, const void *src, u64 bytes);
-// P(bit `lane` == 0), FP64 accumulation; synchronises.
 // Lanes on which earlier collapses left nothing but one value (mask), and the ones among those
 // values (ones): every amplitude whose index differs there is zero.
 struct KnownLanes {
     u64 mask = 0, ones = 0;
 };
+// P(bit `lane` == 0), FP64 accumulation; synchronises.
 template <class R> double calc_prob(const Cx<R> *a, int n_lanes, int lane, const KnownLanes &known);
 // Doubles of partial-sum buffer calc_prob_in needs for this lane (the partials, run sums and
 // total), and calc_prob with that buffer given instead of taken from the allocator (no

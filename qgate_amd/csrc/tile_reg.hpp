@@ -25,8 +25,8 @@
 //   * A diagonal gate is its first entry, which without controls is a phase of the whole state (one
 //     factor per pass, none where only <H> and gradients are wanted), and a ratio.
 // Against passes without these steps, the backward sweep of the 24-qubit, 12-layer ansatz takes 15
-// passes of 272 us instead of 19 of 353, its forward part 15 of 106 us instead of 22 of 129, and 500
-// random gates on 30 qubits 16 of 5.5 ms instead of 20 of 5.8. Vector and scalar issue bound all of
+// passes of 265 us instead of 19 of 353, its forward part 15 of 105 us instead of 22 of 129, and 500
+// random gates on 30 qubits 19 of 4.4 ms instead of 20 of 5.8. Vector and scalar issue bound all of
 // them: a gate costs about 45 scalar instructions to decode and dispatch beside its arithmetic.
 #pragma once
 
@@ -48,7 +48,8 @@ namespace {
 
 // Low: the lowest bits that every tile holds, one 128-byte cache line. Each bit less frees one for a
 // gate's target: with 256-byte rows the 24-qubit ansatz took 19 sweep and 16 forward passes instead of
-// 15 and 15 (sweep 4.36 -> 4.08 ms, forward 1.63 -> 1.59), 500 gates on 30 qubits 17 instead of 16.
+// 15 and 15 (sweep 4.36 -> 4.08 ms, forward 1.63 -> 1.59), 500 gates on 30 qubits 22 instead of 19
+// (86.2 -> 83.4 ms; with 64-byte rows 110).
 template <class R>
 struct TileCfg;
 template <>
